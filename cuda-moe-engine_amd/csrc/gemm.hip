@@ -1,4 +1,4 @@
-// Grouped bf16 expert GEMMs on CDNA4 MFMA (v_mfma_f32_16x16x32_bf16; 32x32x16 on the generic path).
+// Grouped bf16 expert GEMMs on CDNA4 MFMA (v_mfma_f32_16x16x32_bf16).
 //
 // Problem: for every expert e, rows r in [offsets[e], offsets[e+1]) of A
 // [R, K] multiply B[e]^T (B is [E, N, K], K-contiguous like A) into C [R, N].
@@ -10,20 +10,19 @@
 // same lane, so the activation is computed in registers.
 //
 // Design (gfx950):
-//  * Fast path (K % 64 == 0, the block's shapes): ring_tile / grouped_gemm_persistent_kernel
-//    below -- 256 x 256 tiles on four wavefronts of 128 x 128 (16x16x32 MFMAs),
-//    direct-to-LDS buffer loads of whole 128-byte lines into an LDS ring of
-//    64-k stages, MFMAs interleaved with fragment reads and loads, XCD-aware
-//    rounds of full row tiles with the experts' short last row tiles carried
-//    beside them; 32- and 64-column tiles for decode-sized launches.
-//  * Generic path (any K % 8 == 0): grouped_gemm_kernel -- global -> register ->
-//    LDS double buffering with one barrier per 64-wide k-step; LDS rows are 128
-//    bytes with 16-byte chunks XOR-swizzled per row (swz).
-//  * Tile schedule is built on the device from offsets: expert e contributes
-//    ceil(span_e/256) row tiles per column tile (0 for an empty expert). No
-//    offsets are read on the host: the generic grid is an upper bound whose
-//    surplus workgroups exit at once, and the persistent grid is one workgroup
-//    per CU.
+//  * ring_tile / grouped_gemm_persistent_kernel below -- 256 x 256 tiles on
+//    four wavefronts of 128 x 128 (16x16x32 MFMAs), direct-to-LDS buffer loads
+//    of whole 128-byte lines into an LDS ring of 64-k stages, MFMAs interleaved
+//    with fragment reads and loads, XCD-aware rounds of full row tiles with the
+//    experts' short last row tiles carried beside them; 32- and 64-column tiles
+//    for decode-sized launches.
+//  * K not a multiple of 64 runs the same kernels with the last stage
+//    zero-filled past K (TAIL). A register-staged kernel with one barrier per
+//    k-step served those before: at H=1000, I=2744, 12 experts, top-3, gate/up
+//    took 124.9 us and down 109.3 us at 777 tokens against 67.8 and 44.0 us
+//    now, and 43.8 and 95.4 us against 26.5 and 12.4 us at 7.
+//  * The tile schedule is built on the device from offsets: no offsets are read
+//    on the host, and the persistent grid is one workgroup per CU.
 //  * Every output element is one MFMA chain in ascending k with one fp32
 //    accumulator, whichever path and tile shape computes it.
 #include <atomic>
@@ -36,11 +35,7 @@
 namespace moe {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-constexpr int kGemmThreads = 256;
-constexpr int kBK = 64;  // k-step: one 128-byte LDS row
 
 struct GemmParams {
     const uint16_t* a;        // [R, K], or with a_rows the [a_src_rows, K] rows they index
@@ -77,214 +72,8 @@ __device__ __forceinline__ void expert_rows(const GemmParams& p, int e, int& off
     span = static_cast<int>(hi - lo);
 }
 
-// 16-byte chunk c of LDS row r lives at physical chunk c ^ f(r), f(r) = (r ^ (r >> 3)) & 7.
-// A 16-byte read is serviced 16 lanes at a time across 64 four-byte banks (two
-// 128-byte rows); with this f, 16 consecutive rows at one logical chunk hit 16
-// distinct (row parity, chunk) bank groups, so fragment reads are conflict free
-// (and so are 8-lane groups on a 32-bank LDS).
-__device__ __forceinline__ int swz_key(int row) { return (row ^ (row >> 3)) & 7; }
-__device__ __forceinline__ int swz(int row, int chunk) { return row * kBK + ((chunk ^ swz_key(row)) << 3); }
-
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool SWIGLU>
-__global__ __launch_bounds__(kGemmThreads) void grouped_gemm_kernel(GemmParams p) {
-    constexpr int WTM = BM / WAVES_M;
-    constexpr int WTN = BN / WAVES_N;
-    constexpr int SM = WTM / 32;
-    constexpr int SN = WTN / 32;
-    constexpr int A_LOADS = BM * kBK / 8 / kGemmThreads;  // 16-byte chunks per thread
-    constexpr int B_LOADS = BN * kBK / 8 / kGemmThreads;
-    static_assert(WAVES_M * WAVES_N == 4, "4 wavefronts");
-    static_assert(A_LOADS >= 1 && B_LOADS >= 1, "tile too small");
-    static_assert(!SWIGLU || (SN % 2 == 0), "gate/up pairing needs an even sub-tile count");
-
-    __shared__ __attribute__((aligned(16))) uint16_t lds_a[2][BM * kBK];
-    __shared__ __attribute__((aligned(16))) uint16_t lds_b[2][BN * kBK];
-
-    // ---- tile lookup -------------------------------------------------------
-    const int32_t* __restrict__ offs = p.offsets;
-    int total = 0;
-    for (int e = 0; e < p.experts; ++e) {
-        const int span = offs[e + 1] - offs[e];
-        total += ((span + BM - 1) / BM) * p.n_tiles;
-    }
-    const int per_xcd = (total + kNumXcd - 1) / kNumXcd;
-    const int slot = blockIdx.x / kNumXcd;
-    if (slot >= per_xcd) return;
-    const int tile = (blockIdx.x % kNumXcd) * per_xcd + slot;
-    if (tile >= total) return;
-    int expert = 0, base = 0, m_tiles = 0;
-    for (; expert < p.experts; ++expert) {
-        const int span = offs[expert + 1] - offs[expert];
-        m_tiles = (span + BM - 1) / BM;
-        const int t = m_tiles * p.n_tiles;
-        if (tile < base + t) break;
-        base += t;
-    }
-    const int rel = tile - base;
-    const int n_tile = rel / m_tiles;
-    const int m_tile = rel - n_tile * m_tiles;
-    const int64_t row0 = offs[expert] + static_cast<int64_t>(m_tile) * BM;
-    const int64_t row_end = min(static_cast<int64_t>(offs[expert + 1]), p.rows);
-    if (row0 < 0 || row0 >= row_end) return;
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int wm = wave / WAVES_N;
-    const int wn = wave % WAVES_N;
-
-    // ---- per-thread global chunk pointers ----------------------------------
-    const uint16_t* a_src[A_LOADS];
-    int a_dst[A_LOADS];
-    bool a_ok[A_LOADS];
-    int a_kc[A_LOADS];
-#pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) {
-        const int chunk = tid + i * kGemmThreads;
-        const int r = chunk >> 3, c = chunk & 7;
-        const int64_t grow = row0 + r;
-        a_ok[i] = grow < row_end;
-        a_src[i] = p.a + (a_ok[i] ? grow : row0) * p.k + c * 8;
-        a_dst[i] = swz(r, c);
-        a_kc[i] = c * 8;
-    }
-    const uint16_t* b_src[B_LOADS];
-    int b_dst[B_LOADS];
-    bool b_ok[B_LOADS];
-    int b_kc[B_LOADS];
-    const uint16_t* b_expert = p.b + static_cast<int64_t>(expert) * p.nb * p.ldb;
-#pragma unroll
-    for (int i = 0; i < B_LOADS; ++i) {
-        const int chunk = tid + i * kGemmThreads;
-        const int r = chunk >> 3, c = chunk & 7;
-        int64_t brow;
-        bool ok;
-        if constexpr (SWIGLU) {
-            // LDS row r -> wave column block r / WTN; first half gate, second half up.
-            const int wcol = r / WTN, w = r % WTN;
-            constexpr int HALF = WTN / 2;
-            const int64_t col = static_cast<int64_t>(n_tile) * (BN / 2) + wcol * HALF + (w % HALF);
-            ok = col < p.n_out;
-            brow = (w < HALF) ? col : p.n_out + col;
-        } else {
-            const int64_t col = static_cast<int64_t>(n_tile) * BN + r;
-            ok = col < p.n_out;
-            brow = col;
-        }
-        b_ok[i] = ok;
-        b_src[i] = b_expert + (ok ? brow : 0) * p.ldb + c * 8;
-        b_dst[i] = swz(r, c);
-        b_kc[i] = c * 8;
-    }
-
-    floatx16 acc[SM][SN];
-#pragma unroll
-    for (int i = 0; i < SM; ++i)
-#pragma unroll
-        for (int j = 0; j < SN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    uint4 ra[A_LOADS], rb[B_LOADS];
-    const int64_t K = p.k;
-    const int k_steps = static_cast<int>((K + kBK - 1) / kBK);
-
-    auto load_tile = [&](int64_t k0) {
-#pragma unroll
-        for (int i = 0; i < A_LOADS; ++i)
-            ra[i] = (a_ok[i] && k0 + a_kc[i] < K) ? *reinterpret_cast<const uint4*>(a_src[i] + k0)
-                                                  : make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < B_LOADS; ++i)
-            rb[i] = (b_ok[i] && k0 + b_kc[i] < K) ? *reinterpret_cast<const uint4*>(b_src[i] + k0)
-                                                  : make_uint4(0, 0, 0, 0);
-    };
-    auto store_tile = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < A_LOADS; ++i) *reinterpret_cast<uint4*>(&lds_a[buf][a_dst[i]]) = ra[i];
-#pragma unroll
-        for (int i = 0; i < B_LOADS; ++i) *reinterpret_cast<uint4*>(&lds_b[buf][b_dst[i]]) = rb[i];
-    };
-
-    load_tile(0);
-    store_tile(0);
-    __syncthreads();
-
-    const int frag_row = lane & 31;
-    const int frag_half = lane >> 5;
-    for (int kt = 0; kt < k_steps; ++kt) {
-        const int buf = kt & 1;
-        const bool has_next = kt + 1 < k_steps;
-        if (has_next) load_tile(static_cast<int64_t>(kt + 1) * kBK);
-        const uint16_t* la = lds_a[buf];
-        const uint16_t* lb = lds_b[buf];
-#pragma unroll
-        for (int kk = 0; kk < kBK / 16; ++kk) {
-            const int chunk = kk * 2 + frag_half;
-            bf16x8_t af[SM], bfr[SN];
-#pragma unroll
-            for (int i = 0; i < SM; ++i) {
-                const int r = wm * WTM + i * 32 + frag_row;
-                af[i] = *reinterpret_cast<const bf16x8_t*>(&la[swz(r, chunk)]);
-            }
-#pragma unroll
-            for (int j = 0; j < SN; ++j) {
-                const int r = wn * WTN + j * 32 + frag_row;
-                bfr[j] = *reinterpret_cast<const bf16x8_t*>(&lb[swz(r, chunk)]);
-            }
-#pragma unroll
-            for (int i = 0; i < SM; ++i)
-#pragma unroll
-                for (int j = 0; j < SN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
-        }
-        if (has_next) store_tile(buf ^ 1);
-        __syncthreads();
-    }
-
-    // ---- epilogue ------------------------------------------------------------
-    // Accumulator register r of a 32x32 sub-tile holds row 8*(r/4) + 4*(lane/32) + r%4,
-    // column lane%32.
-    const int col_in = lane & 31;
-    const int row_in = (lane >> 5) * 4;
-    if constexpr (SWIGLU) {
-        constexpr int HALF_SN = SN / 2;
-#pragma unroll
-        for (int i = 0; i < SM; ++i) {
-#pragma unroll
-            for (int j = 0; j < HALF_SN; ++j) {
-                const int64_t col = static_cast<int64_t>(n_tile) * (BN / 2) + wn * (WTN / 2) + j * 32 + col_in;
-                if (col >= p.n_out) continue;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int64_t grow = row0 + wm * WTM + i * 32 + (r >> 2) * 8 + row_in + (r & 3);
-                    if (grow < row_end) {
-                        const float g = bf16_to_f32(f32_to_bf16(acc[i][j][r]));
-                        const float u = bf16_to_f32(f32_to_bf16(acc[i][j + HALF_SN][r]));
-                        p.c[grow * p.ldc + col] = f32_to_bf16(silu_f32(g) * u);
-                    }
-                }
-            }
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < SM; ++i) {
-#pragma unroll
-            for (int j = 0; j < SN; ++j) {
-                const int64_t col = static_cast<int64_t>(n_tile) * BN + wn * WTN + j * 32 + col_in;
-                if (col >= p.n_out) continue;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int64_t grow = row0 + wm * WTM + i * 32 + (r >> 2) * 8 + row_in + (r & 3);
-                    if (grow < row_end) p.c[grow * p.ldc + col] = f32_to_bf16(acc[i][j][r]);
-                }
-            }
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------
-// Fast path (K % 64 == 0): 256 x 256 output tiles computed by four wavefronts
+// Ring tiles: 256 x 256 output tiles computed by four wavefronts
 // (one per SIMD), each owning 128 x 128 (or (TM/2) x (BNT/2) for the short last
 // row tile of an expert, the split tail pieces and decode tiles) as a grid of
 // 16 x 16 blocks on v_mfma_f32_16x16x32_bf16.
@@ -315,7 +104,7 @@ __global__ __launch_bounds__(kGemmThreads) void grouped_gemm_kernel(GemmParams p
 //    the current one, each well ahead of its use, and a single set of fragment
 //    registers is live (see ring_tile). sched_barrier fences pin the order.
 //  * The k order of each output's MFMA chain (ascending k in groups of 8, one
-//    accumulator) is the same as the generic path, whatever the tile shape.
+//    accumulator) is the same whatever the tile shape.
 // ---------------------------------------------------------------------------
 constexpr int kStageK = 64;                    // k per LDS stage
 constexpr int kRowBytes = kStageK * 2;         // one 128-byte line per row and stage
@@ -355,9 +144,17 @@ __device__ __forceinline__ float swiglu_fast(float g, float u) {
 // row0 + TMR) of one expert (clamped to row_end) by BNT weight rows from
 // output column col0, in the first LDS_BYTES of `lds`, at most MAXS stages
 // deep. The four waves split the tile as (4/WC) row blocks x WC column blocks.
-template <int TMR, int BNT, bool SWIGLU, uint32_t LDS_BYTES, int WC = 2, int MAXS = 4, bool GATHER = false>
+//
+// TAIL (K not a multiple of 64): the last stage holds only K % 64 values per
+// row. Lanes whose 16-byte chunk lies past K take an offset past the buffer,
+// so the stage is zero-filled in LDS and the MFMAs run unchanged; without it
+// those lanes would read the next row (or a padded row's padding, which may
+// hold NaN). Only loads of that stage carry the select.
+template <int TMR, int BNT, bool SWIGLU, uint32_t LDS_BYTES, int WC = 2, int MAXS = 4, bool GATHER = false,
+          bool TAIL = false>
 struct RingOps {
     static_assert(!GATHER || SWIGLU, "only the gate/up GEMM gathers its rows");
+    static_assert(!(GATHER && TAIL), "gathered rows need K a multiple of 64");
     static constexpr int WAVES = kRingThreads / kWave;
     static constexpr int TM = TMR;
     static constexpr int WTM = TM / (WAVES / WC);  // the four waves as (4/WC) x WC
@@ -389,6 +186,7 @@ struct RingOps {
     uint32_t a_off[A_LOADS], b_off[B_LOADS];
     char* lds;
     int wave;
+    bool in_tail[2];  // TAIL: this lane's chunk of even / odd row groups lies below K in the last stage
 
     // A tile's two buffer resources and its per-lane A offsets. B: the
     // expert's weight rows from the tile's first column on (so the per-lane B
@@ -463,6 +261,12 @@ struct RingOps {
         rsrc_b = res.b;
         const int lrow = lane >> 3;
         const int pchunk = lane & 7;
+        if constexpr (TAIL) {
+            // ring_key of row 8 * g + lrow depends on g's parity only.
+            const int tail = static_cast<int>(p.k % kStageK);
+#pragma unroll
+            for (int g = 0; g < 2; ++g) in_tail[g] = (pchunk ^ ring_key(8 * g + lrow)) * 8 < tail;
+        }
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i) a_off[i] = res.a_off[i];
 #pragma unroll
@@ -484,14 +288,24 @@ struct RingOps {
     }
     // Load l of stage kt into ring slot st, of A and of B (of this tile, or of
     // the tile whose resources are given).
-    __device__ __forceinline__ void issue_a(int kt, int st, int l) const { issue_a(rsrc_a, kt, st, l, a_off[l]); }
-    __device__ __forceinline__ void issue_b(int kt, int st, int l) const { issue_b(rsrc_b, kt, st, l); }
-    __device__ __forceinline__ void issue_a(__amdgpu_buffer_rsrc_t r, int kt, int st, int l, uint32_t off) const {
-        dma16(r, lds + st * A_STAGE + (wave * A_LOADS + l) * 1024, off, static_cast<uint32_t>(kt) * kRowBytes);
+    // `last`: stage kt is the partial one of a TAIL instance.
+    __device__ __forceinline__ void issue_a(__amdgpu_buffer_rsrc_t r, int kt, int st, int l, uint32_t off,
+                                            bool last) const {
+        const int g = wave * A_LOADS + l;
+        dma16(r, lds + st * A_STAGE + g * 1024, tail_offset(off, kt, g, last), static_cast<uint32_t>(kt) * kRowBytes);
     }
-    __device__ __forceinline__ void issue_b(__amdgpu_buffer_rsrc_t r, int kt, int st, int l) const {
-        dma16(r, lds + B_BASE + st * B_STAGE + (wave * B_LOADS + l) * 1024, b_off[l],
+    __device__ __forceinline__ void issue_b(__amdgpu_buffer_rsrc_t r, int kt, int st, int l, bool last) const {
+        const int g = wave * B_LOADS + l;
+        dma16(r, lds + B_BASE + st * B_STAGE + g * 1024, tail_offset(b_off[l], kt, g, last),
               static_cast<uint32_t>(kt) * kRowBytes);
+    }
+    // The lane's offset for row group g, or in the partial stage one whose sum
+    // with the stage's offset is past every buffer (they end below 4 GiB - 16).
+    __device__ __forceinline__ uint32_t tail_offset(uint32_t off, int kt, int g, bool last) const {
+        if constexpr (TAIL) {
+            if (last && !in_tail[g & 1]) return 0xfffffff0u - static_cast<uint32_t>(kt) * kRowBytes;
+        }
+        return off;
     }
     // The windows before stage 0, in the steady-state order (A of stage
     // v+SA, then B of stage v+SB, for v = -SB .. -1; only v = -1 when `last`).
@@ -505,11 +319,13 @@ struct RingOps {
             if (v + SA >= 0) {
                 const int st = a0 + v + SA >= SA ? a0 + v : a0 + v + SA;
 #pragma unroll
-                for (int l = 0; l < A_LOADS; ++l) issue_a(min(v + SA, k_steps - 1), st, l);
+                for (int l = 0; l < A_LOADS; ++l)
+                    issue_a(rsrc_a, min(v + SA, k_steps - 1), st, l, a_off[l], v + SA >= k_steps - 1);
             }
             const int st = b0 + v + SB >= SB ? b0 + v : b0 + v + SB;
 #pragma unroll
-            for (int l = 0; l < B_LOADS; ++l) issue_b(min(v + SB, k_steps - 1), st, l);
+            for (int l = 0; l < B_LOADS; ++l)
+                issue_b(rsrc_b, min(v + SB, k_steps - 1), st, l, v + SB >= k_steps - 1);
         }
     }
 
@@ -542,14 +358,14 @@ struct NoHook {
 // starts at slots (sa0 + k_steps) % SA and (sb0 + k_steps) % SB and its hook
 // only issues the prologue's last window. Requires k_steps >= SB.
 template <int TMR, int BNT, bool SWIGLU, uint32_t LDS_BYTES, typename Hook = NoHook, int WC = 2, int MAXS = 4,
-          bool GATHER = false>
+          bool GATHER = false, bool TAIL = false>
 __device__ __forceinline__ void ring_tile(const GemmParams& p, char* lds, int expert, int64_t col0,
                                           int64_t row0, int64_t row_end, bool own_prologue = true,
                                           bool wait_all = false, const Hook& hook = Hook{}, int sa0 = 0, int sb0 = 0,
                                           bool chain = false,
-                                          typename RingOps<TMR, BNT, SWIGLU, LDS_BYTES, WC, MAXS, GATHER>::Rsrc next = {},
+                                          typename RingOps<TMR, BNT, SWIGLU, LDS_BYTES, WC, MAXS, GATHER, TAIL>::Rsrc next = {},
                                           const uint32_t* a_carry = nullptr) {
-    using R = RingOps<TMR, BNT, SWIGLU, LDS_BYTES, WC, MAXS, GATHER>;
+    using R = RingOps<TMR, BNT, SWIGLU, LDS_BYTES, WC, MAXS, GATHER, TAIL>;
     constexpr int WTM = R::WTM, WTN = R::WTN, FA = R::FA, FB = R::FB;
     constexpr int A_LOADS = R::A_LOADS, B_LOADS = R::B_LOADS;
     constexpr int SA = R::SA, SB = R::SB;
@@ -635,6 +451,7 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, char* lds, int ex
         int kt_a, slot_a, kt_b, slot_b;
         __amdgpu_buffer_rsrc_t ra, rb;  // this tile's or (chained) the next tile's
         bool a_next;                    // A loads of the next tile (its own offsets when gathered)
+        bool a_last, b_last;            // TAIL: the partial stage
     };
     auto refill_at = [&](auto g_c, const Refill& r) {
         constexpr int g = decltype(g_c)::value;  // MFMA slot in the window
@@ -642,12 +459,12 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, char* lds, int ex
             constexpr int l = decltype(l_c)::value;
             constexpr int slot = kQuarters ? l * HM / A_LOADS : l * 4 * HM / LOADS;
             if constexpr (slot == g)
-                ops.issue_a(r.ra, r.kt_a, r.slot_a, l, GATHER && r.a_next ? next.a_off[l] : ops.a_off[l]);
+                ops.issue_a(r.ra, r.kt_a, r.slot_a, l, GATHER && r.a_next ? next.a_off[l] : ops.a_off[l], r.a_last);
         });
         static_for<B_LOADS>([&](auto l_c) {
             constexpr int l = decltype(l_c)::value;
             constexpr int slot = kQuarters ? HM + l * (SWIGLU ? 2 : 3) * HM / B_LOADS : (A_LOADS + l) * 4 * HM / LOADS;
-            if constexpr (slot == g) ops.issue_b(r.rb, r.kt_b, r.slot_b, l);
+            if constexpr (slot == g) ops.issue_b(r.rb, r.kt_b, r.slot_b, l, r.b_last);
         });
     };
     // First half: B [0, HB) x A, reading this sub-step's B [HB, FB) at `bh`.
@@ -687,7 +504,7 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, char* lds, int ex
         });
     };
 
-    const int k_steps = static_cast<int>(K / kStageK);
+    const int k_steps = static_cast<int>((K + kStageK - 1) / kStageK);
     if (own_prologue) ops.prologue(k_steps, sa0, sb0);
     if (wait_all)
         wait_vm_lgkm<0>();
@@ -711,7 +528,7 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, char* lds, int ex
     // stage u+1; this window refills the slots stage u just freed.
     using NoLoads = std::integral_constant<int, -1>;
     using More = std::false_type;
-    const Refill none{0, 0, 0, 0, ops.rsrc_a, ops.rsrc_b, false};
+    const Refill none{0, 0, 0, 0, ops.rsrc_a, ops.rsrc_b, false, false, false};
     first_half(vb[0] + b_first, NoLoads{}, none);
     second_half(va[1] + a_first, vb[1] + b_first, More{}, NoLoads{}, none);
     first_half(vb[1] + b_first, NoLoads{}, none);
@@ -738,11 +555,12 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, char* lds, int ex
     // tile, at stages u+SA and u+SB, run in a loop of their own without
     // selects; only the last SB-1 windows (clamped stages, or the next tile's
     // first stages when chained) compute their refill in full.
+    // (TAIL: also the windows that load the partial stage.)
     int u = 0;
-    for (; u < k_steps - SB; ++u) {
+    for (; u < k_steps - SB - (TAIL ? 1 : 0); ++u) {
         const int na = sa + 1 == SA ? 0 : sa + 1;
         const int nb = sb + 1 == SB ? 0 : sb + 1;
-        window(Refill{u + SA, sa, u + SB, sb, ops.rsrc_a, ops.rsrc_b, false}, na, nb);
+        window(Refill{u + SA, sa, u + SB, sb, ops.rsrc_a, ops.rsrc_b, false, false, false}, na, nb);
         sa = na;
         sb = nb;
     }
@@ -753,9 +571,10 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, char* lds, int ex
         // chained, else this tile's last one again.
         const bool a_next = chain && u + SA >= k_steps;
         const bool b_next = chain && u + SB >= k_steps;
-        window(Refill{a_next ? u + SA - k_steps : min(u + SA, k_steps - 1), sa,
-                      b_next ? u + SB - k_steps : min(u + SB, k_steps - 1), sb,
-                      a_next ? next.a : ops.rsrc_a, b_next ? next.b : ops.rsrc_b, a_next},
+        const int kt_a = a_next ? u + SA - k_steps : min(u + SA, k_steps - 1);
+        const int kt_b = b_next ? u + SB - k_steps : min(u + SB, k_steps - 1);
+        window(Refill{kt_a, sa, kt_b, sb, a_next ? next.a : ops.rsrc_a, b_next ? next.b : ops.rsrc_b, a_next,
+                      kt_a == k_steps - 1, kt_b == k_steps - 1},
                na, nb);
         sa = na;
         sb = nb;
@@ -969,7 +788,7 @@ __device__ __forceinline__ RingSlot ring_slot(const RingPlan& pl, int grid, int 
     return s;
 }
 
-// The fast-path kernel is persistent: one workgroup per CU walks its virtual
+// The wide kernel is persistent: one workgroup per CU walks its virtual
 // workgroups and, once a tile's k-loop is done, issues the next tile's first
 // stages before running the epilogue, so their latency hides behind the
 // epilogue's arithmetic and stores, and the per-workgroup start-up is paid
@@ -1108,33 +927,42 @@ __device__ __forceinline__ RingWork ring_locate(const GemmParams& p, const RingT
     return w;
 }
 
+// A tile shape of the persistent kernel, as a type.
+template <int TMR, int BNT>
+struct RingShape {
+    template <bool SWIGLU, bool GATHER, bool TAIL>
+    using Ops = RingOps<TMR, BNT, SWIGLU, kRingBytes, 2, 4, GATHER, TAIL>;
+};
+
 // Issues tile w's prologue; with GATHER also leaves its A offsets in a_carry.
-template <bool SWIGLU, bool GATHER>
+template <bool SWIGLU, bool GATHER, bool TAIL>
 __device__ __forceinline__ void ring_prologue(const GemmParams& p, char* lds, const RingWork& w, uint32_t* a_carry) {
-    const int k_steps = static_cast<int>(p.k / kStageK);
-    auto go = [&](auto ops) {
+    const int k_steps = static_cast<int>((p.k + kStageK - 1) / kStageK);
+    auto go = [&](auto shape) {
+        using R = typename decltype(shape)::template Ops<SWIGLU, GATHER, TAIL>;
+        const R ops(p, lds, w.expert, w.col0, w.row0, w.row_end);
         ops.prologue(k_steps);
         if constexpr (GATHER) {
 #pragma unroll
-            for (int i = 0; i < decltype(ops)::A_LOADS; ++i) a_carry[i] = ops.a_off[i];
+            for (int i = 0; i < R::A_LOADS; ++i) a_carry[i] = ops.a_off[i];
         }
     };
     switch (w.variant) {
-        case 0: go(RingOps<256, 256, SWIGLU, kRingBytes, 2, 4, GATHER>(p, lds, w.expert, w.col0, w.row0, w.row_end)); break;
-        case 1: go(RingOps<128, 256, SWIGLU, kRingBytes, 2, 4, GATHER>(p, lds, w.expert, w.col0, w.row0, w.row_end)); break;
-        case 2: go(RingOps<64, 256, SWIGLU, kRingBytes, 2, 4, GATHER>(p, lds, w.expert, w.col0, w.row0, w.row_end)); break;
-        case 9: go(RingOps<32, 256, SWIGLU, kRingBytes, 2, 4, GATHER>(p, lds, w.expert, w.col0, w.row0, w.row_end)); break;
-        case 10: go(RingOps<224, 256, SWIGLU, kRingBytes, 2, 4, GATHER>(p, lds, w.expert, w.col0, w.row0, w.row_end)); break;
-        case 11: go(RingOps<192, 256, SWIGLU, kRingBytes, 2, 4, GATHER>(p, lds, w.expert, w.col0, w.row0, w.row_end)); break;
-        case 12: go(RingOps<160, 256, SWIGLU, kRingBytes, 2, 4, GATHER>(p, lds, w.expert, w.col0, w.row0, w.row_end)); break;
+        case 0: go(RingShape<256, 256>{}); break;
+        case 1: go(RingShape<128, 256>{}); break;
+        case 2: go(RingShape<64, 256>{}); break;
+        case 9: go(RingShape<32, 256>{}); break;
+        case 10: go(RingShape<224, 256>{}); break;
+        case 11: go(RingShape<192, 256>{}); break;
+        case 12: go(RingShape<160, 256>{}); break;
         default:
             if constexpr (!SWIGLU) {
-                if (w.variant == 3) go(RingOps<256, 128, false, kRingBytes>(p, lds, w.expert, w.col0, w.row0, w.row_end));
-                else if (w.variant == 4) go(RingOps<128, 128, false, kRingBytes>(p, lds, w.expert, w.col0, w.row0, w.row_end));
-                else if (w.variant == 5) go(RingOps<64, 128, false, kRingBytes>(p, lds, w.expert, w.col0, w.row0, w.row_end));
-                else if (w.variant == 6) go(RingOps<256, 64, false, kRingBytes>(p, lds, w.expert, w.col0, w.row0, w.row_end));
-                else if (w.variant == 7) go(RingOps<128, 64, false, kRingBytes>(p, lds, w.expert, w.col0, w.row0, w.row_end));
-                else go(RingOps<64, 64, false, kRingBytes>(p, lds, w.expert, w.col0, w.row0, w.row_end));
+                if (w.variant == 3) go(RingShape<256, 128>{});
+                else if (w.variant == 4) go(RingShape<128, 128>{});
+                else if (w.variant == 5) go(RingShape<64, 128>{});
+                else if (w.variant == 6) go(RingShape<256, 64>{});
+                else if (w.variant == 7) go(RingShape<128, 64>{});
+                else go(RingShape<64, 64>{});
             }
     }
 }
@@ -1144,12 +972,12 @@ __device__ __forceinline__ void ring_prologue(const GemmParams& p, char* lds, co
 // enough, the two are chained (see ring_tile): `w`'s last windows load `nxt`'s
 // first stages and its hook issues only the prologue's last window. Otherwise
 // the hook issues `nxt`'s whole prologue at slots 0.
-template <int TMR, int BNT, bool SWIGLU, bool GATHER = false>
+template <int TMR, int BNT, bool SWIGLU, bool GATHER, bool TAIL>
 __device__ __forceinline__ void ring_run_shape(const GemmParams& p, char* lds, const RingWork& w,
                                                const RingWork& nxt, bool wait_all, int& sa, int& sb,
                                                uint32_t* a_carry) {
-    using R = RingOps<TMR, BNT, SWIGLU, kRingBytes, 2, 4, GATHER>;
-    const int k_steps = static_cast<int>(p.k / kStageK);
+    using R = RingOps<TMR, BNT, SWIGLU, kRingBytes, 2, 4, GATHER, TAIL>;
+    const int k_steps = static_cast<int>((p.k + kStageK - 1) / kStageK);
     // Wave-uniform (it selects buffer resources, which live in SGPRs).
     const bool chain = __builtin_amdgcn_readfirstlane(nxt.valid && nxt.variant == w.variant && k_steps >= R::SB) != 0;
     typename R::Rsrc next{};
@@ -1177,40 +1005,39 @@ __device__ __forceinline__ void ring_run_shape(const GemmParams& p, char* lds, c
                 R(p, lds, nxt.expert, nxt.col0, nxt.row0, nxt.row_end).prologue(k_steps, na, nb, true);
             }
         } else {
-            ring_prologue<SWIGLU, GATHER>(p, lds, nxt, a_carry);
+            ring_prologue<SWIGLU, GATHER, TAIL>(p, lds, nxt, a_carry);
         }
     };
-    ring_tile<TMR, BNT, SWIGLU, kRingBytes, decltype(hook), 2, 4, GATHER>(p, lds, w.expert, w.col0, w.row0, w.row_end,
-                                                                           false, wait_all, hook, sa, sb, chain, next,
-                                                                           a_carry);
+    ring_tile<TMR, BNT, SWIGLU, kRingBytes, decltype(hook), 2, 4, GATHER, TAIL>(
+        p, lds, w.expert, w.col0, w.row0, w.row_end, false, wait_all, hook, sa, sb, chain, next, a_carry);
     sa = chain ? na : 0;
     sb = chain ? nb : 0;
 }
 
-template <bool SWIGLU, bool GATHER>
+template <bool SWIGLU, bool GATHER, bool TAIL>
 __device__ __forceinline__ void ring_run(const GemmParams& p, char* lds, const RingWork& w, const RingWork& nxt,
                                          bool wait_all, int& sa, int& sb, uint32_t* a_carry) {
     switch (w.variant) {
-        case 0: ring_run_shape<256, 256, SWIGLU, GATHER>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 1: ring_run_shape<128, 256, SWIGLU, GATHER>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 2: ring_run_shape<64, 256, SWIGLU, GATHER>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 9: ring_run_shape<32, 256, SWIGLU, GATHER>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 10: ring_run_shape<224, 256, SWIGLU, GATHER>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 11: ring_run_shape<192, 256, SWIGLU, GATHER>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 12: ring_run_shape<160, 256, SWIGLU, GATHER>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 0: ring_run_shape<256, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 1: ring_run_shape<128, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 2: ring_run_shape<64, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 9: ring_run_shape<32, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 10: ring_run_shape<224, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 11: ring_run_shape<192, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 12: ring_run_shape<160, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
         default:
             if constexpr (!SWIGLU) {
-                if (w.variant == 3) ring_run_shape<256, 128, false>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
-                else if (w.variant == 4) ring_run_shape<128, 128, false>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
-                else if (w.variant == 5) ring_run_shape<64, 128, false>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
-                else if (w.variant == 6) ring_run_shape<256, 64, false>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
-                else if (w.variant == 7) ring_run_shape<128, 64, false>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
-                else ring_run_shape<64, 64, false>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
+                if (w.variant == 3) ring_run_shape<256, 128, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
+                else if (w.variant == 4) ring_run_shape<128, 128, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
+                else if (w.variant == 5) ring_run_shape<64, 128, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
+                else if (w.variant == 6) ring_run_shape<256, 64, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
+                else if (w.variant == 7) ring_run_shape<128, 64, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
+                else ring_run_shape<64, 64, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
             }
     }
 }
 
-template <bool SWIGLU, bool GATHER>
+template <bool SWIGLU, bool GATHER, bool TAIL>
 __global__ __launch_bounds__(kRingThreads) void grouped_gemm_persistent_kernel(GemmParams p) {
     __shared__ __attribute__((aligned(1024))) char lds[kRingBytes];
     // Balanced row tiles for the gate/up GEMM at K >= 2048. There a short last
@@ -1238,7 +1065,7 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_persistent_kernel(G
     RingWork cur = next(q, sub);
     if (!cur.valid) return;
     uint32_t a_carry[8];  // GATHER: the next tile's A offsets (at most 8 loads per wave and stage)
-    ring_prologue<SWIGLU, GATHER>(p, lds, cur, a_carry);
+    ring_prologue<SWIGLU, GATHER, TAIL>(p, lds, cur, a_carry);
     bool after_epilogue = false;
     int sa = 0, sb = 0;  // ring slots of the current tile's first stage
     for (;;) {
@@ -1259,7 +1086,7 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_persistent_kernel(G
             nxt.expert = e;
             nxt.variant = v;
         }
-        ring_run<SWIGLU, GATHER>(p, lds, cur, nxt, after_epilogue, sa, sb, a_carry);
+        ring_run<SWIGLU, GATHER, TAIL>(p, lds, cur, nxt, after_epilogue, sa, sb, a_carry);
         if (!nxt.valid) break;
         cur = nxt;
         q = qn;
@@ -1299,7 +1126,7 @@ constexpr uint32_t decode_lds_bytes() {
     return SWIGLU && MAX_ROWS == 64 ? 3 * (64 + 2 * narrow_cols<SWIGLU, MAX_ROWS>()) * kRowBytes : kRingBytes;
 }
 
-template <bool SWIGLU, int MAX_ROWS, bool GATHER>
+template <bool SWIGLU, int MAX_ROWS, bool GATHER, bool TAIL>
 __global__ __launch_bounds__(kRingThreads) void grouped_gemm_decode_kernel(GemmParams p) {
     constexpr int COLS = narrow_cols<SWIGLU, MAX_ROWS>();
     constexpr int BNT = SWIGLU ? 2 * COLS : COLS;
@@ -1318,7 +1145,7 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_decode_kernel(GemmP
     const int incl = wave_inclusive_sum(count);
     const int first = incl - count;
     const int tiles = __builtin_amdgcn_readlane(incl, kWave - 1);
-    const int k_steps = static_cast<int>(p.k / kStageK);
+    const int k_steps = static_cast<int>((p.k + kStageK - 1) / kStageK);
     struct Work {
         bool valid;
         int tall, expert, row0, row_end, col0;  // tall: more than 64 rows
@@ -1353,23 +1180,23 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_decode_kernel(GemmP
     auto prologue = [&](const Work& w) {
         if constexpr (MAX_ROWS == 128) {
             if (w.tall) {
-                issue(RingOps<128, BNT, SWIGLU, kLds, WC, kDecodeStages, GATHER>(p, lds, w.expert, w.col0, w.row0,
+                issue(RingOps<128, BNT, SWIGLU, kLds, WC, kDecodeStages, GATHER, TAIL>(p, lds, w.expert, w.col0, w.row0,
                                                                                  w.row_end));
                 return;
             }
         }
-        issue(RingOps<64, BNT, SWIGLU, kLds, WC, kDecodeStages, GATHER>(p, lds, w.expert, w.col0, w.row0, w.row_end));
+        issue(RingOps<64, BNT, SWIGLU, kLds, WC, kDecodeStages, GATHER, TAIL>(p, lds, w.expert, w.col0, w.row0, w.row_end));
     };
     auto run = [&](const Work& w, bool wait_all, const auto& hook) {
         using Hook = std::decay_t<decltype(hook)>;
         if constexpr (MAX_ROWS == 128) {
             if (w.tall) {
-                ring_tile<128, BNT, SWIGLU, kLds, Hook, WC, kDecodeStages, GATHER>(
+                ring_tile<128, BNT, SWIGLU, kLds, Hook, WC, kDecodeStages, GATHER, TAIL>(
                     p, lds, w.expert, w.col0, w.row0, w.row_end, false, wait_all, hook, 0, 0, false, {}, a_carry);
                 return;
             }
         }
-        ring_tile<64, BNT, SWIGLU, kLds, Hook, WC, kDecodeStages, GATHER>(
+        ring_tile<64, BNT, SWIGLU, kLds, Hook, WC, kDecodeStages, GATHER, TAIL>(
             p, lds, w.expert, w.col0, w.row0, w.row_end, false, wait_all, hook, 0, 0, false, {}, a_carry);
     };
     int t = blockIdx.x;
@@ -1426,13 +1253,28 @@ static int device_cu_count() {
     return cached[dev];
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool SWIGLU>
+// f(integral_constant<bool, GATHER>, integral_constant<bool, TAIL>) for these
+// parameters (gathered rows come with K a multiple of 64, the ABI's check).
+template <bool SWIGLU, typename F>
+static void with_source(const GemmParams& p, F&& f) {
+    if constexpr (SWIGLU) {
+        if (p.a_rows != nullptr) return f(std::true_type{}, std::false_type{});
+    }
+    if (p.k % kStageK == 0)
+        f(std::false_type{}, std::false_type{});
+    else
+        f(std::false_type{}, std::true_type{});
+}
+
+template <bool SWIGLU>
 static int launch_gemm_t(GemmParams p, int64_t rows, hipStream_t stream) {
-    const int64_t out_per_tile = SWIGLU ? BN / 2 : BN;
-    p.n_tiles = static_cast<int>((p.n_out + out_per_tile - 1) / out_per_tile);
-    // Upper bound on row tiles: sum_e ceil(span_e/BM) <= ceil(R/BM) + E.
-    const int64_t m_bound = (rows + BM - 1) / BM + p.experts;
-    int64_t blocks = m_bound * p.n_tiles;
+    constexpr int64_t kRows = 256, kCols = SWIGLU ? 128 : 256;  // the wide tiles' output
+    if (p.a_rows != nullptr && p.k % kStageK != 0)
+        return fail(MOE_ERR_UNSUPPORTED, "gathered A rows need K a multiple of 64");
+    p.n_tiles = static_cast<int>((p.n_out + kCols - 1) / kCols);
+    // Upper bound on row tiles: sum_e ceil(span_e/256) <= ceil(R/256) + E.
+    const int64_t m_bound = (rows + kRows - 1) / kRows + p.experts;
+    const int64_t blocks = m_bound * p.n_tiles;
     if (blocks == 0) return MOE_OK;
     // Narrow tiles for weight streaming: at most 128 rows in all, or at most 128
     // per expert on average when the wide tiles (rows spread evenly over the
@@ -1440,76 +1282,50 @@ static int launch_gemm_t(GemmParams p, int64_t rows, hipStream_t stream) {
     // gate/up 9.4 -> 7.2 us, down 11.6 -> 7.4 us; at C3 T=256 the gate/up GEMM's
     // 256 wide tiles streamed faster than narrow ones (22.9 vs 24.9 us).
     const int64_t per_expert = (rows + p.experts - 1) / p.experts;
-    const int64_t wide_tiles = static_cast<int64_t>(p.experts) * ((per_expert + BM - 1) / BM) * p.n_tiles;
+    const int64_t wide_tiles = static_cast<int64_t>(p.experts) * ((per_expert + kRows - 1) / kRows) * p.n_tiles;
     const bool narrow = rows <= 128 || (rows <= 128 * static_cast<int64_t>(p.experts) &&
                                         wide_tiles < device_cu_count());
-    if (BM == 256 && BN == 256 && p.k % kStageK == 0 && narrow) {
-        GemmParams q = p;
+    if (narrow) {
         const int max_rows = rows <= 64 ? 64 : 128;
         const int cols = max_rows == 64 ? narrow_cols<SWIGLU, 64>() : narrow_cols<SWIGLU, 128>();
-        q.n_tiles = static_cast<int>((p.n_out + cols - 1) / cols);
+        p.n_tiles = static_cast<int>((p.n_out + cols - 1) / cols);
         // Upper bound on row tiles: sum_e ceil(span_e/max_rows) <= ceil(R/max_rows) + E.
-        const int64_t tiles = ((rows + max_rows - 1) / max_rows + p.experts) * q.n_tiles;
+        const int64_t tiles = ((rows + max_rows - 1) / max_rows + p.experts) * p.n_tiles;
         if (tiles > INT32_MAX) return fail(MOE_ERR_CAPACITY, "grouped GEMM grid too large");
         // As many workgroups as fit the CUs' LDS, at most one per tile.
         const uint32_t lds = rows <= 64 ? decode_lds_bytes<SWIGLU, 64>() : decode_lds_bytes<SWIGLU, 128>();
         int64_t grid = static_cast<int64_t>(device_cu_count()) * (kRingBytes / lds);
         if (tiles < grid) grid = tiles;
-        auto launch = [&](auto gather_c) {
-            constexpr bool G = decltype(gather_c)::value;
+        with_source<SWIGLU>(p, [&](auto gather_c, auto tail_c) {
+            constexpr bool G = decltype(gather_c)::value, T = decltype(tail_c)::value;
             if (rows <= 64)
-                hipLaunchKernelGGL((grouped_gemm_decode_kernel<SWIGLU, 64, G>), dim3(static_cast<unsigned>(grid)),
-                                   dim3(kRingThreads), 0, stream, q);
+                hipLaunchKernelGGL((grouped_gemm_decode_kernel<SWIGLU, 64, G, T>), dim3(static_cast<unsigned>(grid)),
+                                   dim3(kRingThreads), 0, stream, p);
             else
-                hipLaunchKernelGGL((grouped_gemm_decode_kernel<SWIGLU, 128, G>), dim3(static_cast<unsigned>(grid)),
-                                   dim3(kRingThreads), 0, stream, q);
-        };
-        if constexpr (SWIGLU) {
-            if (p.a_rows != nullptr)
-                launch(std::true_type{});
-            else
-                launch(std::false_type{});
-        } else {
-            launch(std::false_type{});
-        }
+                hipLaunchKernelGGL((grouped_gemm_decode_kernel<SWIGLU, 128, G, T>), dim3(static_cast<unsigned>(grid)),
+                                   dim3(kRingThreads), 0, stream, p);
+        });
         return check_launch("grouped_gemm_decode_kernel");
     }
-    if (BM == 256 && BN == 256 && p.k % kStageK == 0) {
-        // One workgroup per CU (the ring fills a CU's LDS), each walking the
-        // virtual workgroups of the device-side plan, whose XCD ranges need a
-        // multiple of 8 workgroups. Row offsets fit 32 bits (checked by the ABI).
-        if (blocks > INT32_MAX) return fail(MOE_ERR_CAPACITY, "grouped GEMM grid too large");
-        int64_t grid = device_cu_count();
-        const int limit = g_gemm_workgroup_limit.load(std::memory_order_relaxed);
-        if (limit > 0 && limit < grid) grid = limit;
-        // At most one workgroup per unit of work: tiles, or for the plain GEMM
-        // the halves and quarters the plan may split them into.
-        const int64_t units = SWIGLU ? blocks : 4 * blocks;
-        if (units < grid) grid = units;
-        grid = grid / kNumXcd * kNumXcd;
-        if (grid < kNumXcd) grid = kNumXcd;
-        if constexpr (SWIGLU) {
-            if (p.a_rows != nullptr)
-                hipLaunchKernelGGL((grouped_gemm_persistent_kernel<true, true>), dim3(static_cast<unsigned>(grid)),
-                                   dim3(kRingThreads), 0, stream, p);
-            else
-                hipLaunchKernelGGL((grouped_gemm_persistent_kernel<true, false>), dim3(static_cast<unsigned>(grid)),
-                                   dim3(kRingThreads), 0, stream, p);
-        } else {
-            hipLaunchKernelGGL((grouped_gemm_persistent_kernel<false, false>), dim3(static_cast<unsigned>(grid)),
-                               dim3(kRingThreads), 0, stream, p);
-        }
-        return check_launch("grouped_gemm_persistent_kernel");
-    }
-    if (p.a_rows != nullptr) return fail(MOE_ERR_UNSUPPORTED, "gathered A rows need K a multiple of 64");
-    // The generic kernel maps workgroup b to tile (b % 8) * per_xcd + b / 8 with
-    // per_xcd = ceil(tiles / 8), which reaches every tile only when the grid
-    // holds all 8 * per_xcd slots: round the upper bound up to a multiple of 8.
-    blocks = (blocks + kNumXcd - 1) / kNumXcd * kNumXcd;
+    // One workgroup per CU (the ring fills a CU's LDS), each walking the
+    // virtual workgroups of the device-side plan, whose XCD ranges need a
+    // multiple of 8 workgroups. Row offsets fit 32 bits (checked by the ABI).
     if (blocks > INT32_MAX) return fail(MOE_ERR_CAPACITY, "grouped GEMM grid too large");
-    hipLaunchKernelGGL((grouped_gemm_kernel<BM, BN, WAVES_M, WAVES_N, SWIGLU>),
-                       dim3(static_cast<unsigned>(blocks)), dim3(kGemmThreads), 0, stream, p);
-    return check_launch("grouped_gemm_kernel");
+    int64_t grid = device_cu_count();
+    const int limit = g_gemm_workgroup_limit.load(std::memory_order_relaxed);
+    if (limit > 0 && limit < grid) grid = limit;
+    // At most one workgroup per unit of work: tiles, or for the plain GEMM
+    // the halves and quarters the plan may split them into.
+    const int64_t units = SWIGLU ? blocks : 4 * blocks;
+    if (units < grid) grid = units;
+    grid = grid / kNumXcd * kNumXcd;
+    if (grid < kNumXcd) grid = kNumXcd;
+    with_source<SWIGLU>(p, [&](auto gather_c, auto tail_c) {
+        constexpr bool G = decltype(gather_c)::value, T = decltype(tail_c)::value;
+        hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, G, T>), dim3(static_cast<unsigned>(grid)),
+                           dim3(kRingThreads), 0, stream, p);
+    });
+    return check_launch("grouped_gemm_persistent_kernel");
 }
 
 int launch_grouped_gemm(const uint16_t* a, const uint16_t* b, int64_t ldb, uint16_t* c, const int32_t* offsets,
@@ -1526,7 +1342,7 @@ int launch_grouped_gemm(const uint16_t* a, const uint16_t* b, int64_t ldb, uint1
     p.n_out = n;
     p.ldc = n;
     p.experts = experts;
-    return launch_gemm_t<256, 256, 2, 2, false>(p, rows, stream);
+    return launch_gemm_t<false>(p, rows, stream);
 }
 
 int launch_gateup_swiglu(const uint16_t* a, const uint16_t* gate_up, int64_t ldb, uint16_t* act,
@@ -1544,7 +1360,7 @@ int launch_gateup_swiglu(const uint16_t* a, const uint16_t* gate_up, int64_t ldb
     p.n_out = intermediate;
     p.ldc = intermediate;
     p.experts = experts;
-    return launch_gemm_t<256, 256, 2, 2, true>(p, rows, stream);
+    return launch_gemm_t<true>(p, rows, stream);
 }
 
 // launch_gateup_swiglu with A row r read from row a_rows[r] of x (zero when
@@ -1567,7 +1383,7 @@ int launch_gateup_swiglu_gathered(const uint16_t* x, const int32_t* a_rows, int6
     p.n_out = intermediate;
     p.ldc = intermediate;
     p.experts = experts;
-    return launch_gemm_t<256, 256, 2, 2, true>(p, rows, stream);
+    return launch_gemm_t<true>(p, rows, stream);
 }
 
 }  // namespace moe

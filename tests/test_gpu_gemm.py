@@ -298,6 +298,43 @@ def test_row_padded_weights_equal_contiguous(ext, counts, alignment, n, k, pad):
         assert torch.equal(gathered[0], act[0])
 
 
+PARTIAL_STAGE_CASES = [
+    # counts per expert, alignment, n (intermediate for gate/up), k: K % 64 from 8 to 56
+    ([2, 0, 5], 1, 104, 8),                              # one stage, weight-streaming 64-row instance
+    ([60, 40, 20], 8, 96, 72),                           # 128-row instance; two stages, fewer than the ring holds
+    ([700, 3, 0, 260, 129], 8, 384, 56),                 # persistent kernel, one stage: tiles are not chained
+    ([700, 3, 40, 260, 1100], 8, 520, 248),              # four stages: chained tiles, short tiles
+    ([1030, 1030, 2048], 8, 512, 328),                   # column pieces left after the rounds
+    ([300, 420, 520, 700, 1034, 100], 8, 136, 2744),     # balanced row tiles (gate/up at K >= 2048)
+]
+
+
+@pytest.mark.parametrize("counts,alignment,n,k", PARTIAL_STAGE_CASES)
+def test_partial_last_stage_equals_zero_padded(ext, counts, alignment, n, k):
+    """K not a multiple of 64: the last 64-k stage is zero-filled past K, so the outputs
+    equal, bit for bit, those of operands zero-padded to whole stages (the same MFMA
+    chains, plus products of zeros). The weights' row padding holds NaN, and one row
+    of A does, whose outputs alone may be NaN."""
+    experts = len(counts)
+    a, offsets, rows = _inputs(counts, alignment, k, seed=5 * k + n)
+    used = int(to_np(offsets)[-1])
+    a[used // 2] = float("nan")
+    g = torch.Generator(device="cuda").manual_seed(11 * k + n)
+    full = -(-k // 64) * 64
+    a_full = torch.nn.functional.pad(a, (0, full - k)).contiguous()
+    a_full[used // 2] = float("nan")
+    for width, run in ((n, ext.grouped_gemm_out), (2 * n, ext.gateup_swiglu_out)):
+        w = (torch.randn(experts, width, k, device="cuda", generator=g) / k**0.5).bfloat16()
+        got = torch.full((rows, n), 3.0, device="cuda").bfloat16()
+        want = got.clone()
+        run(a, _row_padded(w, 72), offsets, got)
+        run(a_full, torch.nn.functional.pad(w, (0, full - k)).contiguous(), offsets, want)
+        nan_rows = torch.isnan(got.float()).any(dim=1).nonzero().flatten().tolist()
+        assert nan_rows == [used // 2]
+        keep = torch.arange(rows, device="cuda") != used // 2
+        assert torch.equal(got[keep], want[keep])
+
+
 def test_weights_of_other_layouts_are_refused(ext):
     a, offsets, rows = _inputs([10, 20], 8, 64, seed=1)
     out = torch.empty(rows, 64, device="cuda", dtype=torch.bfloat16)
