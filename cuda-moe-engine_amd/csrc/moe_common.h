@@ -60,6 +60,13 @@ __device__ __forceinline__ uint16_t f32_to_f16(float f) {
     return h;
 }
 
+// N elements at any element's address, moved as one vector (global loads and
+// stores of up to 16 bytes need no wider alignment on gfx950).
+template <typename T, int N>
+struct __attribute__((packed, aligned(alignof(T)))) Unaligned {
+    T v[N];
+};
+
 // Element access by storage dtype (MOE_DTYPE_*), used by the transport and
 // activation kernels that support fp32 / fp16 / bf16.
 template <int DT> struct Elem;
@@ -67,33 +74,43 @@ template <> struct Elem<MOE_DTYPE_F32> {
     using T = float;
     static __device__ __forceinline__ float load(T v) { return v; }
     static __device__ __forceinline__ T store(float f) { return f; }
+    static __device__ __forceinline__ T store_product(float a, float b) { return a * b; }
 };
 template <> struct Elem<MOE_DTYPE_F16> {
     using T = uint16_t;
     static __device__ __forceinline__ float load(T v) { return f16_to_f32(v); }
     static __device__ __forceinline__ T store(float f) { return f32_to_f16(f); }
+    // a * b rounded once (v_fma_mixlo_f16). Paired conversions (v_cvt_pk_f16_f32)
+    // would round the fp32 product first; the empty asm keeps the compiler from pairing.
+    static __device__ __forceinline__ T store_product(float a, float b) {
+        T h = f32_to_f16(a * b);
+        asm("" : "+v"(h));
+        return h;
+    }
 };
 template <> struct Elem<MOE_DTYPE_BF16> {
     using T = uint16_t;
     static __device__ __forceinline__ float load(T v) { return bf16_to_f32(v); }
     static __device__ __forceinline__ T store(float f) { return f32_to_bf16(f); }
+    static __device__ __forceinline__ T store_product(float a, float b) { return f32_to_bf16(a * b); }
 };
 
 // ---------------------------------------------------------------------------
-// exp and SiLU with a fixed operation sequence, so a CPU restatement with
-// IEEE fp32 operations reproduces them bit for bit: Cody-Waite reduction
-// x = n*ln2 + r (ln2 = 16-bit head + tail, so n*ln2_hi is exact), degree-7
-// Taylor polynomial of e^r in Horner form with separately rounded multiply and
-// add, then ldexp. Within 2 ulp of exp on [-80, 88]; +inf above, 0 below
-// (where 1 + e^x already rounds to 1).
+// SiLU, g / (1 + exp(-g)) with a correctly rounded fp32 division, in a fixed
+// operation sequence that a CPU restatement with IEEE fp32 operations reproduces
+// bit for bit. exp(x): Cody-Waite reduction x = n*ln2 + r (ln2 = 16-bit head +
+// tail; n*ln2_hi is exact, so the fma rounds as a separate subtraction would),
+// degree-7 Taylor polynomial of e^r in Horner form with separately rounded
+// multiply and add, then ldexp; +inf above 88. Within 2 ulp of exp on [-80, 88].
+// Below -80 any tiny exp leaves 1 + exp at 1, so one clamp stands for a test,
+// and a NaN g is NaN through the division whatever exp is: about 40 VALU
+// operations, which is what a bf16 or fp16 activation kernel is bound by.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float exp_f32(float x) {
+__device__ __forceinline__ float silu_f32(float g) {
 #pragma clang fp contract(off)
-    if (x != x) return x;
-    if (x > 88.0f) return __builtin_inff();
-    if (x < -80.0f) return 0.0f;
+    const float x = __builtin_amdgcn_fmed3f(-g, -80.0f, 1000.0f);
     const float n = rintf(x * __uint_as_float(0x3fb8aa3bu));  // log2(e)
-    float r = x - n * __uint_as_float(0x3f317200u);            // ln2 head
+    float r = __builtin_fmaf(-n, __uint_as_float(0x3f317200u), x);  // ln2 head
     r = r - n * __uint_as_float(0x35bfbe8eu);                  // ln2 tail
     float p = __uint_as_float(0x39500d01u);                    // 1/7!
     p = p * r + __uint_as_float(0x3ab60b61u);                  // 1/6!
@@ -103,13 +120,8 @@ __device__ __forceinline__ float exp_f32(float x) {
     p = p * r + 0.5f;
     p = p * r + 1.0f;
     p = p * r + 1.0f;
-    return ldexpf(p, static_cast<int>(n));
-}
-
-// silu(g) = g / (1 + exp(-g)) with a correctly rounded fp32 division.
-__device__ __forceinline__ float silu_f32(float g) {
-#pragma clang fp contract(off)
-    return g / (1.0f + exp_f32(-g));
+    const float e = x > 88.0f ? __builtin_inff() : __builtin_amdgcn_ldexpf(p, static_cast<int>(n));
+    return g / (1.0f + e);
 }
 
 inline int dtype_size(int dtype) {

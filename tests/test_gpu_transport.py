@@ -175,3 +175,30 @@ def test_reference_runtime_validation_suite(ext):
     summary = run_tests(ext)
     assert summary["passed"] == 36 and summary["failed"] == 0
     assert summary["max_absolute_error"] < 2e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,width", [(5, 1), (3, 7), (9, 8), (300, 9), (40, 257), (2, 2049), (3000, 40)])
+def test_standalone_swiglu_widths(ext, dtype, rows, width):
+    """Widths around whole vectors, rows and blocks, with special gate values: bit-exact
+    (16 bits: the fp32 activation times up, rounded once)."""
+    g = torch.Generator(device="cuda").manual_seed(rows + width)
+    projection = (8 * torch.randn(rows, 2 * width, device="cuda", generator=g)).to(dtype)
+    special = torch.tensor([0.0, -0.0, float("inf"), float("-inf"), float("nan"), -88.0, -88.5, -200.0, 80.0, 1e4],
+                           device="cuda").to(dtype)
+    n = min(width, special.numel())
+    projection[0, :n] = special[:n]
+    valid = rows - rows // 3
+    out = torch.full((rows, width), 7.0, device="cuda", dtype=dtype)
+    ext.swiglu_out(projection, torch.tensor([valid], device="cuda", dtype=torch.int32), out)
+    p = to_np(projection).astype(np.float32)
+    silu, up = oracle.silu_f32(p[:, :width]), p[:, width:]
+    with np.errstate(all="ignore"):
+        if dtype == torch.float16:
+            expected = (silu.astype(np.float64) * up.astype(np.float64)).astype(np.float16).astype(np.float32)
+        else:
+            expected = silu * up
+            if dtype == torch.bfloat16:
+                expected = oracle.bf16_round(expected)
+    expected[valid:] = 0
+    np.testing.assert_array_equal(to_np(out).astype(np.float32), expected)
