@@ -11,6 +11,7 @@
 // from run to run; here slots follow the flat assignment order, computed with
 // wavefront ballots and per-chunk counts, and every output is deterministic.
 #include <algorithm>
+#include <type_traits>
 
 #include "moe_common.h"
 
@@ -91,6 +92,12 @@ __global__ __launch_bounds__(kRankThreads) void count_rank_kernel(
 // token row once from x to its K destinations with VB-byte accesses. Blocks
 // e, e+grid, ... also zero the padding rows of expert e.
 //
+// A row that is no multiple of VB bytes ends in a vector that starts VB bytes
+// before its end and rewrites the overlap with the same bytes; vectors then
+// start at any element, which global loads and stores take. Such rows ran
+// element by element before (float32 rows of 1023, 2048 tokens, top-2: 20.8 us a
+// dispatch for 25 MB moved, 11.3 now; bf16 rows of 1537, 4096 tokens: 26.7, 10.9).
+//
 // The source rows do not depend on the destinations, so each thread loads its
 // first kPackEarly vectors of x before the prefix work and stores them after:
 // all blocks start together, and the prefix's dependent global reads and
@@ -101,17 +108,11 @@ constexpr int kPackThreads = 256;
 constexpr int kPackMaxAssign = 256;  // pack_tokens * K upper bound
 constexpr int kPackEarly = 4;        // vectors of x per thread loaded before the prefix
 
-template <int VB> struct VecOf;
-template <> struct VecOf<16> { using T = uint4; };
-template <> struct VecOf<8> { using T = uint2; };
-template <> struct VecOf<4> { using T = uint32_t; };
-template <> struct VecOf<2> { using T = uint16_t; };
-
-template <typename V> __device__ __forceinline__ V zero_vec();
-template <> __device__ __forceinline__ uint4 zero_vec<uint4>() { return make_uint4(0, 0, 0, 0); }
-template <> __device__ __forceinline__ uint2 zero_vec<uint2>() { return make_uint2(0, 0); }
-template <> __device__ __forceinline__ uint32_t zero_vec<uint32_t>() { return 0u; }
-template <> __device__ __forceinline__ uint16_t zero_vec<uint16_t>() { return 0; }
+template <int VB, bool WHOLE> struct VecOf;
+template <> struct VecOf<16, true> { using T = uint4; };
+template <> struct VecOf<16, false> { using T = Unaligned<uint16_t, 8>; };
+template <> struct VecOf<4, true> { using T = uint32_t; };
+template <> struct VecOf<2, true> { using T = uint16_t; };
 
 // COUNT (at most kSmallAssign assignments): no count_rank_kernel; every block
 // ranks all assignments itself (the same ballots, in flat order) and keeps
@@ -127,14 +128,16 @@ constexpr int kSmallAssign = 1024;
 // ROWS: the layout without the rows. Instead of copying x rows into packed,
 // row_src[r] receives the token whose row packed row r would hold (-1 for
 // padding rows), for a GEMM that reads its A rows from x through it.
-template <int VB, bool COUNT, bool ROWS>
+// WHOLE: rows are a multiple of VB bytes at VB-aligned addresses (no overlapping
+// vectors, and at 4096 rows of 8 KiB 3% less time than the general form).
+template <int VB, bool COUNT, bool ROWS, bool WHOLE>
 __global__ __launch_bounds__(kPackThreads) void pack_kernel(
     const char* __restrict__ x, const int32_t* __restrict__ ids, int32_t* slots,
     const int32_t* ranks, const int32_t* __restrict__ chunk_counts, int32_t* __restrict__ counts,
     int32_t* __restrict__ offsets, char* __restrict__ packed, int32_t* __restrict__ inverse,
     int32_t* __restrict__ row_src, int64_t tokens, int64_t row_bytes, int experts, int topk, int alignment,
     int64_t chunk_tokens, int pack_tokens, int n_chunks, int experts_pow2, int64_t packed_rows) {
-    using V = typename VecOf<VB>::T;
+    using V = typename VecOf<VB, WHOLE>::T;
     __shared__ int part_all[kPackThreads / kWave][kMaxExperts];
     __shared__ int part_before[kPackThreads / kWave][kMaxExperts];
     __shared__ int total[kMaxExperts];
@@ -152,11 +155,19 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(
     const int n_tok = static_cast<int>(max<int64_t>(t_end - t0, 0));
     // Item i of this block is vector i % nv of token t0 + i / nv (the launcher
     // keeps pack_tokens * nv within int32).
-    const int nv = static_cast<int>(row_bytes / VB);
+    const int nv = static_cast<int>(WHOLE ? row_bytes / VB : (row_bytes + VB - 1) / VB);
     const int items = n_tok * nv;
+    // Vector v of a row.
+    auto vec_of = [&](auto* row, int v) {
+        using P = std::conditional_t<std::is_const_v<std::remove_pointer_t<decltype(row)>>, const V*, V*>;
+        if constexpr (WHOLE)
+            return reinterpret_cast<P>(row) + v;
+        else
+            return reinterpret_cast<P>(row + min(static_cast<int64_t>(v) * VB, row_bytes - VB));
+    };
     auto src = [&](int i) {
         const int tl = i / nv;
-        return reinterpret_cast<const V*>(x + (t0 + tl) * row_bytes)[i - tl * nv];
+        return *vec_of(x + (t0 + tl) * row_bytes, i - tl * nv);
     };
     V early[kPackEarly];
     if constexpr (!ROWS) {
@@ -314,7 +325,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(
         const int v = i - tl * nv;
         for (int k = 0; k < topk; ++k) {
             const int64_t d = dest[tl * topk + k];
-            if (d >= 0) reinterpret_cast<V*>(packed + d * row_bytes)[v] = val;
+            if (d >= 0) *vec_of(packed + d * row_bytes, v) = val;
         }
     };
     if constexpr (!ROWS) {
@@ -333,9 +344,15 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(
         if constexpr (ROWS) {
             for (int64_t r = r0 + tid; r < r1; r += kPackThreads) row_src[r] = -1;
         } else {
-            const int64_t pad_items = (r1 - r0) * nv;
-            V* base = reinterpret_cast<V*>(packed + r0 * row_bytes);
-            for (int64_t i = tid; i < pad_items; i += kPackThreads) base[i] = zero_vec<V>();
+            if constexpr (WHOLE) {
+                const int64_t pad_items = (r1 - r0) * nv;
+                V* base = reinterpret_cast<V*>(packed + r0 * row_bytes);
+                for (int64_t i = tid; i < pad_items; i += kPackThreads) base[i] = V{};
+            } else {
+                const int64_t bytes = (r1 - r0) * row_bytes;  // at least VB when positive
+                for (int64_t i = static_cast<int64_t>(tid) * VB; i < bytes; i += kPackThreads * VB)
+                    *reinterpret_cast<V*>(packed + r0 * row_bytes + min(i, bytes - VB)) = V{};
+            }
         }
     }
 }
@@ -343,36 +360,50 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(
 // ---------------------------------------------------------------------------
 // Combine: out[t] = round(sum_k w[t,k] * y[inverse[t,k]]) in fp32, k order,
 // separate multiply and add (no contraction), skipped rows outside [0, R).
-// Each thread owns VECS VE-element vectors of one token and issues all
-// K * VECS gathers before reducing.
+// Each thread owns VECS VE-element vectors of one token and gathers its K
+// rows two at a time, their loads issued before reducing (four at a time took
+// 37.6 against 34.4 us at H=2048, 8192 tokens, top-6, and 11.2 against 9.0 at
+// 4096 tokens, top-2: fewer waves fit a CU). As in pack_kernel,
+// the last vector of a row that is no multiple of VE overlaps the one before.
 // ---------------------------------------------------------------------------
-template <int DT, int VE, int VECS>
+// WHOLE: every vector is VE elements of its own at a VE-aligned address.
+template <int DT, int VE, int VECS, bool WHOLE>
 __global__ __launch_bounds__(256) void combine_kernel(
     const typename Elem<DT>::T* __restrict__ y, const int32_t* __restrict__ inverse,
     const float* __restrict__ weights, typename Elem<DT>::T* __restrict__ out, int64_t tokens,
     int64_t hidden, int topk, int64_t rows) {
 #pragma clang fp contract(off)
+    constexpr int KB = 2;
     using T = typename Elem<DT>::T;
-    struct alignas(sizeof(T) * VE) Pack {
+    struct alignas(sizeof(T) * VE) Aligned {
         T v[VE];
     };
-    const int64_t nv = hidden / VE;
+    using Pack = std::conditional_t<WHOLE, Aligned, Unaligned<T, VE>>;
+    const int64_t nv = WHOLE ? hidden / VE : (hidden + VE - 1) / VE;
     const int64_t groups = (nv + VECS - 1) / VECS;  // vector groups per token
     const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     const int64_t t = idx / groups;
     if (t >= tokens) return;
     const int64_t v0 = (idx - t * groups) * VECS;
+    // Vector u of this thread in a row (element indices stay below 2^31 + VE * VECS).
+    auto vec_of = [&](auto* row, int u) {
+        using P = std::conditional_t<std::is_const_v<std::remove_pointer_t<decltype(row)>>, const Pack*, Pack*>;
+        if constexpr (WHOLE)
+            return reinterpret_cast<P>(row) + (v0 + u);
+        else
+            return reinterpret_cast<P>(row + min(static_cast<uint32_t>(v0 + u) * VE, static_cast<uint32_t>(hidden) - VE));
+    };
     float acc[VECS][VE];
 #pragma unroll
     for (int u = 0; u < VECS; ++u)
 #pragma unroll
         for (int j = 0; j < VE; ++j) acc[u][j] = 0.0f;
-    for (int k0 = 0; k0 < topk; k0 += 2) {
-        Pack in[2][VECS];
-        float w[2];
-        bool ok[2];
+    for (int k0 = 0; k0 < topk; k0 += KB) {
+        Pack in[KB][VECS];
+        float w[KB];
+        bool ok[KB];
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
+        for (int kk = 0; kk < KB; ++kk) {
             const int k = k0 + kk;
             ok[kk] = false;
             w[kk] = 0.0f;
@@ -382,15 +413,15 @@ __global__ __launch_bounds__(256) void combine_kernel(
                 ok[kk] = row >= 0 && row < rows;
                 if (ok[kk]) {
                     w[kk] = weights[pa];
-                    const Pack* src = reinterpret_cast<const Pack*>(y + static_cast<int64_t>(row) * hidden);
+                    const T* src = y + static_cast<int64_t>(row) * hidden;
 #pragma unroll
                     for (int u = 0; u < VECS; ++u)
-                        if (v0 + u < nv) in[kk][u] = src[v0 + u];
+                        if (v0 + u < nv) in[kk][u] = *vec_of(src, u);
                 }
             }
         }
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
+        for (int kk = 0; kk < KB; ++kk) {
             if (!ok[kk]) continue;
 #pragma unroll
             for (int u = 0; u < VECS; ++u)
@@ -407,7 +438,7 @@ __global__ __launch_bounds__(256) void combine_kernel(
         Pack o;
 #pragma unroll
         for (int j = 0; j < VE; ++j) o.v[j] = Elem<DT>::store(acc[u][j]);
-        reinterpret_cast<Pack*>(out + t * hidden)[v0 + u] = o;
+        *vec_of(out + t * hidden, u) = o;
     }
 }
 
@@ -579,7 +610,7 @@ static int launch_pack(const void* x, int dtype, const int32_t* ids, int32_t* co
     const int experts_pow2_rows = static_cast<int>(pow2_at_least(experts));
     if (row_src != nullptr) {  // the row table instead of the rows (x and packed unused)
 #define MOE_ROWS_LAUNCH(CNT)                                                                             \
-    hipLaunchKernelGGL((pack_kernel<16, CNT, true>), dim3(static_cast<unsigned>(plan.pack_blocks)),       \
+    hipLaunchKernelGGL((pack_kernel<16, CNT, true, true>), dim3(static_cast<unsigned>(plan.pack_blocks)),       \
                        dim3(kPackThreads), 0, stream, nullptr, ids, slots, ranks, chunk_counts, counts,    \
                        offsets, nullptr, inverse, row_src, tokens, int64_t{16}, experts, topk, alignment, \
                        plan.chunk_tokens, plan.pack_tokens, static_cast<int>(plan.n_chunks),              \
@@ -593,39 +624,34 @@ static int launch_pack(const void* x, int dtype, const int32_t* ids, int32_t* co
     }
     const int64_t elem = dtype_size(dtype);
     const int64_t row_bytes = hidden * elem;
-    // The widest access that divides the row size and both base addresses (an
-    // offset view of a larger tensor may start at any element).
-    int vb = static_cast<int>(elem);
-    if (vectorized) {
-        const uint64_t bits = static_cast<uint64_t>(row_bytes) | reinterpret_cast<uintptr_t>(x) |
-                              reinterpret_cast<uintptr_t>(packed);
-        for (int w : {16, 8, 4}) {
-            if (w > vb && bits % w == 0) {
-                vb = w;
-                break;
-            }
-        }
-    }
-    MOE_REQUIRE(plan.pack_tokens * (row_bytes / vb) <= INT32_MAX, MOE_ERR_UNSUPPORTED,
+    // 16-byte accesses at any element (see pack_kernel), elements for shorter rows.
+    const int vb = vectorized && row_bytes >= 16 ? 16 : static_cast<int>(elem);
+    MOE_REQUIRE(plan.pack_tokens * ((row_bytes + vb - 1) / vb) <= INT32_MAX, MOE_ERR_UNSUPPORTED,
                 "row of %lld bytes too large for the pack kernel", (long long)row_bytes);
     const int experts_pow2 = static_cast<int>(pow2_at_least(experts));
     const dim3 grid(static_cast<unsigned>(plan.pack_blocks));
-#define MOE_PACK_LAUNCH(VBV, CNT)                                                              \
-    hipLaunchKernelGGL((pack_kernel<VBV, CNT, false>), grid, dim3(kPackThreads), 0, stream,     \
+#define MOE_PACK_LAUNCH(VBV, CNT, WHL)                                                           \
+    hipLaunchKernelGGL((pack_kernel<VBV, CNT, false, WHL>), grid, dim3(kPackThreads), 0, stream,     \
                        static_cast<const char*>(x), ids, slots, ranks, chunk_counts, counts, offsets, \
                        static_cast<char*>(packed), inverse, nullptr, tokens, row_bytes, experts, topk, \
                        alignment, plan.chunk_tokens, plan.pack_tokens,                          \
                        static_cast<int>(plan.n_chunks), experts_pow2, packed_rows)
-#define MOE_PACK_CASE(VBV)                 \
+#define MOE_PACK_CASE(VBV, WHL)            \
     if (count_in_pack)                     \
-        MOE_PACK_LAUNCH(VBV, true);        \
+        MOE_PACK_LAUNCH(VBV, true, WHL);   \
     else                                   \
-        MOE_PACK_LAUNCH(VBV, false)
+        MOE_PACK_LAUNCH(VBV, false, WHL)
     switch (vb) {
-        case 16: MOE_PACK_CASE(16); break;
-        case 8: MOE_PACK_CASE(8); break;
-        case 4: MOE_PACK_CASE(4); break;
-        case 2: MOE_PACK_CASE(2); break;
+        case 16:
+            if ((static_cast<uint64_t>(row_bytes) | reinterpret_cast<uintptr_t>(x) |
+                 reinterpret_cast<uintptr_t>(packed)) % 16 == 0) {
+                MOE_PACK_CASE(16, true);
+            } else {
+                MOE_PACK_CASE(16, false);
+            }
+            break;
+        case 4: MOE_PACK_CASE(4, true); break;
+        case 2: MOE_PACK_CASE(2, true); break;
         default: return fail(MOE_ERR_UNSUPPORTED, "row size %lld bytes", (long long)row_bytes);
     }
 #undef MOE_PACK_CASE
@@ -641,38 +667,47 @@ static void launch_combine_t(const void* y, const int32_t* inverse, const float*
     // Two vectors per thread, one for rows of 8 KiB and up (vectorized): at
     // H=4096 bf16, 4096 tokens, top-2, 17.7 against 18.6 us; at H=2048 one
     // vector took 9.85 against 9.46 us.
-    auto go = [&](auto vecs_c) {
+    // Whole, aligned vectors (an offset view of a larger tensor may start at any element).
+    const bool whole = hidden % VE == 0 &&
+                       (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(out)) % (sizeof(T) * VE) == 0;
+    auto go = [&](auto vecs_c, auto whole_c) {
         constexpr int VECS = decltype(vecs_c)::value;
-        const int64_t groups = (hidden / VE + VECS - 1) / VECS;
+        constexpr bool WHOLE = decltype(whole_c)::value;
+        const int64_t groups = ((hidden + VE - 1) / VE + VECS - 1) / VECS;
         const int64_t threads = tokens * groups;
         const dim3 grid(static_cast<unsigned>((threads + 255) / 256));
-        hipLaunchKernelGGL((combine_kernel<DT, VE, VECS>), grid, dim3(256), 0, stream,
+        hipLaunchKernelGGL((combine_kernel<DT, VE, VECS, WHOLE>), grid, dim3(256), 0, stream,
                            static_cast<const T*>(y), inverse, weights, static_cast<T*>(out), tokens,
                            hidden, topk, rows);
     };
-    if (VE > 1 && hidden * static_cast<int64_t>(sizeof(T)) >= 8192)
-        go(std::integral_constant<int, 1>{});
+    auto vecs = [&](auto whole_c) {
+        if (VE > 1 && hidden * static_cast<int64_t>(sizeof(T)) >= 8192)
+            go(std::integral_constant<int, 1>{}, whole_c);
+        else
+            go(std::integral_constant<int, 2>{}, whole_c);
+    };
+    if (VE == 1 || whole)
+        vecs(std::true_type{});
     else
-        go(std::integral_constant<int, 2>{});
+        vecs(std::false_type{});
 }
 
 int launch_combine(const void* y, int dtype, const int32_t* inverse, const float* weights,
                    void* out, int64_t tokens, int64_t hidden, int topk, int64_t rows,
                    hipStream_t stream) {
     if (tokens == 0) return MOE_OK;
-    // 16-byte vectors need both row arrays 16-byte aligned (rows then are too).
-    const bool vec_ok = (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+    // 16-byte vectors at any element, elements for rows shorter than one.
     switch (dtype) {
         case MOE_DTYPE_BF16:
-            if (vec_ok && hidden % 8 == 0) launch_combine_t<MOE_DTYPE_BF16, 8>(y, inverse, weights, out, tokens, hidden, topk, rows, stream);
+            if (hidden >= 8) launch_combine_t<MOE_DTYPE_BF16, 8>(y, inverse, weights, out, tokens, hidden, topk, rows, stream);
             else launch_combine_t<MOE_DTYPE_BF16, 1>(y, inverse, weights, out, tokens, hidden, topk, rows, stream);
             break;
         case MOE_DTYPE_F16:
-            if (vec_ok && hidden % 8 == 0) launch_combine_t<MOE_DTYPE_F16, 8>(y, inverse, weights, out, tokens, hidden, topk, rows, stream);
+            if (hidden >= 8) launch_combine_t<MOE_DTYPE_F16, 8>(y, inverse, weights, out, tokens, hidden, topk, rows, stream);
             else launch_combine_t<MOE_DTYPE_F16, 1>(y, inverse, weights, out, tokens, hidden, topk, rows, stream);
             break;
         case MOE_DTYPE_F32:
-            if (vec_ok && hidden % 4 == 0) launch_combine_t<MOE_DTYPE_F32, 4>(y, inverse, weights, out, tokens, hidden, topk, rows, stream);
+            if (hidden >= 4) launch_combine_t<MOE_DTYPE_F32, 4>(y, inverse, weights, out, tokens, hidden, topk, rows, stream);
             else launch_combine_t<MOE_DTYPE_F32, 1>(y, inverse, weights, out, tokens, hidden, topk, rows, stream);
             break;
         default: return fail(MOE_ERR_INVALID_ARGUMENT, "unknown dtype %d", dtype);

@@ -178,6 +178,42 @@ def test_reference_runtime_validation_suite(ext):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("row_bytes", [4, 12, 16, 20, 28, 32, 44, 1020, 4092])
+def test_rows_of_any_length_and_offset_views(ext, dtype, row_bytes):
+    """Rows shorter than, equal to and past whole 16-byte vectors (the last vector
+    overlaps the one before), from tensors that start at any element, with padding
+    rows to zero; nothing outside the rows is written."""
+    hidden = row_bytes // torch.empty((), dtype=dtype).element_size()
+    tokens, experts, topk, alignment = 70, 6, 3, 8
+    _, i32, i64, w = make_transport_case(tokens, hidden, experts, topk, dtype, seed=row_bytes)
+
+    def view(rows, offset, fill=None):
+        flat = torch.randn(rows * hidden + 32, device="cuda").to(dtype)
+        if fill is not None:
+            flat.fill_(fill)
+        return flat, flat[offset:offset + rows * hidden].view(rows, hidden)
+
+    _, x = view(tokens, 1)
+    layout = oracle.dispatch_layout(to_np(i32), experts, alignment)
+    rows = CudaWorkspace(tokens, hidden, experts, topk, dtype, alignment=alignment, extension=ext).capacity_rows
+    used = int(layout["offsets"][-1])
+    for offset in (0, 3):
+        store, packed = view(rows, offset, 7.0)
+        index = [torch.empty(n, device="cuda", dtype=torch.int32) for n in (experts, experts + 1, tokens * topk)]
+        inverse = torch.empty(tokens, topk, device="cuda", dtype=torch.int32)
+        ext.dispatch_aligned_out(x, i32, index[0], index[1], index[2], packed, inverse, True, alignment)
+        assert_packed_equal(packed, x, layout, topk)
+        np.testing.assert_array_equal(to_np(inverse), layout["inverse"])
+        assert torch.all(store[:offset] == 7.0) and torch.all(store[offset + used * hidden:] == 7.0)
+        out_store, out = view(tokens, offset, 7.0)
+        _, y = view(rows, 5)
+        ext.combine_out(y, inverse, w, out)
+        expected = oracle.combine(to_np(y), layout["inverse"], to_np(w), NP_DTYPE[dtype])
+        np.testing.assert_array_equal(to_np(out), expected)
+        assert torch.all(out_store[:offset] == 7.0) and torch.all(out_store[offset + tokens * hidden:] == 7.0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rows,width", [(5, 1), (3, 7), (9, 8), (300, 9), (40, 257), (2, 2049), (3000, 40)])
 def test_standalone_swiglu_widths(ext, dtype, rows, width):
     """Widths around whole vectors, rows and blocks, with special gate values: bit-exact
