@@ -172,49 +172,73 @@ __global__ __launch_bounds__(256) void router_split_kernel(const float* __restri
 // Rows of 128 bytes hold 8 chunks of 16 bytes; chunk c of row r sits at
 // physical chunk c ^ ((r >> 1) & 7), so 16 lanes reading 16 consecutive rows
 // at one chunk are conflict free.
+// The value of another lane of the same eight: the neighbour (STEP 0), the lane
+// two further (1), and for values equal inside each half of the eight the other
+// half's (2, a mirror). DPP moves take a few cycles where a shuffle goes through
+// LDS, and a selection has 6 * K of them one after another.
+template <int STEP>
+__device__ __forceinline__ int eight_lane_peer(int v) {
+    constexpr int ctrl = STEP == 0 ? 0xB1 : STEP == 1 ? 0x4E : 0x141;  // quad_perm 1032, 2301, row_half_mirror
+    return __builtin_amdgcn_update_dpp(v, v, ctrl, 0xf, 0xf, false);
+}
+
 // Top-k over one token's biased logits held by eight lanes (lane `sub` holds
 // experts sub*EPL .. sub*EPL+EPL-1; -inf past E). K rounds of: argmax over
 // the lane's values (the lower expert wins a tie), the same across the eight
-// lanes with three xor shuffles, then the winner is removed -- the
-// reference's iterative argmax with ties to the lower id. Lane 0 writes.
+// lanes in three exchanges, then the winner is removed -- the
+// reference's iterative argmax with ties to the lower id. Lane j keeps round j's
+// winner, so the weights (write_route's, in its order: K = 1 and 2 are cases of
+// the general form, whose first term is exactly 1) take one exp, and a lane
+// each stores the ids and weights. With the rounds unrolled into register
+// arrays that one lane turned into weights and stores, the selection was 6-8 KB
+// of straight-line code, and fetching it cost the small routers more than their
+// products. With the rank step below, H=2048, E=64, top-6 went from 30.8 to 19.1
+// us at 1000 tokens and 22.3 to 19.8 at 8192; H=4096, E=8, top-2, 4096 tokens 8.5
+// to 7.7; H=1000, E=12, top-3, 777 tokens 6.6 to 4.9.
 template <int EPL>
 __device__ __forceinline__ void select_eight_lanes(float (&v)[EPL], int sub, int topk, int64_t token,
                                                    int32_t* ids32, int64_t* ids64, float* weights,
                                                    int* tile_ids = nullptr) {
-    float sel_v[kMaxTopk];
-    int sel_i[kMaxTopk];
+    float first = 0.0f, value = 0.0f;  // round 0's winner; this lane's round's
+    int id = 0;
+#pragma unroll 1
+    for (int k = 0; k < topk; ++k) {
+        float bv = v[0];
+        int bi = sub * EPL;
 #pragma unroll
-    for (int k = 0; k < kMaxTopk; ++k) {
-        if (k < topk) {
-            float bv = v[0];
-            int bi = sub * EPL;
-#pragma unroll
-            for (int j = 1; j < EPL; ++j) {
-                const bool take = v[j] > bv;
-                bv = take ? v[j] : bv;
-                bi = take ? sub * EPL + j : bi;
-            }
-#pragma unroll
-            for (int msk = 1; msk < 8; msk <<= 1) {
-                const float ov = __shfl_xor(bv, msk);
-                const int oi = __shfl_xor(bi, msk);
-                const bool take = ov > bv || (ov == bv && oi < bi);
-                bv = take ? ov : bv;
-                bi = take ? oi : bi;
-            }
-            sel_v[k] = bv;
-            sel_i[k] = bi;
-#pragma unroll
-            for (int j = 0; j < EPL; ++j) v[j] = (sub * EPL + j == bi) ? -INFINITY : v[j];
+        for (int j = 1; j < EPL; ++j) {
+            const bool take = v[j] > bv;
+            bv = take ? v[j] : bv;
+            bi = take ? sub * EPL + j : bi;
         }
+        static_for<3>([&](auto step_c) {
+            const float ov = __int_as_float(eight_lane_peer<decltype(step_c)::value>(__float_as_int(bv)));
+            const int oi = eight_lane_peer<decltype(step_c)::value>(bi);
+            const bool take = ov > bv || (ov == bv && oi < bi);
+            bv = take ? ov : bv;
+            bi = take ? oi : bi;
+        });
+        first = k == 0 ? bv : first;
+        value = sub == k ? bv : value;
+        id = sub == k ? bi : id;
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) v[j] = (sub * EPL + j == bi) ? -INFINITY : v[j];
     }
-    if (sub == 0) {
-        write_route(sel_v, sel_i, topk, token, ids32, ids64, weights);
-        if (tile_ids) {
+    const float rel = expf(value - first);
+    const int lane0 = static_cast<int>(threadIdx.x & 63) - sub;
+    float total = 0.0f;
 #pragma unroll
-            for (int k = 0; k < kMaxTopk; ++k)
-                if (k < topk) tile_ids[k] = sel_i[k];
-        }
+    for (int j = 0; j < kMaxTopk; ++j) {
+        const float r = __shfl(rel, lane0 + j);
+        total = j < topk ? total + r : total;
+    }
+    const float weight = rel * (1.0f / total);
+    if (sub < topk) {
+        const int64_t at = token * topk + sub;
+        ids32[at] = id;
+        if (ids64) ids64[at] = id;
+        weights[at] = weight;
+        if (tile_ids) tile_ids[sub] = id;
     }
 }
 
@@ -224,8 +248,9 @@ __device__ __forceinline__ void select_eight_lanes(float (&v)[EPL], int sub, int
 // order). One wave walks them in rounds of 64: lanes holding the same id are
 // found by intersecting six bit-plane ballots, and a lane's rank is the number
 // of such lanes below it plus its expert's count from earlier rounds, which
-// lane e keeps in a register (read with a cross-lane shuffle; one ballot per
-// expert adds each round's counts). ranks[p] <- rank of assignment p among
+// lane e keeps in a register (read with a cross-lane shuffle; lane e finds each
+// round's lanes with expert e by intersecting the same ballots by its own
+// number's bits). ranks[p] <- rank of assignment p among
 // the tile's earlier assignments to the same expert; counts_row[e] <- the
 // tile's assignments to expert e.
 __device__ __forceinline__ void rank_tile(const int* tile_ids, int n, int64_t p0, int experts, int32_t* ranks,
@@ -237,19 +262,17 @@ __device__ __forceinline__ void rank_tile(const int* tile_ids, int n, int64_t p0
         const int i = base + lane;
         const bool valid = i < n;
         const int e = valid ? tile_ids[i] : 0;
-        uint64_t same = __ballot(valid);
+        uint64_t same = __ballot(valid), mine = same;
 #pragma unroll
         for (int b = 0; b < 6; ++b) {
             const bool bit = (e >> b) & 1;
             const uint64_t plane = __ballot(valid && bit);
             same &= bit ? plane : ~plane;
+            mine &= (lane >> b) & 1 ? plane : ~plane;
         }
         const int prior = __shfl(run, e);
         if (valid) ranks[p0 + i] = prior + __popcll(same & lanes_below);
-        for (int x = 0; x < experts; ++x) {
-            const int c = __popcll(__ballot(valid && e == x));
-            if (lane == x) run += c;
-        }
+        run += __popcll(mine);
     }
     if (lane < experts) counts_row[lane] = run;
 }
