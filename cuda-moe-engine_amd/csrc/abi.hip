@@ -14,6 +14,11 @@ int launch_topk_route(const float*, const float*, int32_t*, int64_t*, float*, in
                       hipStream_t);
 int launch_router_fused(const uint16_t*, const float*, const float*, int32_t*, int64_t*, float*,
                         float*, uint16_t*, int64_t, int, int, int, int32_t*, int32_t*, hipStream_t);
+int64_t route_rows_bytes(int64_t tokens, int64_t hidden, int64_t experts, int64_t topk);
+int launch_route_rows(const uint16_t* x, const float* router_w, const float* bias, int32_t* ids32, int64_t* ids64,
+                      float* weights, uint16_t* planes, float* sums, int32_t* counts, int32_t* offsets,
+                      int32_t* slots, int32_t* inverse, int32_t* row_src, int tokens, int hidden, int experts,
+                      int topk, int alignment, int64_t packed_rows, hipStream_t stream);
 int64_t router_rank_tile(int64_t, int64_t);
 int launch_router_split(const float*, uint16_t*, int, int, hipStream_t);
 int64_t router_scratch_bytes(int64_t, int64_t);
@@ -353,6 +358,36 @@ int moe_dispatch_ranked_rows(const int32_t* ids, int32_t* counts, int32_t* offse
     return launch_dispatch_rows(ids, counts, offsets, slots, inverse, row_src, ranks,
                                 const_cast<int32_t*>(tile_counts), tile, tokens, (int)experts, (int)topk,
                                 (int)alignment, packed_rows, static_cast<hipStream_t>(stream));
+}
+
+int64_t moe_route_rows_scratch_bytes(int64_t tokens, int64_t hidden, int64_t experts, int64_t topk) {
+    if (tokens < 1 || hidden < 8 || hidden % 8 != 0 || experts < 1 || experts > kMaxExperts || topk < 1 ||
+        topk > kMaxTopk || topk > experts)
+        return -1;
+    return route_rows_bytes(tokens, hidden, experts, topk);
+}
+
+int moe_route_rows(const void* x, const float* router_w, const float* bias, int32_t* ids32, int64_t* ids64,
+                   float* weights, void* scratch, int64_t scratch_bytes, int32_t* counts, int32_t* offsets,
+                   int32_t* slots, int32_t* inverse, int32_t* row_src, void* sums, int64_t sums_bytes,
+                   int64_t tokens, int64_t hidden, int64_t experts, int64_t topk, int64_t alignment,
+                   int64_t packed_rows, void* stream) {
+    int rc = check_router_fused(x, router_w, bias, ids32, ids64, weights, nullptr, scratch, scratch_bytes, tokens,
+                                hidden, experts, topk);
+    if (rc != MOE_OK) return rc;
+    rc = check_dispatch_rows(ids32, counts, offsets, slots, inverse, row_src, nullptr, tokens, experts, topk,
+                             alignment, packed_rows);
+    if (rc != MOE_OK) return rc;
+    const int64_t need = moe_route_rows_scratch_bytes(tokens, hidden, experts, topk);
+    MOE_REQUIRE(need >= 0, MOE_ERR_UNSUPPORTED,
+                "no one-pass route for %lld tokens (moe_route_rows_scratch_bytes returned -1)", (long long)tokens);
+    MOE_REQUIRE(sums_bytes >= need && (need == 0 || sums), MOE_ERR_WORKSPACE, "plane sums need %lld bytes, got %lld",
+                (long long)need, (long long)sums_bytes);
+    MOE_REQUIRE(aligned_to(sums, 16), MOE_ERR_INVALID_ARGUMENT, "plane sums must be 16-byte aligned");
+    return launch_route_rows(static_cast<const uint16_t*>(x), router_w, bias, ids32, ids64, weights,
+                             static_cast<uint16_t*>(scratch), static_cast<float*>(sums), counts, offsets, slots,
+                             inverse, row_src, (int)tokens, (int)hidden, (int)experts, (int)topk, (int)alignment,
+                             packed_rows, static_cast<hipStream_t>(stream));
 }
 
 int moe_combine(const void* expert_output, int dtype, const int32_t* inverse,

@@ -828,6 +828,302 @@ __global__ __launch_bounds__(kWideWaves * 64) void router_wide_kernel(
     }
 }
 
+// ---------------------------------------------------------------------------
+// Small batches: routing in few blocks, and with the whole batch's ids in one
+// block also the dispatch's row-table layout (moe_route_rows), so that a
+// decoding step spends one or two launches before its GEMMs where the router
+// (one or two kernels) and the row-table dispatch took two or three.
+// ---------------------------------------------------------------------------
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallWaves = kSmallThreads / kWave;
+constexpr int kSmallTokens = 128;           // eight lanes per token in the selection
+constexpr int kSmallRouteAssign = 1024;     // one thread per assignment in the layout
+
+// Outputs of the row-table layout (all null: none).
+struct RowsOut {
+    int32_t *counts, *offsets, *slots, *inverse, *row_src;
+    int alignment;
+    int64_t packed_rows;
+};
+
+// The row-table layout of n = tokens * topk <= 1024 assignments whose expert
+// ids sit in LDS in flat order, by one block of 1024 threads: slots are ranks in
+// flat order, spans are aligned, as pack_kernel writes them. Ballots rank each
+// wave's 64 assignments; the waves' counts are prefixed through LDS.
+__device__ __forceinline__ void write_rows_layout(const int* ids, int n, int experts, int topk, const RowsOut& o) {
+    __shared__ int wave_counts[kSmallWaves][kMaxExperts];  // then: the counts of earlier waves
+    __shared__ int total[kMaxExperts];
+    __shared__ int offs[kMaxExperts + 1];
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+    const uint64_t lanes_below = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
+    for (int i = tid; i < kSmallWaves * kMaxExperts; i += kSmallThreads) (&wave_counts[0][0])[i] = 0;
+    __syncthreads();
+    const bool valid = tid < n;
+    const int e = valid ? ids[tid] : -1;
+    const bool in_range = valid && e >= 0 && e < experts;
+    uint64_t same = __ballot(in_range);
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+        const bool bit = (e >> b) & 1;
+        const uint64_t plane = __ballot(in_range && bit);
+        same &= bit ? plane : ~plane;
+    }
+    const int rank = __popcll(same & lanes_below);
+    if (in_range && rank == 0) wave_counts[wave][e] = __popcll(same);
+    __syncthreads();
+    if (wave == 0) {
+        int run = 0;
+#pragma unroll
+        for (int w = 0; w < kSmallWaves; ++w) {
+            const int c = wave_counts[w][lane];
+            wave_counts[w][lane] = run;
+            run += c;
+        }
+        int incl = (run + o.alignment - 1) / o.alignment * o.alignment;
+        for (int d = 1; d < kWave; d <<= 1) {
+            const int up = __shfl_up(incl, d);
+            if (lane >= d) incl += up;
+        }
+        total[lane] = run;
+        offs[lane + 1] = incl;
+        if (lane == 0) offs[0] = 0;
+        if (lane < experts) {
+            o.counts[lane] = run;
+            o.offsets[lane + 1] = incl;
+        }
+        if (lane == 0) o.offsets[0] = 0;
+    }
+    __syncthreads();
+    if (valid) {
+        int slot = -1;
+        if (in_range) {
+            slot = wave_counts[wave][e] + rank;
+            const int64_t row = static_cast<int64_t>(offs[e]) + slot;
+            if (row < o.packed_rows) {
+                o.inverse[tid] = static_cast<int32_t>(row);
+                o.row_src[row] = tid / topk;
+            }
+        }
+        o.slots[tid] = slot;
+    }
+    // Padding rows, one expert per wave in turn.
+    for (int x = wave; x < experts; x += kSmallWaves)
+        for (int64_t r = offs[x] + total[x] + lane; r < min(static_cast<int64_t>(offs[x + 1]), o.packed_rows); r += kWave)
+            o.row_src[r] = -1;
+}
+
+// E <= 16, hidden <= 8192, at most 16 tokens: the batch in one block of 16 waves
+// that split the 64-k steps, on router_direct_kernel's operands. Bound by the
+// latency of its loads, exchanges and code, not by bytes. H=4096, E=8, with the
+// layout: 6.9 us at one token and 7.9 at 16, where split-k partials, their sum
+// and the pack kernel took 12.6 and 13.8. Two or more token tiles in the block
+// lost to one block each and a separate row-table dispatch (17 tokens: 10.0
+// against 9.7 us; 128 tokens of 512: 8.8 against 7.9).
+template <int F>
+constexpr int small_depth() {  // 1024 threads leave 128 VGPRs a lane
+    return 22 / (2 + F);
+}
+
+template <int PER, int F>
+__global__ __launch_bounds__(kSmallThreads) void route_small_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ frags, const float* __restrict__ bias,
+    int32_t* __restrict__ ids32, int64_t* __restrict__ ids64, float* __restrict__ weights,
+    float* __restrict__ logits_out, int tokens, int hidden, int experts, int topk, int32_t* __restrict__ ranks,
+    int32_t* __restrict__ tile_counts, RowsOut rows_out) {
+    constexpr int TB = kRouterTokens, PR = 8 * F, PRP = 2 * PR + 1;
+    constexpr int D = small_depth<F>() < PER ? small_depth<F>() : PER;
+    __shared__ float part[kSmallWaves][TB][PRP];  // [wave][token][half * PR + plane row]
+    __shared__ float sums[TB][PR + 1];             // [token][plane row]
+    __shared__ float sbias[kDirectMaxExperts];
+    __shared__ int ids_lds[TB * kMaxTopk];
+    static_assert(TB * PR <= kSmallThreads, "a thread per plane sum");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t row_bytes = static_cast<uint32_t>(hidden) * 2;
+    const int steps = (hidden + 63) / 64;
+    const __amdgpu_buffer_rsrc_t rsrc_x = make_rsrc(x, static_cast<uint32_t>(tokens) * row_bytes);
+    const __amdgpu_buffer_rsrc_t rsrc_f = make_rsrc(frags, static_cast<uint32_t>(steps) * F * 1024u);
+    const int per = (steps + kSmallWaves - 1) / kSmallWaves;  // <= PER (the launcher's choice)
+    const int s_begin = min(steps, wave * per);
+    const int s_end = min(steps, s_begin + per);
+    const int m = lane & 15, kq = lane >> 4, h = m & 1;
+    const int k_lane = h * 32 + kq * 8;
+    const uint32_t x_off = static_cast<uint32_t>(m >> 1) * row_bytes + k_lane * 2;
+    struct Frag {
+        ru32x4_t a[2], b[F];
+    };
+    auto load = [&](int s, Frag& fr) {
+        const bool in = s < s_end;
+        const bool k_in = in && s * 64 + k_lane < hidden;
+        const uint32_t k_bytes = static_cast<uint32_t>(s) * 128;
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+            fr.a[g] = __builtin_amdgcn_raw_buffer_load_b128(
+                rsrc_x, k_in ? x_off + g * 8 * row_bytes + k_bytes : kRouterOob, 0, 0);
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+            fr.b[f] = __builtin_amdgcn_raw_buffer_load_b128(
+                rsrc_f, in ? static_cast<uint32_t>((s * F + f) * 64 + lane) * 16 : kRouterOob, 0, 0);
+    };
+    rfloatx4_t acc[2][F];
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int f = 0; f < F; ++f) acc[g][f] = rfloatx4_t{0.f, 0.f, 0.f, 0.f};
+    Frag fr[D];
+    static_for<D>([&](auto u_c) { load(s_begin + decltype(u_c)::value, fr[decltype(u_c)::value]); });
+    if (threadIdx.x < experts) sbias[threadIdx.x] = bias[threadIdx.x];
+    static_for<PER>([&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int f = 0; f < F; ++f)
+                acc[g][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(rbf16x8_t, fr[i % D].a[g]),
+                                                                    __builtin_bit_cast(rbf16x8_t, fr[i % D].b[f]),
+                                                                    acc[g][f], 0, 0, 0);
+        if constexpr (i + D < PER) load(s_begin + i + D, fr[i % D]);
+        __builtin_amdgcn_sched_barrier(0);
+    });
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+#pragma unroll
+            for (int jj = 0; jj < 2; ++jj) {
+                const int j = 2 * jj + h;
+                part[wave][8 * g + 2 * kq + jj][h * PR + 8 * f + (m >> 1)] = acc[g][f][j];
+            }
+    __syncthreads();
+    // Plane sums over the halves and the waves, in order, a thread each (as a loop
+    // of the selecting lanes, the chain of LDS reads took 5 us).
+    if (threadIdx.x < TB * PR) {
+        const int t = threadIdx.x / PR, pr = threadIdx.x % PR;
+        float v[kSmallWaves];
+#pragma unroll
+        for (int w = 0; w < kSmallWaves; ++w) v[w] = part[w][t][pr] + part[w][t][PR + pr];
+        float sum = v[0];
+#pragma unroll
+        for (int w = 1; w < kSmallWaves; ++w) sum = sum + v[w];
+        sums[t][pr] = sum;
+    }
+    __syncthreads();
+    constexpr int EPL = kDirectMaxExperts / 8;
+    const int token = threadIdx.x >> 3, sub = threadIdx.x & 7;
+    if (token < tokens) {  // uniform across each group of eight lanes
+        float v[EPL];
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) {
+            const int e = min(sub * EPL + j, experts - 1);
+            const float* q = sums[token] + e;
+            const float logit = (q[2 * experts] + q[experts]) + q[0];
+            const bool in = sub * EPL + j < experts;
+            if (logits_out && in) logits_out[token * experts + e] = logit;
+            v[j] = in ? logit + sbias[e] : -INFINITY;
+        }
+        select_eight_lanes<EPL>(v, sub, topk, token, ids32, ids64, weights, ids_lds + token * topk);
+    }
+    __syncthreads();
+    if (ranks && wave == 0) rank_tile(ids_lds, tokens * topk, 0, experts, ranks, tile_counts);
+    if (rows_out.counts) write_rows_layout(ids_lds, tokens * topk, experts, topk, rows_out);
+}
+
+// 16 < E <= 64, hidden <= 4096, first of two kernels: block (tile, fragment) is
+// one wave that multiplies one weight fragment with G groups of 8 tokens over
+// the whole k range and writes the plane sums [token][3][64]. Each sum is the same
+// MFMA chain, and its halves are added, as in router_wide_kernel, so the logits
+// are bit-identical to its. One block of that kernel moves 1.25 MiB through one
+// CU's load units for up to 32 tokens (17-19 us at H=2048, E=64); here that is
+// spread over ceil(6E/16) CUs (3-5 us), and the finishing block takes about 5.
+constexpr int kPlaneSums = 3 * kMaxExperts;  // floats per token
+
+template <int PER, int G>
+__global__ __launch_bounds__(kWave) void route_planes_kernel(const uint16_t* __restrict__ x,
+                                                             const uint16_t* __restrict__ frags,
+                                                             float* __restrict__ sums, int tokens, int hidden,
+                                                             int experts, int fragments) {
+    constexpr int kAhead = 40 / (G + 1);
+    constexpr int D = kAhead < PER ? kAhead : PER;
+    const int lane = threadIdx.x;
+    const int tile = static_cast<int>(blockIdx.x) / fragments;
+    const int f = static_cast<int>(blockIdx.x) - tile * fragments;
+    const int t0 = tile * 8 * G;
+    const uint32_t row_bytes = static_cast<uint32_t>(hidden) * 2;
+    const int steps = (hidden + 63) / 64;  // <= PER (the launcher's choice)
+    const __amdgpu_buffer_rsrc_t rsrc_x =
+        make_rsrc(x + static_cast<int64_t>(t0) * hidden, static_cast<uint32_t>(min(8 * G, tokens - t0)) * row_bytes);
+    const __amdgpu_buffer_rsrc_t rsrc_f = make_rsrc(frags, static_cast<uint32_t>(steps) * fragments * 1024u);
+    const int m = lane & 15, kq = lane >> 4, h = m & 1;
+    const int k_lane = h * 32 + kq * 8;
+    const uint32_t x_off = static_cast<uint32_t>(m >> 1) * row_bytes + k_lane * 2;
+    struct Frag {
+        ru32x4_t a[G], b;
+    };
+    auto load = [&](int s, Frag& fr) {
+        const bool in = s < steps;
+        const bool k_in = in && s * 64 + k_lane < hidden;
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            fr.a[g] = __builtin_amdgcn_raw_buffer_load_b128(
+                rsrc_x, k_in ? x_off + g * 8 * row_bytes + static_cast<uint32_t>(s) * 128 : kRouterOob, 0, 0);
+        fr.b = __builtin_amdgcn_raw_buffer_load_b128(
+            rsrc_f, in ? static_cast<uint32_t>((s * fragments + f) * 64 + lane) * 16 : kRouterOob, 0, 0);
+    };
+    rfloatx4_t acc[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[g] = rfloatx4_t{0.f, 0.f, 0.f, 0.f};
+    Frag fr[D];
+    static_for<D>([&](auto u_c) { load(decltype(u_c)::value, fr[decltype(u_c)::value]); });
+    static_for<PER>([&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(rbf16x8_t, fr[i % D].a[g]),
+                                                             __builtin_bit_cast(rbf16x8_t, fr[i % D].b), acc[g], 0, 0, 0);
+        if constexpr (i + D < PER) load(i + D, fr[i % D]);
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    const int pr = 8 * f + (m >> 1);
+    const int plane = pr / experts, e = pr - plane * experts;
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj) {
+            const float own = h ? acc[g][2 * jj + 1] : acc[g][2 * jj];  // this lane's half
+            const float sum = own + __shfl_xor(own, 1);
+            const int token = t0 + 8 * g + 2 * kq + jj;
+            if (h == 0 && token < tokens && pr < 3 * experts) sums[token * kPlaneSums + plane * kMaxExperts + e] = sum;
+        }
+}
+
+// Second: the batch's logits from the plane sums, the selection and the
+// row-table layout, in one block.
+__global__ __launch_bounds__(kSmallThreads) void route_finish_kernel(
+    const float* __restrict__ sums, const float* __restrict__ bias, int32_t* __restrict__ ids32,
+    int64_t* __restrict__ ids64, float* __restrict__ weights, int tokens, int experts, int topk, RowsOut rows_out) {
+    __shared__ int ids_lds[kSmallRouteAssign];
+    constexpr int EPL = kMaxExperts / 8;
+    const int token = threadIdx.x >> 3, sub = threadIdx.x & 7;
+    if (token < tokens) {
+        // Entries past E are never written: their lanes hold -inf whatever they read.
+        float q[3][EPL], v[EPL];
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+#pragma unroll
+            for (int j = 0; j < EPL; j += 4)
+                *reinterpret_cast<float4*>(&q[p][j]) =
+                    *reinterpret_cast<const float4*>(sums + token * kPlaneSums + p * kMaxExperts + sub * EPL + j);
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) {
+            const int e = min(sub * EPL + j, experts - 1);
+            v[j] = sub * EPL + j < experts ? ((q[2][j] + q[1][j]) + q[0][j]) + bias[e] : -INFINITY;
+        }
+        select_eight_lanes<EPL>(v, sub, topk, token, ids32, ids64, weights, ids_lds + token * topk);
+    }
+    __syncthreads();
+    write_rows_layout(ids_lds, tokens * topk, experts, topk, rows_out);
+}
+
 // Sum of a token tile's k-slices in slice order, the bias, and the same
 // selection as router_ring_kernel (16 tokens x 16 expert slots, E <= 16).
 __global__ __launch_bounds__(256) void router_reduce_kernel(
@@ -954,6 +1250,84 @@ int64_t router_rank_tile(int64_t tokens, int64_t experts) {
     return tile;
 }
 
+// Whether a batch routes in one block (route_small_kernel).
+static bool small_route(int64_t tokens, int64_t hidden, int64_t experts) {
+    return experts <= kDirectMaxExperts && tokens > 0 && tokens <= kRouterTokens && hidden <= 8192;
+}
+
+static int launch_route_small(const uint16_t* x, const uint16_t* frags, const float* bias, int32_t* ids32,
+                              int64_t* ids64, float* weights, float* logits_out, int tokens, int hidden, int experts,
+                              int topk, int32_t* ranks, int32_t* tile_counts, const RowsOut& rows,
+                              hipStream_t stream) {
+    const int per = ((hidden + 63) / 64 + kSmallWaves - 1) / kSmallWaves;
+#define MOE_SMALL_CASE(P, FV)                                                                                  \
+    hipLaunchKernelGGL((route_small_kernel<P, FV>), dim3(1), dim3(kSmallThreads), 0, stream, x, frags, bias, ids32, \
+                       ids64, weights, logits_out, tokens, hidden, experts, topk, ranks, tile_counts, rows)
+#define MOE_SMALL_PER(FV)                   \
+    if (per <= 2) MOE_SMALL_CASE(2, FV);      \
+    else if (per <= 4) MOE_SMALL_CASE(4, FV); \
+    else MOE_SMALL_CASE(8, FV);
+    switch (router_fragments(experts)) {
+        case 1: MOE_SMALL_PER(1) break;
+        case 2: MOE_SMALL_PER(2) break;
+        case 3: MOE_SMALL_PER(3) break;
+        case 4: MOE_SMALL_PER(4) break;
+        case 5: MOE_SMALL_PER(5) break;
+        default: MOE_SMALL_PER(6) break;
+    }
+#undef MOE_SMALL_PER
+#undef MOE_SMALL_CASE
+    return check_launch("route_small_kernel");
+}
+
+// Bytes of plane sums launch_route_rows needs, or -1 when the shape has no
+// small-batch route (then moe_router_fused and a dispatch).
+int64_t route_rows_bytes(int64_t tokens, int64_t hidden, int64_t experts, int64_t topk) {
+    if (small_route(tokens, hidden, experts)) return 0;
+    if (experts <= kDirectMaxExperts || tokens <= 0 || tokens > kSmallTokens || tokens * topk > kSmallRouteAssign ||
+        (hidden + 63) / 64 > kWideMaxPer)
+        return -1;
+    return tokens * kPlaneSums * static_cast<int64_t>(sizeof(float));
+}
+
+int launch_route_rows(const uint16_t* x, const float* router_w, const float* bias, int32_t* ids32, int64_t* ids64,
+                      float* weights, uint16_t* planes, float* sums, int32_t* counts, int32_t* offsets,
+                      int32_t* slots, int32_t* inverse, int32_t* row_src, int tokens, int hidden, int experts,
+                      int topk, int alignment, int64_t packed_rows, hipStream_t stream) {
+    if (router_w != nullptr) {
+        const int rc = launch_router_split(router_w, planes, experts, hidden, stream);
+        if (rc != MOE_OK) return rc;
+    }
+    const RowsOut rows{counts, offsets, slots, inverse, row_src, alignment, packed_rows};
+    const uint16_t* frags = reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(planes) +
+                                                              router_fragments_offset(experts, hidden));
+    if (small_route(tokens, hidden, experts))
+        return launch_route_small(x, frags, bias, ids32, ids64, weights, nullptr, tokens, hidden, experts, topk,
+                                  nullptr, nullptr, rows, stream);
+    const int fragments = router_fragments(experts);
+    const int steps = (hidden + 63) / 64;
+#define MOE_PLANES_CASE(P, GV)                                                                                 \
+    hipLaunchKernelGGL((route_planes_kernel<P, GV>),                                                           \
+                       dim3(static_cast<unsigned>((tokens + 8 * GV - 1) / (8 * GV) * fragments)), dim3(kWave), 0, \
+                       stream, x, frags, sums, tokens, hidden, experts, fragments)
+#define MOE_PLANES_PER(GV)                     \
+    if (steps <= 16) MOE_PLANES_CASE(16, GV);    \
+    else if (steps <= 32) MOE_PLANES_CASE(32, GV); \
+    else MOE_PLANES_CASE(64, GV);
+    if (tokens <= 8) {
+        MOE_PLANES_PER(1)
+    } else {
+        MOE_PLANES_PER(2)
+    }
+#undef MOE_PLANES_PER
+#undef MOE_PLANES_CASE
+    const int rc = check_launch("route_planes_kernel");
+    if (rc != MOE_OK) return rc;
+    hipLaunchKernelGGL(route_finish_kernel, dim3(1), dim3(kSmallThreads), 0, stream, sums, bias, ids32, ids64,
+                       weights, tokens, experts, topk, rows);
+    return check_launch("route_finish_kernel");
+}
+
 int launch_router_fused(const uint16_t* x, const float* router_w, const float* bias,
                         int32_t* ids32, int64_t* ids64, float* weights, float* logits_out,
                         uint16_t* planes, int64_t tokens, int hidden, int experts, int topk,
@@ -966,9 +1340,15 @@ int launch_router_fused(const uint16_t* x, const float* router_w, const float* b
     // Buffer offsets are 32-bit: 3*E*H*2 bytes of planes and 32 rows of x must fit.
     MOE_REQUIRE(hidden <= (1 << 20), MOE_ERR_UNSUPPORTED, "fused router supports hidden <= 1048576 (got %d)",
                 hidden);
+    if (small_route(tokens, hidden, experts)) {
+        const uint16_t* frags = reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(planes) +
+                                                                  router_fragments_offset(experts, hidden));
+        return launch_route_small(x, frags, bias, ids32, ids64, weights, logits_out, static_cast<int>(tokens), hidden,
+                                  experts, topk, ranks, tile_counts, RowsOut{}, stream);
+    }
     const int k_stages = (hidden + 63) / 64;
     constexpr int kSplitMaxPer = RouterShape<1, 1>::STAGES;  // a slice fits the ring at once
-    if (experts <= 16 && tokens <= kRouterSplitTokens && k_stages >= 16 &&
+    if (experts <= 16 && tokens <= kRouterSplitTokens && k_stages > kDirectWaves * kDirectMaxPer &&
         k_stages <= kRouterSplitSlices * kSplitMaxPer) {
         // Split k: slices of about 8 stages (64 KiB of loads per workgroup),
         // none empty.

@@ -49,6 +49,8 @@ _SIGNATURES = {
     ),
     "moe_dispatch_rows": (_int, [_c_void_p] * 7 + [_i64] * 6 + [_c_void_p]),
     "moe_dispatch_ranked_rows": (_int, [_c_void_p] * 8 + [_i64] * 7 + [_c_void_p]),
+    "moe_route_rows_scratch_bytes": (_i64, [_i64] * 4),
+    "moe_route_rows": (_int, [_c_void_p] * 7 + [_i64] + [_c_void_p] * 6 + [_i64] * 7 + [_c_void_p]),
     "moe_combine": (_int, [_c_void_p, _int, _c_void_p, _c_void_p, _c_void_p] + [_i64] * 4 + [_c_void_p]),
     "moe_swiglu": (_int, [_c_void_p, _int, _c_void_p, _c_void_p, _i64, _i64, _c_void_p]),
     "moe_grouped_gemm": (_int, [_c_void_p] * 4 + [_i64] * 4 + [_c_void_p]),

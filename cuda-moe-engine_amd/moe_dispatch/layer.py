@@ -92,7 +92,6 @@ def make_weights(config, device, dtype, seed=42):
 # not a power of two apart.
 GATE_UP_ROW_PADDING = 64
 
-
 def padded_gate_up(weight):
     """``weight`` ([E, 2I, H]) as a ``[:, :, :H]`` view of row-padded storage when
     its rows are a power of two bytes of at least 8 KiB long, else contiguous."""
@@ -322,7 +321,8 @@ class MoEBlock(torch.nn.Module):
         fused = self.implementation == "cuda_fused"
         # The fused router does the dispatch's counting pass when the shape allows.
         ranked = fused and state.transport.rank_tile > 0
-        gathered = fused and _gathers(x, self.config.topk)
+        gathered = fused and (_one_pass_bytes(self._extension.lib, x, self.config) is not None
+                              or _gathers(x, self.config.topk))
         ids32, ids64, weights = self._route(x, state.transport if ranked else None)
         transport = state.transport
         if gathered:
@@ -346,6 +346,11 @@ class MoEBlock(torch.nn.Module):
         return state.transport.output
 
 
+def _can_gather(x):
+    """Whether the gate/up GEMM can read its rows from x (hidden a multiple of 64, x below 2 GiB)."""
+    return x.shape[1] % 64 == 0 and x.numel() * x.element_size() < 2**31
+
+
 def _gathers(x, topk):
     """Whether the fused forward skips the packed copy, the gate/up GEMM reading
     x through the dispatch's row table. It needs the ring kernels (hidden a
@@ -357,7 +362,16 @@ def _gathers(x, topk):
     that configuration's Zipf routing the gathered GEMM is itself faster than
     the packed one (560 against 638 us): it reads x's 33.6 MB where the packed
     kernel reads a 201 MB copy."""
-    return topk >= 3 and x.shape[1] % 64 == 0 and x.numel() * x.element_size() < 2**31
+    return topk >= 3 and _can_gather(x)
+
+
+def _one_pass_bytes(lib, x, cfg):
+    """Plane-sum bytes of the small-batch route that also writes the row table
+    (``moe_route_rows``), or None where the shape has none. It replaces the router
+    and the dispatch whatever top-k is: H=4096, E=8, top-2: 12.6 -> 6.6 us at one
+    token, 13.8 -> 7.5 at 16; H=2048, E=64, top-6, 48 tokens: 33.6 -> 10.5 us."""
+    need = lib.moe_route_rows_scratch_bytes(x.shape[0], cfg.hidden, cfg.experts, cfg.topk)
+    return need if need >= 0 and _can_gather(x) else None
 
 
 class _FusedLaunches:
@@ -367,7 +381,7 @@ class _FusedLaunches:
     the two grouped GEMMs, combine) fixes every argument but x's address and
     the stream: workspace and weight pointers, sizes, the dtype code. Later
     forwards of the same token count on the same device make the same five
-    calls with those arguments while every parameter tensor the calls read is
+    calls (four where a small batch routes and dispatches in one pass) with those arguments while every parameter tensor the calls read is
     the object it was, at the same address, with the same dtype, shape and
     layout (an in-place update keeps all of these; the router split follows
     the weights' version as in ``MoEBlock.route``). Anything else sends the
@@ -394,15 +408,25 @@ class _FusedLaunches:
                        tokens, hidden, cfg.experts, cfg.topk)
         # A ranked route (the router counts for the dispatch) whenever the shape
         # has one, and the row table instead of the packed copy whenever the
-        # gate/up GEMM can gather, as in forward().
+        # gate/up GEMM gathers, as in forward().
         self.ranked = t.rank_tile > 0
-        self.gathered = _gathers(x, cfg.topk)
+        sums_bytes = _one_pass_bytes(self.lib, x, cfg)
+        self.gathered = sums_bytes is not None or _gathers(x, cfg.topk)
         # The weights' row strides (contiguous, or gate/up rows padded); anything
         # else was refused by the validating forward that built these launches.
         gate_up_stride = weight_row_stride(block.gate_up_weight)
         down_stride = weight_row_stride(block.down_weight)
         if gate_up_stride is None or down_stride is None:
             raise RuntimeError("expert weights must be contiguous or row-padded")
+        # Small batches: routing and the row-table dispatch in one pass (every
+        # output as the two calls write it), its plane sums owned by these launches.
+        self.route_rows = None
+        if sums_bytes is not None:
+            self.sums = torch.empty(max(sums_bytes, 4), dtype=torch.uint8, device=x.device)
+            self.route_rows = self.router[:4] + self.router[5:7] + (
+                t.counts.data_ptr(), t.offsets.data_ptr(), t.slots.data_ptr(), t.inverse.data_ptr(),
+                t.row_src.data_ptr(), self.sums.data_ptr(), self.sums.numel(), tokens, hidden, cfg.experts, cfg.topk,
+                t.alignment, rows)
         index = (ids32.data_ptr(), t.counts.data_ptr(), t.offsets.data_ptr(), t.slots.data_ptr())
         if self.ranked:
             self.router += (t.tile_ranks.data_ptr(), t.tile_counts.data_ptr(), t.tile_counts.numel() * 4)
@@ -456,16 +480,19 @@ class _FusedLaunches:
         stream = current_stream_handle(self.device_index)
         x_ptr = x.data_ptr()
         router_weight, split_of = block._router_split_plan()
-        if self.ranked:
+        if self.route_rows is not None:
+            lib.check(lib.moe_route_rows(x_ptr, router_weight, *self.route_rows, stream), "route_rows")
+        elif self.ranked:
             lib.check(lib.moe_router_fused_ranked(x_ptr, router_weight, *self.router, stream), "router_fused_out")
         else:
             lib.check(lib.moe_router_fused(x_ptr, router_weight, *self.router, stream), "router_fused_out")
         block._router_split_of = split_of
         if self.gathered:
-            if self.ranked:
-                lib.check(lib.moe_dispatch_ranked_rows(*self.dispatch, stream), "dispatch")
-            else:
-                lib.check(lib.moe_dispatch_rows(*self.dispatch, stream), "dispatch")
+            if self.route_rows is None:
+                if self.ranked:
+                    lib.check(lib.moe_dispatch_ranked_rows(*self.dispatch, stream), "dispatch")
+                else:
+                    lib.check(lib.moe_dispatch_rows(*self.dispatch, stream), "dispatch")
             lib.check(lib.moe_grouped_gateup_swiglu_gathered_strided(x_ptr, *self.gateup, stream),
                       "gateup_swiglu_out")
         else:
@@ -480,7 +507,8 @@ class _FusedLaunches:
 
     def stage_calls(self, x):
         """Each stage of __call__ as a zero-argument callable on the current
-        stream (the router with the split it holds), for per-stage timing."""
+        stream (the router with the split it holds), for per-stage timing. A
+        small batch's one-pass route is timed as its two stages' own calls."""
         lib, x_ptr = self.lib, x.data_ptr()
 
         def bind(name, *args):

@@ -76,7 +76,7 @@ int moe_topk_route(const float* logits, const float* bias, int32_t* ids32, int64
 
 /* Bytes of scratch moe_router_fused needs for (E, H): the bf16 split of
  * router_w, then 64 KiB of partial logits for the small-batch (T <= 64,
- * E <= 16) split-k path, then a copy of the split in the MFMA operand order
+ * E <= 16, 8192 < H <= 16384) split-k path, then a copy of the split in the MFMA operand order
  * the VGPR-load kernels read (ceil(H/64) * ceil(6E/16) KiB). */
 int64_t moe_router_scratch_bytes(int64_t experts, int64_t hidden);
 
@@ -223,6 +223,28 @@ int moe_dispatch_ranked_rows(const int32_t* ids, int32_t* counts, int32_t* offse
                              int32_t* inverse, int32_t* row_src, const int32_t* ranks, const int32_t* tile_counts,
                              int64_t tile_counts_bytes, int64_t tile_tokens, int64_t tokens, int64_t experts,
                              int64_t topk, int64_t alignment, int64_t packed_rows, void* stream);
+
+/* Bytes of plane sums moe_route_rows needs for this shape (0: none), or -1
+ * when it has no one-pass route (then moe_router_fused and a dispatch): it has
+ * one up to 16 tokens and 8192 hidden for E <= 16, and up to 128 tokens, 1024
+ * assignments and 4096 hidden above. */
+int64_t moe_route_rows_scratch_bytes(int64_t tokens, int64_t hidden, int64_t experts, int64_t topk);
+
+/*
+ * Small batches: moe_router_fused and moe_dispatch_rows in one pass, one launch
+ * for E <= 16 and two above. Every output equals the pair's bit for bit; x,
+ * router_w, bias, ids32, ids64, weights and scratch as moe_router_fused takes
+ * them (router_w == NULL carries its precondition), counts, offsets, slots,
+ * inverse and row_src as moe_dispatch_rows writes them. sums: at least
+ * moe_route_rows_scratch_bytes bytes, for this call alone (16-byte aligned; may
+ * be NULL when that is 0). MOE_ERR_UNSUPPORTED when that is -1. No counterpart in
+ * the reference.
+ */
+int moe_route_rows(const void* x, const float* router_w, const float* bias, int32_t* ids32, int64_t* ids64,
+                   float* weights, void* scratch, int64_t scratch_bytes, int32_t* counts, int32_t* offsets,
+                   int32_t* slots, int32_t* inverse, int32_t* row_src, void* sums, int64_t sums_bytes,
+                   int64_t tokens, int64_t hidden, int64_t experts, int64_t topk, int64_t alignment,
+                   int64_t packed_rows, void* stream);
 
 /*
  * Weighted combine: out[t] = round(sum_k w[t,k] * float(y[inverse[t,k]])),

@@ -241,3 +241,28 @@ def test_row_table_entry_points_check_their_arguments_without_launching():
     assert lib.moe_grouped_gateup_swiglu_gathered(A, A + 2, 16, A, A, A, 16, 64, 64, 1, None) == 1
     assert lib.moe_grouped_gateup_swiglu_gathered(A, None, 16, A, A, A, 16, 64, 64, 1, None) == 1
     assert lib.moe_grouped_gateup_swiglu_gathered(A, A, 16, A, A, A, 0, 64, 64, 1, None) == 0  # no rows
+
+
+@stand_in_addresses
+def test_route_rows_arguments_are_checked_before_launch():
+    """moe_route_rows refuses what its two stages refuse, shapes without a one-pass
+    route, and short, missing or misaligned plane sums (nothing is launched)."""
+    lib = _lib.load_library()
+    scratch = lib.moe_router_scratch_bytes(64, 512)
+    sums = lib.moe_route_rows_scratch_bytes(100, 512, 64, 6)
+    assert sums == 100 * 3 * 64 * 4 and lib.moe_route_rows_scratch_bytes(16, 512, 8, 2) == 0
+    assert lib.moe_route_rows_scratch_bytes(0, 512, 8, 2) == -1
+    rows = 100 * 6
+
+    def call(x=16, scratch_bytes=scratch, sums_ptr=16, sums_bytes=sums, tokens=100, experts=64, packed_rows=rows,
+             row_src=16):
+        return lib.moe_route_rows(x, 16, 16, 16, 16, 16, 16, scratch_bytes, 16, 16, 16, 16, row_src, sums_ptr,
+                                  sums_bytes, tokens, 512, experts, 6, 1, packed_rows, None)
+
+    ok, invalid, unsupported = 0, 1, 2
+    assert call(x=8) == invalid and call(x=None) == invalid and call(row_src=None) == invalid
+    assert call(scratch_bytes=scratch - 1) not in (ok, invalid, unsupported)
+    assert call(packed_rows=rows - 1) not in (ok, invalid, unsupported)
+    assert call(sums_bytes=sums - 1) not in (ok, invalid, unsupported)
+    assert call(sums_ptr=None) not in (ok, unsupported) and call(sums_ptr=24) == invalid
+    assert call(tokens=129, packed_rows=129 * 6) == unsupported and call(tokens=17, experts=16) == unsupported
