@@ -78,19 +78,28 @@ def make_weights(config, device, dtype, seed=42):
     return MoEWeights(router, gate_up, down)
 
 
-# Elements of padding after each gate/up weight row whose length is a power
-# of two bytes of at least 8 KiB (H = 4096, 8192, ...), for the fused block.
-# The weight-streaming GEMMs read every row of a tile at the same k offset at
-# once, and rows a power of two apart then fall on the same memory channels.
-# Measured at H = 4096, I = 14336, 8 experts, top-2, alternating on one box:
-# padded rows make the gate/up GEMM 11% faster at 1 token and 10% at 16
-# (91.8 -> 82.1 and 337.8 -> 304.7 us; forwards 165 -> 154.5 and 527 -> 495
-# us) and leave it unchanged at 4096 tokens. At H = 2048 (4 KiB rows; 8192
-# tokens, 64 experts, top-6) the gathered gate/up GEMM ran 1% slower with
-# padded rows, so those are not padded. The results are the same bit for bit
-# (each output is the same MFMA chain). The down GEMM's rows (I = 14336) are
-# not a power of two apart.
+# Elements of padding after each expert weight row whose length is a multiple of
+# WEIGHT_ROW_CONFLICT bytes, for the fused block. The GEMMs read every row of a
+# tile, on every CU, at the same k offset at once, and rows a multiple of 4 KiB
+# apart then fall on the same memory channels. Measured, padded against
+# contiguous rows: gate/up at H=2048, I=4096, 16 experts, 128 rows 121.6 -> 93.0
+# us (4.4 -> 5.8 TB/s) and at H=2048, I=1408, 64 experts, 288 rows 139.2 -> 125.2;
+# at H=4096, I=14336, 8 experts, 2 rows 90.0 -> 80.3 and 32 rows 338 -> 302; down
+# at I=14336 (7 x 4 KiB) with 32 rows 182 -> 158 and 666 rows 217 -> 206. Full
+# prefill is unchanged (4096 tokens at H=4096: 1447 and 1441 us). Rows of 2 KiB
+# multiples gained 1-8% at H=1024 with few rows and nothing with many, and stay
+# contiguous; so do rows of other lengths. The results are the same bit for bit
+# (each output is the same MFMA chain).
 GATE_UP_ROW_PADDING = 64
+WEIGHT_ROW_CONFLICT = 4096
+
+
+def _row_padded(weight):
+    e, n, k = weight.shape
+    storage = torch.zeros(e, n, k + GATE_UP_ROW_PADDING, device=weight.device, dtype=weight.dtype)
+    storage[:, :, :k].copy_(weight)
+    return storage[:, :, :k]
+
 
 def padded_gate_up(weight):
     """``weight`` ([E, 2I, H]) as a ``[:, :, :H]`` view of row-padded storage when
@@ -98,10 +107,18 @@ def padded_gate_up(weight):
     row_bytes = weight.shape[2] * weight.element_size()
     if row_bytes < 8192 or row_bytes & (row_bytes - 1):
         return weight.contiguous()
-    e, n, k = weight.shape
-    storage = torch.zeros(e, n, k + GATE_UP_ROW_PADDING, device=weight.device, dtype=weight.dtype)
-    storage[:, :, :k].copy_(weight)
-    return storage[:, :, :k]
+    return _row_padded(weight)
+
+
+def padded_weight(weight):
+    """``weight`` ([E, N, K]) as a ``[:, :, :K]`` view of row-padded storage when its
+    rows are a multiple of WEIGHT_ROW_CONFLICT bytes and one expert stays below the
+    GEMMs' 4 GiB with the padding, else contiguous."""
+    _, n, k = weight.shape
+    size = weight.element_size()
+    if k * size % WEIGHT_ROW_CONFLICT or n * (k + GATE_UP_ROW_PADDING) * size >= 2**32:
+        return weight.contiguous()
+    return _row_padded(weight)
 
 
 @dataclass
@@ -152,11 +169,11 @@ class MoEBlock(torch.nn.Module):
         if weights.router.shape != (cfg.experts, cfg.hidden):
             raise ValueError("router weights do not match the block configuration")
         self.register_buffer("router_weight", weights.router.contiguous())
-        # The fused block keeps power-of-two gate/up rows padded (GATE_UP_ROW_PADDING);
-        # the tensor is a view of that storage, so in-place updates reach the kernels.
-        gate_up = padded_gate_up(weights.gate_up) if implementation == "cuda_fused" else weights.gate_up.contiguous()
-        self.register_buffer("gate_up_weight", gate_up)
-        self.register_buffer("down_weight", weights.down.contiguous())
+        # The fused block keeps conflicting weight rows padded (WEIGHT_ROW_CONFLICT); its
+        # tensors are views of that storage, so in-place updates of them reach the kernels.
+        laid_out = padded_weight if implementation == "cuda_fused" else torch.Tensor.contiguous
+        self.register_buffer("gate_up_weight", laid_out(weights.gate_up))
+        self.register_buffer("down_weight", laid_out(weights.down))
         self.register_buffer("routing_bias", torch.zeros(cfg.experts, device=device))
         self._workspaces = {}
         self._route_buffers = {}

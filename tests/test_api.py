@@ -105,3 +105,16 @@ def test_fused_block_pads_power_of_two_gate_up_rows():
         assert p.stride(1) == (hidden + GATE_UP_ROW_PADDING if padded else hidden), hidden
     # fp32 rows of 2048 elements are 8 KiB: padded too.
     assert padded_gate_up(torch.zeros(1, 2, 2048)).stride(1) == 2048 + GATE_UP_ROW_PADDING
+
+
+def test_fused_block_pads_weight_rows_that_conflict():
+    from moe_dispatch._extension import weight_row_stride
+    from moe_dispatch.layer import GATE_UP_ROW_PADDING, padded_weight
+
+    for k, padded in ((2048, True), (4096, True), (6144, True), (14336, True), (1024, False), (1408, False),
+                      (2056, False), (8, False)):
+        w = torch.randn(2, 3, k).bfloat16()
+        p = padded_weight(w)
+        assert torch.equal(p, w)
+        assert weight_row_stride(p) == (k + GATE_UP_ROW_PADDING if padded else k), k
+    assert weight_row_stride(padded_weight(torch.zeros(1, 1, 2048).bfloat16())) % 8 == 0  # one row, one expert

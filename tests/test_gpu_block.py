@@ -306,6 +306,26 @@ def test_padded_gate_up_rows_equal_contiguous_weights(cfg):
     assert torch.equal(block(x).clone(), twin(x))
 
 
+@pytest.mark.parametrize("cfg", [MoEConfig(2048, 256, 8, 2), MoEConfig(128, 4096, 8, 2), MoEConfig(2048, 2048, 16, 6)])
+def test_padded_weight_rows_equal_contiguous_weights(cfg):
+    """Gate/up or down rows of a multiple of 4 KiB are kept padded: the forward equals that
+    of a twin with contiguous copies, bit for bit, and in-place updates reach the kernels."""
+    block = MoEBlock(cfg, device="cuda", implementation="cuda_fused", seed=3)
+    twin = MoEBlock(cfg, device="cuda", implementation="cuda_fused", seed=3)
+    for name, k in (("gate_up_weight", cfg.hidden), ("down_weight", cfg.intermediate)):
+        assert getattr(block, name).stride(1) == (k + GATE_UP_ROW_PADDING if k % 2048 == 0 else k)
+        setattr(twin, name, getattr(block, name).contiguous())
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    for tokens in (1, 20, 700):
+        x = torch.randn(tokens, cfg.hidden, device="cuda", generator=gen).bfloat16()
+        assert torch.equal(block(x).clone(), twin(x)), tokens
+    new = (torch.randn(block.down_weight.shape, device="cuda", generator=gen) / 45).bfloat16()
+    block.down_weight.copy_(new)
+    twin.down_weight.copy_(new)
+    x = torch.randn(300, cfg.hidden, device="cuda", generator=gen).bfloat16()
+    assert torch.equal(block(x).clone(), twin(x))
+
+
 def test_empty_batch():
     block = MoEBlock(MoEConfig(64, 128, 8, 2), device="cuda", implementation="cuda_fused")
     out = block(torch.empty(0, 64, device="cuda", dtype=torch.bfloat16))
