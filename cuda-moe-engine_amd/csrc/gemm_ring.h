@@ -1104,9 +1104,8 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_persistent_kernel(G
 // tile) and issue the next tile's first stages before the current tile's
 // epilogue. Tiles are narrow so that a single token's two
 // experts still spread over the CUs: 64 activation columns (128 weight rows,
-// waves 2 x 2) for the gate/up GEMM, 64 output columns for the down GEMM, and
-// 32 (waves 4 x 1) when at most 64 rows are packed (at T=16 the 4 x 1 waves,
-// which all read every B fragment, ran 7% slower than 64 columns). Their
+// waves 2 x 2) for the gate/up GEMM; for the plain GEMM 64 output columns, 32
+// (waves 4 x 1) when at most 64 rows are packed, or wider (narrow_shift). Their
 // stages are small (12-32 KiB), so the ring holds up to eight: a CU has to
 // keep about 32 KiB of loads in flight to stream at the HBM rate (a plain
 // read kernel reaches 6.3-6.4 TB/s with 32 KiB per CU, 5.2 TB/s with 16 KiB).
@@ -1118,7 +1117,34 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_persistent_kernel(G
 // 64 rows runs the 64-row instance. At C1 (T=128, E=8: about 32 rows per
 // expert) the wide tiles kept 64 (gate/up) and 16 (down) CUs busy.
 template <bool SWIGLU, int MAX_ROWS>
-constexpr int narrow_cols() { return SWIGLU || MAX_ROWS == 128 ? 64 : 32; }
+constexpr int narrow_cols() { return SWIGLU || MAX_ROWS == 128 ? 64 : 32; }  // the narrowest
+
+// Plain GEMM: log2 of the launch's column width, doubled from the narrowest up to 128
+// while a CU's most loaded share of rounds, each of A rows + columns per k,
+// falls below 0.7 of the narrower one's, or falls at all where the narrower
+// tiles leave a fifth of their slots empty. `groups`: row tiles over all experts.
+// Wider tiles read A less often (128-row tiles of 64 columns read twice as much
+// A as weights); at the HBM rate that gains nothing, and narrow tiles balance
+// better. K=14336, N=4096, 8 experts: 666 rows 204 -> 174 us and 512 rows 191 ->
+// 172 (128 columns), 4 rows 87 -> 82 (64, from 32), 8 rows 126 -> 109 (128); 32 to
+// 128 rows stay at 64 (157-167 us, 5.6-6.0 TB/s, within 4% of 128).
+__device__ __forceinline__ int narrow_shift(int shift, int groups, int n_out, int a_rows, int grid) {
+    auto tiles_of = [&](int s) { return groups * ((n_out + (1 << s) - 1) >> s); };
+    int tiles = tiles_of(shift);
+    int rounds = static_cast<int>((static_cast<uint32_t>(tiles) + grid - 1) / static_cast<uint32_t>(grid));
+    for (; shift < 7; ++shift) {
+        const int wide_tiles = tiles_of(shift + 1);
+        const int wide_rounds =
+            static_cast<int>((static_cast<uint32_t>(wide_tiles) + grid - 1) / static_cast<uint32_t>(grid));
+        const int64_t now = static_cast<int64_t>(rounds) * (a_rows + (1 << shift));
+        const int64_t wide = static_cast<int64_t>(wide_rounds) * (a_rows + (2 << shift));
+        const bool empty = 10 * static_cast<int64_t>(tiles) < 8 * static_cast<int64_t>(rounds) * grid;
+        if (!(10 * wide <= 7 * now || (empty && wide < now))) break;
+        tiles = wide_tiles;
+        rounds = wide_rounds;
+    }
+    return shift;
+}
 
 constexpr int kDecodeStages = 8;
 
@@ -1129,9 +1155,6 @@ constexpr uint32_t decode_lds_bytes() {
 
 template <bool SWIGLU, int MAX_ROWS, bool GATHER, bool TAIL>
 __global__ __launch_bounds__(kRingThreads) void grouped_gemm_decode_kernel(GemmParams p) {
-    constexpr int COLS = narrow_cols<SWIGLU, MAX_ROWS>();
-    constexpr int BNT = SWIGLU ? 2 * COLS : COLS;
-    constexpr int WC = BNT == 32 ? 1 : 2;
     constexpr uint32_t kLds = decode_lds_bytes<SWIGLU, MAX_ROWS>();
     static_assert(MAX_ROWS == 64 || MAX_ROWS == 128, "decode row tiles");
     __shared__ __attribute__((aligned(1024))) char lds[kLds];
@@ -1142,10 +1165,19 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_decode_kernel(GemmP
     int off = 0, span = 0;
     if (lane < p.experts) expert_rows(p, lane, off, span);
     const int m_tiles = (span + MAX_ROWS - 1) / MAX_ROWS;
-    const int count = m_tiles * p.n_tiles;
-    const int incl = wave_inclusive_sum(count);
-    const int first = incl - count;
-    const int tiles = __builtin_amdgcn_readlane(incl, kWave - 1);
+    const int incl = wave_inclusive_sum(m_tiles);
+    const int groups = __builtin_amdgcn_readlane(incl, kWave - 1);
+    int shift = narrow_cols<SWIGLU, MAX_ROWS>() == 32 ? 5 : 6;
+    if constexpr (!SWIGLU) {
+        const int a_rows = MAX_ROWS == 128 && __ballot(span > 64) != 0 ? 128 : 64;
+        shift = __builtin_amdgcn_readfirstlane(
+            narrow_shift(shift, groups, static_cast<int>(p.n_out), a_rows, static_cast<int>(gridDim.x)));
+    }
+    const int cols = 1 << shift;
+    const int n_tiles = static_cast<int>((p.n_out + cols - 1) >> shift);
+    const int count = m_tiles * n_tiles;
+    const int first = (incl - m_tiles) * n_tiles;
+    const int tiles = groups * n_tiles;
     const int k_steps = static_cast<int>((p.k + kStageK - 1) / kStageK);
     struct Work {
         bool valid;
@@ -1166,7 +1198,7 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_decode_kernel(GemmP
         if (w.row0 < 0 || w.row0 >= w.row_end) return w;
         w.tall = MAX_ROWS == 128 && w.row_end - w.row0 > 64;
         w.expert = e;
-        w.col0 = n_tile * COLS;
+        w.col0 = n_tile * cols;
         w.valid = true;
         return w;
     };
@@ -1178,27 +1210,40 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_decode_kernel(GemmP
             for (int i = 0; i < decltype(ops)::A_LOADS; ++i) a_carry[i] = ops.a_off[i];
         }
     };
-    auto prologue = [&](const Work& w) {
-        if constexpr (MAX_ROWS == 128) {
-            if (w.tall) {
-                issue(RingOps<128, BNT, SWIGLU, kLds, WC, kDecodeStages, GATHER, TAIL>(p, lds, w.expert, w.col0, w.row0,
-                                                                                 w.row_end));
-                return;
+    // f(Shape<rows, weight rows>) for a tile of this launch's width.
+    auto with_shape = [&](const Work& w, auto&& f) {
+        auto rows = [&](auto bnt_c) {
+            if constexpr (MAX_ROWS == 128) {
+                if (w.tall) return f(std::integral_constant<int, 128>{}, bnt_c);
             }
+            f(std::integral_constant<int, 64>{}, bnt_c);
+        };
+        if constexpr (SWIGLU) {
+            rows(std::integral_constant<int, 2 * narrow_cols<true, MAX_ROWS>()>{});
+        } else {
+            if constexpr (MAX_ROWS == 64) {
+                if (cols == 32) return rows(std::integral_constant<int, 32>{});
+            }
+            if (cols == 64)
+                rows(std::integral_constant<int, 64>{});
+            else
+                rows(std::integral_constant<int, 128>{});
         }
-        issue(RingOps<64, BNT, SWIGLU, kLds, WC, kDecodeStages, GATHER, TAIL>(p, lds, w.expert, w.col0, w.row0, w.row_end));
+    };
+    auto prologue = [&](const Work& w) {
+        with_shape(w, [&](auto rows_c, auto bnt_c) {
+            constexpr int BNT = decltype(bnt_c)::value;
+            issue(RingOps<decltype(rows_c)::value, BNT, SWIGLU, kLds, BNT == 32 ? 1 : 2, kDecodeStages, GATHER, TAIL>(
+                p, lds, w.expert, w.col0, w.row0, w.row_end));
+        });
     };
     auto run = [&](const Work& w, bool wait_all, const auto& hook) {
-        using Hook = std::decay_t<decltype(hook)>;
-        if constexpr (MAX_ROWS == 128) {
-            if (w.tall) {
-                ring_tile<128, BNT, SWIGLU, kLds, Hook, WC, kDecodeStages, GATHER, TAIL>(
-                    p, lds, w.expert, w.col0, w.row0, w.row_end, false, wait_all, hook, 0, 0, false, {}, a_carry);
-                return;
-            }
-        }
-        ring_tile<64, BNT, SWIGLU, kLds, Hook, WC, kDecodeStages, GATHER, TAIL>(
-            p, lds, w.expert, w.col0, w.row0, w.row_end, false, wait_all, hook, 0, 0, false, {}, a_carry);
+        with_shape(w, [&](auto rows_c, auto bnt_c) {
+            constexpr int BNT = decltype(bnt_c)::value;
+            ring_tile<decltype(rows_c)::value, BNT, SWIGLU, kLds, std::decay_t<decltype(hook)>, BNT == 32 ? 1 : 2,
+                      kDecodeStages, GATHER, TAIL>(p, lds, w.expert, w.col0, w.row0, w.row_end, false, wait_all, hook,
+                                                   0, 0, false, {}, a_carry);
+        });
     };
     int t = blockIdx.x;
     Work cur = locate(t);

@@ -335,6 +335,28 @@ def test_partial_last_stage_equals_zero_padded(ext, counts, alignment, n, k):
         assert torch.equal(got[keep], want[keep])
 
 
+@pytest.mark.parametrize("counts,n", [
+    ([2, 2], 4096),            # 32 columns (256 CUs: one tile each)
+    ([1, 3, 2, 2], 8192),      # 64 columns
+    ([1, 0, 3, 2, 1], 8200),   # 64 columns, a last tile of 8
+    ([100] * 8, 4104),         # 128 columns, 128-row tiles
+    ([20, 1, 0, 5, 60], 4096), # 128 columns, 64-row tiles
+    ([100, 10] * 4, 1000),     # 64 columns, tall and short tiles
+])
+def test_weight_streaming_widths(ext, counts, n):
+    """The plain weight-streaming GEMM at each column width, against the oracle."""
+    k = 192
+    a, offsets, rows = _inputs(counts, 1, k, seed=n)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    b = (torch.randn(len(counts), n, k, device="cuda", generator=g) / k**0.5).bfloat16()
+    c = torch.full((rows, n), 7.0, device="cuda").bfloat16()
+    ext.grouped_gemm_out(a, b, offsets, c)
+    used = int(to_np(offsets)[-1])
+    mfma = oracle.grouped_gemm(to_np(a), to_np(b), to_np(offsets), order="mfma")
+    assert_near_bit_exact(to_np(c)[:used], oracle.bf16_round(mfma)[:used])
+    assert np.all(to_np(c)[used:] == 7.0)
+
+
 def test_weights_of_other_layouts_are_refused(ext):
     a, offsets, rows = _inputs([10, 20], 8, 64, seed=1)
     out = torch.empty(rows, 64, device="cuda", dtype=torch.bfloat16)
