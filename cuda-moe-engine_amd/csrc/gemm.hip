@@ -63,6 +63,7 @@ static int launch_gemm_t(GemmParams p, int64_t rows, hipStream_t stream) {
                                         wide_tiles < device_cu_count());
     if (narrow) {
         const int max_rows = rows <= 64 ? 64 : 128;
+        // The narrowest tiles; the kernel may take wider ones (fewer).
         const int cols = max_rows == 64 ? narrow_cols<SWIGLU, 64>() : narrow_cols<SWIGLU, 128>();
         p.n_tiles = static_cast<int>((p.n_out + cols - 1) / cols);
         // Upper bound on row tiles: sum_e ceil(span_e/max_rows) <= ceil(R/max_rows) + E.
@@ -85,15 +86,31 @@ static int launch_gemm_t(GemmParams p, int64_t rows, hipStream_t stream) {
     int64_t grid = device_cu_count();
     const int limit = g_gemm_workgroup_limit.load(std::memory_order_relaxed);
     if (limit > 0 && limit < grid) grid = limit;
-    // At most one workgroup per unit of work: tiles, or for the plain GEMM
-    // the halves and quarters the plan may split them into.
-    const int64_t units = SWIGLU ? blocks : 4 * blocks;
+    // Gate/up tiles split into pieces only where the estimated tiles (rows spread
+    // evenly) leave a last round at most half full in the first four, or where so
+    // few rows per expert leave it open how many experts hold any. The instance
+    // that splits is 390 KB of code instead of 220, and a launch that fetches it
+    // cold takes 2-3 us longer: forwards at H=1024, I=2048, 16 experts, 8192 rows
+    // 153 -> 156 us with it, at H=2048, I=1408, 64 experts, 288 rows 219.7 ->
+    // 221.4; against 603 -> 550 (with the down GEMM's widths) at H=4096, I=14336, 8
+    // experts, 666 rows, whose 896 tiles fill three and a half rounds.
+    bool pieces = !SWIGLU;
+    if constexpr (SWIGLU) {
+        const int64_t cus = device_cu_count(), last = wide_tiles % cus;
+        pieces = per_expert < 12 || (last > 0 && 2 * last <= cus && wide_tiles < 4 * cus);
+    }
+    // At most one workgroup per unit of work: tiles, or the halves and quarters
+    // the plan may split them into.
+    const int64_t units = pieces ? 4 * blocks : blocks;
     if (units < grid) grid = units;
     grid = grid / kNumXcd * kNumXcd;
     if (grid < kNumXcd) grid = kNumXcd;
     with_source<SWIGLU>(p, [&](auto gather_c, auto tail_c) {
-        launch_ring<SWIGLU, decltype(gather_c)::value, decltype(tail_c)::value>(p, RingKernel::kPersistent,
-                                                                                 static_cast<unsigned>(grid), stream);
+        constexpr bool G = decltype(gather_c)::value, T = decltype(tail_c)::value;
+        if constexpr (SWIGLU) {
+            if (pieces) return launch_pieces<G, T>(p, static_cast<unsigned>(grid), stream);
+        }
+        launch_ring<SWIGLU, G, T>(p, RingKernel::kPersistent, static_cast<unsigned>(grid), stream);
     });
     return check_launch("grouped_gemm_persistent_kernel");
 }

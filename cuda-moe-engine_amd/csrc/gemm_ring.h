@@ -668,32 +668,42 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, char* lds, int ex
 // by column tile, row tiles fastest. Measured at H=4096, I=14336, 4096 tokens:
 // the short tiles took 250 us after the 1418 us of phase 1 when run last.
 //
-// For the plain GEMM a short last round (at most half of the slots busy) of
-// phase 1 (when there is no phase 2) or of the leftover phase-2 tiles is split
-// into 128-column pieces, and leftover phase-2 tiles into 64-column quarters
-// when at most a quarter of the slots would be busy. When phase 1 fills at
-// most half of the slots of one round beside a phase 2, its tiles run as
-// 128-column halves (the two halves of a tile in neighbouring slots of one
-// XCD, sharing the A slab in L2): at H=1024, I=2048, E=16, 4096 tokens the
-// down GEMM's 128 full tiles otherwise took one whole K=2048 chain on half of
-// the CUs. Every tile or piece runs its whole k chain in order on one
+// A short last round (at most half of the slots busy) of phase 1 (when there is
+// no phase 2) or of the leftover phase-2 tiles is split into column halves, and
+// leftover phase-2 tiles into quarters when at most a quarter of the slots would
+// be busy (halves and quarters of a tile's output columns: 128 and 64 for the
+// plain GEMM, 64 and 32 for gate/up). Gate/up tiles were not split before: H=4096,
+// I=14336, 8 experts, 666 rows (896 tiles, three and a half rounds) 342 -> 328
+// us, 2048 rows 559 -> 541; H=2048, I=1408, 64 experts, 6 rows 21-25 -> 15-17, 96
+// rows 115 -> 104; H=512, I=1024, 8192 rows 28 -> 25. Halves of its short tiles
+// after rounds of full ones lose, though (H=1024, I=2048, 16 experts, 8192 rows: in
+// the forward 82 -> 85 us; they are HBM-bound whole, and a half reads A again).
+//
+// For the plain GEMM, when phase 1 fills at most half of the slots of one round
+// beside a phase 2, its tiles run as halves (the two halves of a tile in
+// neighbouring slots of one XCD, sharing the A slab in L2): at H=1024, I=2048,
+// E=16, 4096 tokens the down GEMM's 128 full tiles otherwise took one whole
+// K=2048 chain on half of the CUs. (Gate/up with the same choice at run time kept
+// more of the plan live through the k-loop and spilled: H=4096, I=14336, 4096
+// tokens 1460 -> 1587 us.) Every tile or piece runs its whole k chain in order on one
 // workgroup, so results do not depend on the schedule or on G.
 struct RingPhase {
     int count;   // tiles
     int main;    // tiles mapped XCD-contiguously
     int blocks;  // virtual workgroups of the main part (multiple of 8)
     int pieces;  // split tail pieces (`ways` per split tile)
-    int ways;    // 2 (128-column pieces) or 4 (64-column pieces of short tiles)
+    int ways;    // 2 (column halves) or 4 (column quarters of short tiles)
 };
 
 // Short tiles (phase 2) split four ways when that still fits the slots: their
 // cost is streaming the weight slab, which more CUs pull faster.
-__device__ __forceinline__ RingPhase ring_phase(int count, int grid, bool allow_split, bool short_tiles) {
+__device__ __forceinline__ RingPhase ring_phase(int count, int grid, bool pieces, bool short_tiles, bool halves) {
     RingPhase ph;
     ph.count = count;
     const int rem = count % grid;
-    const bool split = allow_split && rem > 0 && 2 * rem <= grid;
-    ph.ways = short_tiles && 4 * rem <= grid ? 4 : 2;
+    const bool quarters = short_tiles && 4 * rem <= grid;
+    const bool split = pieces && rem > 0 && (quarters || (halves && 2 * rem <= grid));
+    ph.ways = quarters ? 4 : 2;
     ph.main = split ? count - rem : count;
     ph.blocks = (ph.main + kNumXcd - 1) / kNumXcd * kNumXcd;
     ph.pieces = split ? ph.ways * rem : 0;
@@ -703,7 +713,7 @@ __device__ __forceinline__ RingPhase ring_phase(int count, int grid, bool allow_
 struct RingPlan {
     int n1;           // phase-1 tiles
     int n2;           // phase-2 tiles
-    bool half1;       // phase 1 runs as 128-column halves in the rounds
+    bool half1;       // phase 1 runs as column halves in the rounds
     int u1;           // phase-1 units of the rounds (tiles, or halves)
     int per1;         // phase-1 tiles per XCD range
     int cpr;          // phase-1 tiles per XCD and round
@@ -717,11 +727,11 @@ struct RingPlan {
 };
 
 // grid is a positive multiple of 8.
-__device__ __forceinline__ RingPlan ring_plan(int n1, int n2, int grid, bool allow_split) {
+__device__ __forceinline__ RingPlan ring_plan(int n1, int n2, int grid, bool swiglu, bool pieces) {
     RingPlan pl{};
     pl.n1 = n1;
     pl.n2 = n2;
-    pl.half1 = allow_split && n2 > 0 && n1 > 0 && 2 * n1 <= grid;
+    pl.half1 = !swiglu && n2 > 0 && n1 > 0 && 2 * n1 <= grid;
     pl.u1 = pl.half1 ? 2 * n1 : n1;
     if (n2 > 0 && n1 > 0) {
         pl.per1 = (pl.u1 + kNumXcd - 1) / kNumXcd;
@@ -734,7 +744,7 @@ __device__ __forceinline__ RingPlan ring_plan(int n1, int n2, int grid, bool all
         pl.slots = rounds * grid - kNumXcd * pl.per1;
         pl.carried = min(n2, 2 * pl.slots);
     }
-    pl.rest = ring_phase(n2 > 0 ? n2 - pl.carried : n1, grid, allow_split, n2 > 0);
+    pl.rest = ring_phase(n2 > 0 ? n2 - pl.carried : n1, grid, pieces, n2 > 0, !swiglu || n1 == 0 || n2 == 0);
     pl.virtual_blocks = pl.rounds * grid + pl.rest.blocks + pl.rest.pieces;
     return pl;
 }
@@ -742,7 +752,7 @@ __device__ __forceinline__ RingPlan ring_plan(int n1, int n2, int grid, bool all
 struct RingSlot {
     int phase;  // 0 / 1 for phase 1 / 2; -1: no tile
     int tile;   // index inside the phase of the first tile
-    int piece;  // -1; 0 / 1 for the two 128-column halves; 4 + q for 64-column quarter q
+    int piece;  // -1; 0 / 1 for the two column halves; 4 + q for quarter q
     int count;  // tiles tile, tile + 1, ... of this slot (0 to 2)
 };
 
@@ -799,7 +809,7 @@ __device__ __forceinline__ RingSlot ring_slot(const RingPlan& pl, int grid, int 
 struct RingWork {
     bool valid;
     int expert;
-    int variant;  // row tile 256 / 128 / 64 = 0 / 1 / 2; +3 for a 128-column piece, +6 for a 64-column one;
+    int variant;  // row tile 256 / 128 / 64 = 0 / 1 / 2; +3 for a half, +6 for a quarter (of 128 or 64 rows);
                   // whole 256-column tiles of 32 / 224 / 192 / 160 rows = 9 / 10 / 11 / 12
     int64_t row0, row_end, col0;
 };
@@ -908,16 +918,14 @@ __device__ __forceinline__ RingWork ring_locate(const GemmParams& p, const RingT
                     : h > 64  ? 1
                     : h > 32  ? 2
                               : 9;
-    if constexpr (SWIGLU) {
-        w.col0 = static_cast<int64_t>(n_tile) * 128;
-    } else if (s.piece < 0) {
-        w.col0 = static_cast<int64_t>(n_tile) * 256;
-    } else if (s.piece < 4) {
-        w.col0 = static_cast<int64_t>(n_tile) * 256 + s.piece * 128;
-        w.variant += 3;
-    } else {
-        w.col0 = static_cast<int64_t>(n_tile) * 256 + (s.piece - 4) * 64;
+    constexpr int kTileCols = SWIGLU ? 128 : 256;  // output columns; a piece covers a half or a quarter
+    w.col0 = static_cast<int64_t>(n_tile) * kTileCols;
+    if (s.piece >= 4) {
+        w.col0 += (s.piece - 4) * (kTileCols / 4);
         w.variant += 6;
+    } else if (s.piece >= 0) {
+        w.col0 += s.piece * (kTileCols / 2);
+        w.variant += 3;
     }
     // A piece of the last column tile can start at or past the last output
     // column (N < 256, or a last tile of at most 192 columns): it has no
@@ -936,7 +944,7 @@ struct RingShape {
 };
 
 // Issues tile w's prologue; with GATHER also leaves its A offsets in a_carry.
-template <bool SWIGLU, bool GATHER, bool TAIL>
+template <bool SWIGLU, bool GATHER, bool TAIL, bool PIECES>
 __device__ __forceinline__ void ring_prologue(const GemmParams& p, char* lds, const RingWork& w, uint32_t* a_carry) {
     const int k_steps = static_cast<int>((p.k + kStageK - 1) / kStageK);
     auto go = [&](auto shape) {
@@ -957,11 +965,10 @@ __device__ __forceinline__ void ring_prologue(const GemmParams& p, char* lds, co
         case 11: go(RingShape<192, 256>{}); break;
         case 12: go(RingShape<160, 256>{}); break;
         default:
-            if constexpr (!SWIGLU) {
+            if constexpr (PIECES) {
                 if (w.variant == 3) go(RingShape<256, 128>{});
                 else if (w.variant == 4) go(RingShape<128, 128>{});
                 else if (w.variant == 5) go(RingShape<64, 128>{});
-                else if (w.variant == 6) go(RingShape<256, 64>{});
                 else if (w.variant == 7) go(RingShape<128, 64>{});
                 else go(RingShape<64, 64>{});
             }
@@ -973,7 +980,7 @@ __device__ __forceinline__ void ring_prologue(const GemmParams& p, char* lds, co
 // enough, the two are chained (see ring_tile): `w`'s last windows load `nxt`'s
 // first stages and its hook issues only the prologue's last window. Otherwise
 // the hook issues `nxt`'s whole prologue at slots 0.
-template <int TMR, int BNT, bool SWIGLU, bool GATHER, bool TAIL>
+template <int TMR, int BNT, bool SWIGLU, bool GATHER, bool TAIL, bool PIECES>
 __device__ __forceinline__ void ring_run_shape(const GemmParams& p, char* lds, const RingWork& w,
                                                const RingWork& nxt, bool wait_all, int& sa, int& sb,
                                                uint32_t* a_carry) {
@@ -1006,7 +1013,7 @@ __device__ __forceinline__ void ring_run_shape(const GemmParams& p, char* lds, c
                 R(p, lds, nxt.expert, nxt.col0, nxt.row0, nxt.row_end).prologue(k_steps, na, nb, true);
             }
         } else {
-            ring_prologue<SWIGLU, GATHER, TAIL>(p, lds, nxt, a_carry);
+            ring_prologue<SWIGLU, GATHER, TAIL, PIECES>(p, lds, nxt, a_carry);
         }
     };
     ring_tile<TMR, BNT, SWIGLU, kRingBytes, decltype(hook), 2, 4, GATHER, TAIL>(
@@ -1015,30 +1022,29 @@ __device__ __forceinline__ void ring_run_shape(const GemmParams& p, char* lds, c
     sb = chain ? nb : 0;
 }
 
-template <bool SWIGLU, bool GATHER, bool TAIL>
+template <bool SWIGLU, bool GATHER, bool TAIL, bool PIECES>
 __device__ __forceinline__ void ring_run(const GemmParams& p, char* lds, const RingWork& w, const RingWork& nxt,
                                          bool wait_all, int& sa, int& sb, uint32_t* a_carry) {
     switch (w.variant) {
-        case 0: ring_run_shape<256, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 1: ring_run_shape<128, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 2: ring_run_shape<64, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 9: ring_run_shape<32, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 10: ring_run_shape<224, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 11: ring_run_shape<192, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
-        case 12: ring_run_shape<160, 256, SWIGLU, GATHER, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 0: ring_run_shape<256, 256, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 1: ring_run_shape<128, 256, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 2: ring_run_shape<64, 256, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 9: ring_run_shape<32, 256, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 10: ring_run_shape<224, 256, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 11: ring_run_shape<192, 256, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
+        case 12: ring_run_shape<160, 256, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry); break;
         default:
-            if constexpr (!SWIGLU) {
-                if (w.variant == 3) ring_run_shape<256, 128, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
-                else if (w.variant == 4) ring_run_shape<128, 128, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
-                else if (w.variant == 5) ring_run_shape<64, 128, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
-                else if (w.variant == 6) ring_run_shape<256, 64, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
-                else if (w.variant == 7) ring_run_shape<128, 64, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
-                else ring_run_shape<64, 64, false, false, TAIL>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
+            if constexpr (PIECES) {
+                if (w.variant == 3) ring_run_shape<256, 128, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
+                else if (w.variant == 4) ring_run_shape<128, 128, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
+                else if (w.variant == 5) ring_run_shape<64, 128, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
+                else if (w.variant == 7) ring_run_shape<128, 64, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
+                else ring_run_shape<64, 64, SWIGLU, GATHER, TAIL, PIECES>(p, lds, w, nxt, wait_all, sa, sb, a_carry);
             }
     }
 }
 
-template <bool SWIGLU, bool GATHER, bool TAIL>
+template <bool SWIGLU, bool GATHER, bool TAIL, bool PIECES>
 __global__ __launch_bounds__(kRingThreads) void grouped_gemm_persistent_kernel(GemmParams p) {
     __shared__ __attribute__((aligned(1024))) char lds[kRingBytes];
     // Balanced row tiles for the gate/up GEMM at K >= 2048. There a short last
@@ -1049,7 +1055,7 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_persistent_kernel(G
     // as column pieces on every CU (781 -> 800 us at H=4096, I=14336).
     const RingTable table = ring_table(p, SWIGLU && p.k >= 2048);
     const int grid = static_cast<int>(gridDim.x);
-    const RingPlan plan = ring_plan(table.n_full, table.n_part, grid, !SWIGLU);
+    const RingPlan plan = ring_plan(table.n_full, table.n_part, grid, SWIGLU, PIECES);
     // The next tile of this workgroup at or after tile `sub` of virtual workgroup q.
     auto next = [&](int& q, int& sub) {
         RingWork w{false, 0, 0, 0, 0, 0};
@@ -1066,7 +1072,7 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_persistent_kernel(G
     RingWork cur = next(q, sub);
     if (!cur.valid) return;
     uint32_t a_carry[8];  // GATHER: the next tile's A offsets (at most 8 loads per wave and stage)
-    ring_prologue<SWIGLU, GATHER, TAIL>(p, lds, cur, a_carry);
+    ring_prologue<SWIGLU, GATHER, TAIL, PIECES>(p, lds, cur, a_carry);
     bool after_epilogue = false;
     int sa = 0, sb = 0;  // ring slots of the current tile's first stage
     for (;;) {
@@ -1087,7 +1093,7 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_persistent_kernel(G
             nxt.expert = e;
             nxt.variant = v;
         }
-        ring_run<SWIGLU, GATHER, TAIL>(p, lds, cur, nxt, after_epilogue, sa, sb, a_carry);
+        ring_run<SWIGLU, GATHER, TAIL, PIECES>(p, lds, cur, nxt, after_epilogue, sa, sb, a_carry);
         if (!nxt.valid) break;
         cur = nxt;
         q = qn;
@@ -1276,7 +1282,8 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_decode_kernel(GemmP
 }
 
 // Launches one of an instance family's kernels: the weight-streaming kernel with
-// row tiles of at most 64 or 128 rows, or the persistent one. Each family is
+// row tiles of at most 64 or 128 rows, or the persistent one; launch_pieces the
+// gate/up kernel that splits tiles (the plain one always does). Each family is
 // compiled in a file of its own (gemm_*.hip), which is minutes of work.
 enum class RingKernel { kStream64, kStream128, kPersistent };
 
@@ -1289,8 +1296,14 @@ void launch_ring(const GemmParams& p, RingKernel kernel, unsigned grid, hipStrea
         hipLaunchKernelGGL((grouped_gemm_decode_kernel<SWIGLU, 128, GATHER, TAIL>), dim3(grid), dim3(kRingThreads), 0,
                            stream, p);
     else
-        hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, GATHER, TAIL>), dim3(grid), dim3(kRingThreads), 0,
-                           stream, p);
+        hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, GATHER, TAIL, !SWIGLU>), dim3(grid),
+                           dim3(kRingThreads), 0, stream, p);
+}
+
+template <bool GATHER, bool TAIL>
+void launch_pieces(const GemmParams& p, unsigned grid, hipStream_t stream) {
+    hipLaunchKernelGGL((grouped_gemm_persistent_kernel<true, GATHER, TAIL, true>), dim3(grid), dim3(kRingThreads), 0,
+                       stream, p);
 }
 
 extern template void launch_ring<true, false, false>(const GemmParams&, RingKernel, unsigned, hipStream_t);
@@ -1298,5 +1311,8 @@ extern template void launch_ring<true, true, false>(const GemmParams&, RingKerne
 extern template void launch_ring<true, false, true>(const GemmParams&, RingKernel, unsigned, hipStream_t);
 extern template void launch_ring<false, false, false>(const GemmParams&, RingKernel, unsigned, hipStream_t);
 extern template void launch_ring<false, false, true>(const GemmParams&, RingKernel, unsigned, hipStream_t);
+extern template void launch_pieces<false, false>(const GemmParams&, unsigned, hipStream_t);
+extern template void launch_pieces<true, false>(const GemmParams&, unsigned, hipStream_t);
+extern template void launch_pieces<false, true>(const GemmParams&, unsigned, hipStream_t);
 
 }  // namespace moe

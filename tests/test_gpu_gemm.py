@@ -335,6 +335,48 @@ def test_partial_last_stage_equals_zero_padded(ext, counts, alignment, n, k):
         assert torch.equal(got[keep], want[keep])
 
 
+GATEUP_PIECES_CASES = [
+    # counts per expert, alignment, intermediate, k, workgroup bounds (0: one per CU)
+    ([90, 3, 128, 0, 64, 33], 8, 1400, 128, (0, 8, 24)),       # short tiles alone: halves, quarters
+    ([5] * 40, 8, 200, 192, (0, 8, 16)),                        # few rows per expert; a last piece past the columns
+    ([700, 300, 900], 8, 264, 2048, (0, 8, 16, 24)),            # balanced tiles alone: halves of a last round
+    ([520, 40, 260, 7], 8, 384, 64, (0, 8, 24)),                # short tiles after rounds: quarters, never halves
+    ([90, 3, 128, 0, 64, 33], 8, 1400, 200, (0, 8)),            # K not a multiple of 64
+]
+
+
+@pytest.mark.parametrize("counts,alignment,inter,k,grids", GATEUP_PIECES_CASES)
+def test_gateup_pieces_do_not_change_results(ext, counts, alignment, inter, k, grids):
+    """Gate/up tiles split into column halves and quarters: the fused output equals the
+    unfused pipeline's (near bit-exact) and is the same bit for bit on every grid size,
+    packed and gathered; rows past offsets[E] stay untouched."""
+    experts = len(counts)
+    a, offsets, rows = _inputs(counts, alignment, k, seed=inter + k)
+    g = torch.Generator(device="cuda").manual_seed(k)
+    w = (torch.randn(experts, 2 * inter, k, device="cuda", generator=g) / k**0.5).bfloat16()
+    used = int(to_np(offsets)[-1])
+    projection = torch.empty(rows, 2 * inter, device="cuda", dtype=torch.bfloat16)
+    ext.grouped_gemm_out(a, w, offsets, projection)
+    unfused = torch.empty(rows, inter, device="cuda", dtype=torch.bfloat16)
+    ext.swiglu_out(projection, offsets[-1:], unfused)
+    outs = []
+    try:
+        for grid in grids:
+            ext.set_gemm_workgroups(grid)
+            out = torch.full((rows, inter), 3.0, device="cuda").bfloat16()
+            ext.gateup_swiglu_out(a, w, offsets, out)
+            outs.append(out)
+            if k % 64 == 0:
+                out = torch.full((rows, inter), 3.0, device="cuda").bfloat16()
+                ext.gateup_swiglu_gathered_out(a, torch.arange(rows, device="cuda", dtype=torch.int32), w, offsets, out)
+                outs.append(out)
+    finally:
+        ext.set_gemm_workgroups(0)
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+    assert_near_bit_exact(to_np(outs[0])[:used], to_np(unfused)[:used], max_fraction=1e-4, max_steps=1.0)
+    assert torch.all(outs[0][used:] == 3.0)
+
+
 @pytest.mark.parametrize("counts,n", [
     ([2, 2], 4096),            # 32 columns (256 CUs: one tile each)
     ([1, 3, 2, 2], 8192),      # 64 columns

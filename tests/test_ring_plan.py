@@ -46,17 +46,19 @@ def balanced_for(swiglu, k):
     return swiglu and k >= 2048
 
 
-def ring_phase(count, grid, allow_split, short_tiles=False):
+def ring_phase(count, grid, allow_split, short_tiles=False, halves=True):
     rem = count % grid
-    split = allow_split and rem > 0 and 2 * rem <= grid
     ways = 4 if short_tiles and 4 * rem <= grid else 2
+    split = allow_split and rem > 0 and (ways == 4 or (halves and 2 * rem <= grid))
     main = count - rem if split else count
     return {"main": main, "blocks": (main + XCD - 1) // XCD * XCD, "pieces": ways * rem if split else 0,
             "ways": ways}
 
 
-def ring_plan(n1, n2, grid, allow_split):
-    half1 = allow_split and n2 > 0 and n1 > 0 and 2 * n1 <= grid
+def ring_plan(n1, n2, grid, allow_split, gateup_pieces=False):
+    """The plan of the plain GEMM (allow_split), of the gate/up kernel without pieces
+    (not allow_split), or with gateup_pieces of the gate/up kernel that splits tiles."""
+    half1 = allow_split and not gateup_pieces and n2 > 0 and n1 > 0 and 2 * n1 <= grid
     pl = {"n1": n1, "n2": n2, "half1": half1, "u1": 2 * n1 if half1 else n1, "per1": 0, "cpr": 0, "rounds": 0,
           "full_rounds": 0, "last_cols": 0, "slots": 0, "carried": 0}
     if n2 > 0 and n1 > 0:
@@ -68,7 +70,8 @@ def ring_plan(n1, n2, grid, allow_split):
         slots = rounds * grid - XCD * per1
         pl.update(per1=per1, rounds=rounds, cpr=cpr, full_rounds=per1 // cpr,
                   last_cols=per1 - (per1 // cpr) * cpr, slots=slots, carried=min(n2, 2 * slots))
-    pl["rest"] = ring_phase(n2 - pl["carried"] if n2 > 0 else n1, grid, allow_split, n2 > 0)
+    pl["rest"] = ring_phase(n2 - pl["carried"] if n2 > 0 else n1, grid, allow_split, n2 > 0,
+                            not gateup_pieces or n1 == 0 or n2 == 0)
     pl["virtual_blocks"] = pl["rounds"] * grid + pl["rest"]["blocks"] + pl["rest"]["pieces"]
     return pl
 
@@ -111,9 +114,9 @@ def ring_slot(pl, grid, q, sub):
     return None
 
 
-def walk(n1, n2, grid, allow_split):
+def walk(n1, n2, grid, allow_split, gateup_pieces=False):
     """Per workgroup, the (phase, tile, piece) sequence it runs."""
-    pl = ring_plan(n1, n2, grid, allow_split)
+    pl = ring_plan(n1, n2, grid, allow_split, gateup_pieces)
     runs = []
     for wg in range(grid):
         seq = []
@@ -126,8 +129,8 @@ def walk(n1, n2, grid, allow_split):
     return pl, runs
 
 
-def check_cover(n1, n2, grid, allow_split):
-    pl, runs = walk(n1, n2, grid, allow_split)
+def check_cover(n1, n2, grid, allow_split, gateup_pieces=False):
+    pl, runs = walk(n1, n2, grid, allow_split, gateup_pieces)
     seen = {}
     for seq in runs:
         for _, (phase, tile, piece) in seq:
@@ -277,3 +280,20 @@ def test_phase1_tile_order_covers_each_tile_once_in_groups_of_eight():
     for start in range(0, len(tiles) - 32, 32):
         window = tiles[start:start + 32]
         assert len({m for _, m in window}) <= 16 and len({n for n, _ in window}) >= 2
+
+
+def test_gateup_pieces_plans():
+    """The gate/up kernel that splits tiles: every tile or its pieces run once, and the
+    measured shapes get their plans."""
+    rng = random.Random(11)
+    for _ in range(200):
+        grid = 8 * rng.randint(1, 32)
+        check_cover(rng.choice([0, rng.randint(0, 900)]), rng.choice([0, rng.randint(0, 900)]), grid, True, True)
+    # H=4096, I=14336, 8 experts of at most 128 rows: three rounds and 256 halves.
+    pl, _ = check_cover(0, 8 * 112, 256, True, True)
+    assert (pl["rest"]["main"], pl["rest"]["pieces"], pl["rest"]["ways"]) == (768, 256, 2)
+    # H=2048, I=1408: six active experts as 132 halves, 51 as two rounds and 196 quarters.
+    assert check_cover(0, 66, 256, True, True)[0]["rest"]["pieces"] == 132
+    assert check_cover(0, 561, 256, True, True)[0]["rest"]["pieces"] == 196
+    # H=1024, I=2048, 8192 rows: 128 short tiles after full rounds stay whole.
+    assert check_cover(512, 128, 256, True, True)[0]["rest"]["pieces"] == 0
