@@ -519,6 +519,57 @@ int moe_grouped_gateup_swiglu_gathered_strided(const void* x, const int32_t* row
                                          rows, hidden, intermediate, (int)experts, static_cast<hipStream_t>(stream));
 }
 
+int moe_block_forward(const moe_block_args* args, const void* x, const float* router_w, void* stream) {
+    MOE_REQUIRE(args, MOE_ERR_INVALID_ARGUMENT, "null pointer");
+    const moe_block_args& a = *args;
+    MOE_REQUIRE(a.struct_bytes == static_cast<int64_t>(sizeof(moe_block_args)), MOE_ERR_INVALID_ARGUMENT,
+                "moe_block_args has %lld bytes, expected %lld", (long long)a.struct_bytes,
+                (long long)sizeof(moe_block_args));
+    const bool rows = a.gathered != 0 || a.one_pass != 0;
+    int rc;
+    if (a.one_pass != 0) {
+        rc = moe_route_rows(x, router_w, a.bias, a.ids32, a.ids64, a.weights, a.router_scratch,
+                            a.router_scratch_bytes, a.counts, a.offsets, a.slots, a.inverse, a.row_src, a.sums,
+                            a.sums_bytes, a.tokens, a.hidden, a.experts, a.topk, a.alignment, a.packed_rows, stream);
+    } else {
+        const bool ranked = a.tile_tokens > 0;
+        rc = ranked ? moe_router_fused_ranked(x, router_w, a.bias, a.ids32, a.ids64, a.weights, nullptr,
+                                              a.router_scratch, a.router_scratch_bytes, a.tokens, a.hidden, a.experts,
+                                              a.topk, a.ranks, a.tile_counts, a.tile_counts_bytes, stream)
+                    : moe_router_fused(x, router_w, a.bias, a.ids32, a.ids64, a.weights, nullptr, a.router_scratch,
+                                       a.router_scratch_bytes, a.tokens, a.hidden, a.experts, a.topk, stream);
+        if (rc != MOE_OK) return rc;
+        if (rows && ranked)
+            rc = moe_dispatch_ranked_rows(a.ids32, a.counts, a.offsets, a.slots, a.inverse, a.row_src, a.ranks,
+                                          a.tile_counts, a.tile_counts_bytes, a.tile_tokens, a.tokens, a.experts,
+                                          a.topk, a.alignment, a.packed_rows, stream);
+        else if (rows)
+            rc = moe_dispatch_rows(a.ids32, a.counts, a.offsets, a.slots, a.inverse, a.row_src, a.dispatch_scratch,
+                                   a.dispatch_scratch_bytes, a.tokens, a.experts, a.topk, a.alignment, a.packed_rows,
+                                   stream);
+        else if (ranked)
+            rc = moe_dispatch_ranked(x, MOE_DTYPE_BF16, a.ids32, a.counts, a.offsets, a.slots, a.packed, a.inverse,
+                                     a.ranks, a.tile_counts, a.tile_counts_bytes, a.tile_tokens, a.tokens, a.hidden,
+                                     a.experts, a.topk, a.alignment, a.packed_rows, a.vectorized != 0, stream);
+        else
+            rc = moe_dispatch(x, MOE_DTYPE_BF16, a.ids32, a.counts, a.offsets, a.slots, a.packed, a.inverse,
+                              a.dispatch_scratch, a.dispatch_scratch_bytes, a.tokens, a.hidden, a.experts, a.topk,
+                              a.alignment, a.packed_rows, a.vectorized != 0, stream);
+    }
+    if (rc != MOE_OK) return rc;
+    rc = rows ? moe_grouped_gateup_swiglu_gathered_strided(x, a.row_src, a.tokens, a.gate_up, a.gate_up_row_stride,
+                                                           a.activated, a.offsets, a.packed_rows, a.hidden,
+                                                           a.intermediate, a.experts, stream)
+              : moe_grouped_gateup_swiglu_strided(a.packed, a.gate_up, a.gate_up_row_stride, a.activated, a.offsets,
+                                                  a.packed_rows, a.hidden, a.intermediate, a.experts, stream);
+    if (rc != MOE_OK) return rc;
+    rc = moe_grouped_gemm_strided(a.activated, a.down, a.down_row_stride, a.expert_output, a.offsets, a.packed_rows,
+                                  a.hidden, a.intermediate, a.experts, stream);
+    if (rc != MOE_OK) return rc;
+    return moe_combine(a.expert_output, MOE_DTYPE_BF16, a.inverse, a.weights, a.output, a.tokens, a.hidden, a.topk,
+                       a.packed_rows, stream);
+}
+
 int moe_set_gemm_workgroups(int64_t workgroups) {
     MOE_REQUIRE(workgroups >= 0 && workgroups <= INT_MAX, MOE_ERR_INVALID_ARGUMENT,
                 "workgroups must be in [0, INT_MAX]");

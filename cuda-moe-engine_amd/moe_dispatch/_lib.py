@@ -62,10 +62,28 @@ _SIGNATURES = {
                                           + [_c_void_p]),
     "moe_grouped_gateup_swiglu_gathered_strided": (_int, [_c_void_p, _c_void_p, _i64, _c_void_p, _i64]
                                                    + [_c_void_p] * 2 + [_i64] * 4 + [_c_void_p]),
+    "moe_block_forward": (_int, [_c_void_p] * 4),
     "moe_set_gemm_workgroups": (_int, [_i64]),
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
+
+
+class BlockArgs(ctypes.Structure):
+    """``moe_block_args``: pointers and 64-bit sizes, all of eight bytes, in the header's order."""
+
+    _POINTERS = ("bias", "ids32", "ids64", "weights", "router_scratch", "counts", "offsets", "slots", "inverse",
+                 "row_src", "packed", "dispatch_scratch", "ranks", "tile_counts", "sums", "gate_up", "down",
+                 "activated", "expert_output", "output")
+    _ORDER = ("struct_bytes", "bias", "ids32", "ids64", "weights", "router_scratch", "router_scratch_bytes", "counts",
+              "offsets", "slots", "inverse", "row_src", "packed", "dispatch_scratch", "dispatch_scratch_bytes",
+              "ranks", "tile_counts", "tile_counts_bytes", "tile_tokens", "sums", "sums_bytes", "gate_up",
+              "gate_up_row_stride", "down", "down_row_stride", "activated", "expert_output", "output", "tokens",
+              "hidden", "intermediate", "experts", "topk", "alignment", "packed_rows", "vectorized", "gathered",
+              "one_pass")
+
+
+BlockArgs._fields_ = [(name, _c_void_p if name in BlockArgs._POINTERS else _i64) for name in BlockArgs._ORDER]
 
 
 def library_path() -> Path:

@@ -16,6 +16,7 @@ Top-k may be 1..8 (the reference allows 1 or 2); ``set_routing_bias`` sets an
 arbitrary router bias.
 """
 
+import ctypes
 from dataclasses import dataclass
 import math
 
@@ -322,18 +323,22 @@ class MoEBlock(torch.nn.Module):
         )
         return state.expert_output
 
-    @torch.inference_mode()
     def forward(self, x):
+        if self.implementation == "cuda_fused" and x.ndim == 2:
+            # No torch operator runs on this path, so it needs no inference mode.
+            launches = self._launches.get((x.shape[0], x.device))
+            if launches is not None and launches.accepts(x) and launches.still_valid(self):
+                return launches(self, x)
+        return self._validated_forward(x)
+
+    @torch.inference_mode()
+    def _validated_forward(self, x):
         if x.ndim != 2 or x.shape[1] != self.config.hidden or not x.is_contiguous():
             raise ValueError("expected contiguous x[T,hidden]")
         if x.dtype != self.gate_up_weight.dtype or x.device != self.gate_up_weight.device:
             raise ValueError("input dtype/device must match expert weights")
         if x.shape[0] == 0:
             return torch.empty_like(x)
-        if self.implementation == "cuda_fused":
-            launches = self._launches.get((x.shape[0], x.device))
-            if launches is not None and launches.still_valid(self):
-                return launches(self, x)
         state = self.workspace(x)
         fused = self.implementation == "cuda_fused"
         # The fused router does the dispatch's counting pass when the shape allows.
@@ -397,14 +402,15 @@ class _FusedLaunches:
     A forward through the validating operators (router_fused_out, dispatch,
     the two grouped GEMMs, combine) fixes every argument but x's address and
     the stream: workspace and weight pointers, sizes, the dtype code. Later
-    forwards of the same token count on the same device make the same five
-    calls (four where a small batch routes and dispatches in one pass) with those arguments while every parameter tensor the calls read is
+    forwards of the same token count on the same device make the same launches
+    through one native call (``moe_block_forward``) on those arguments while every
+    parameter tensor the kernels read is
     the object it was, at the same address, with the same dtype, shape and
     layout (an in-place update keeps all of these; the router split follows
     the weights' version as in ``MoEBlock.route``). Anything else sends the
     forward back through the validating path, which raises on a bad tensor.
-    This removes about 50 us of host work per forward (validation and stream
-    lookups), which dominates the eager latency of small batches.
+    Host work per forward: about 80 us through the operators, 31 with one foreign call
+    per launch, 24 with one, at 128 tokens of 512 where the kernels take about 22.
     """
 
     _PARAMETERS = ("router_weight", "gate_up_weight", "down_weight", "routing_bias", "_router_scratch")
@@ -437,13 +443,8 @@ class _FusedLaunches:
             raise RuntimeError("expert weights must be contiguous or row-padded")
         # Small batches: routing and the row-table dispatch in one pass (every
         # output as the two calls write it), its plane sums owned by these launches.
-        self.route_rows = None
         if sums_bytes is not None:
             self.sums = torch.empty(max(sums_bytes, 4), dtype=torch.uint8, device=x.device)
-            self.route_rows = self.router[:4] + self.router[5:7] + (
-                t.counts.data_ptr(), t.offsets.data_ptr(), t.slots.data_ptr(), t.inverse.data_ptr(),
-                t.row_src.data_ptr(), self.sums.data_ptr(), self.sums.numel(), tokens, hidden, cfg.experts, cfg.topk,
-                t.alignment, rows)
         index = (ids32.data_ptr(), t.counts.data_ptr(), t.offsets.data_ptr(), t.slots.data_ptr())
         if self.ranked:
             self.router += (t.tile_ranks.data_ptr(), t.tile_counts.data_ptr(), t.tile_counts.numel() * 4)
@@ -479,47 +480,58 @@ class _FusedLaunches:
         self.output = t.output
         if x.dtype != torch.bfloat16:
             raise RuntimeError("cuda_fused launches are bf16")
+        # The whole forward as one call (moe_block_forward).
+        args = _lib.BlockArgs(
+            struct_bytes=ctypes.sizeof(_lib.BlockArgs), router_scratch_bytes=scratch.numel() * scratch.element_size(),
+            dispatch_scratch_bytes=t.scratch.numel() * t.scratch.element_size(),
+            tile_counts_bytes=t.tile_counts.numel() * 4, tile_tokens=t.rank_tile,
+            sums_bytes=self.sums.numel() if sums_bytes is not None else 0, gate_up_row_stride=gate_up_stride,
+            down_row_stride=down_stride, tokens=tokens, hidden=hidden, intermediate=cfg.intermediate,
+            experts=cfg.experts, topk=cfg.topk, alignment=t.alignment, packed_rows=rows,
+            vectorized=int(bool(t.vectorized)), gathered=int(self.gathered), one_pass=int(sums_bytes is not None))
+        for name, tensor in (
+                ("bias", block.routing_bias), ("ids32", ids32), ("ids64", ids64), ("weights", weights),
+                ("router_scratch", scratch), ("counts", t.counts), ("offsets", t.offsets), ("slots", t.slots),
+                ("inverse", t.inverse), ("row_src", t.row_src), ("packed", t.packed), ("dispatch_scratch", t.scratch),
+                ("ranks", t.tile_ranks), ("tile_counts", t.tile_counts),
+                ("sums", self.sums if sums_bytes is not None else None), ("gate_up", block.gate_up_weight),
+                ("down", block.down_weight), ("activated", state.activated), ("expert_output", state.expert_output),
+                ("output", t.output)):
+            setattr(args, name, None if tensor is None else tensor.data_ptr())
+        self.args = args
+        self.args_address = ctypes.addressof(args)
 
     @classmethod
     def _fingerprint(cls, block):
         tensors = tuple(getattr(block, name) for name in cls._PARAMETERS)
-        return tensors, tuple((v.data_ptr(), v.dtype, tuple(v.shape), v.stride()) for v in tensors)
+        return tuple((name, v, v.data_ptr(), v.dtype, v.shape, v.stride()) for name, v in zip(cls._PARAMETERS, tensors))
 
     def still_valid(self, block):
-        tensors, described = self.fingerprint
-        current = tuple(getattr(block, name) for name in self._PARAMETERS)
-        if not all(a is b for a, b in zip(current, tensors)):
-            return False
-        return all((v.data_ptr(), v.dtype, tuple(v.shape), v.stride()) == d for v, d in zip(current, described))
+        buffers, plain = block._buffers, block.__dict__
+        for name, v, address, dtype, shape, stride in self.fingerprint:
+            current = plain.get(name)
+            if current is None:  # getattr's other places: buffers, and parameters set over one
+                current = buffers.get(name)
+                if current is None:
+                    current = block._parameters.get(name)
+            if current is not v or v.data_ptr() != address or v.shape != shape or v.stride() != stride \
+                    or v.dtype != dtype:
+                return False
+        return True
+
+    def accepts(self, x):
+        """The caller's half of the checks (the key these launches are kept under has its
+        token count and device; the weights' device and dtype are theirs)."""
+        return x.dtype == torch.bfloat16 and x.shape[1] == self.args.hidden and x.is_contiguous()
 
     def __call__(self, block, x):
-        lib = self.lib
-        stream = current_stream_handle(self.device_index)
-        x_ptr = x.data_ptr()
         router_weight, split_of = block._router_split_plan()
-        if self.route_rows is not None:
-            lib.check(lib.moe_route_rows(x_ptr, router_weight, *self.route_rows, stream), "route_rows")
-        elif self.ranked:
-            lib.check(lib.moe_router_fused_ranked(x_ptr, router_weight, *self.router, stream), "router_fused_out")
-        else:
-            lib.check(lib.moe_router_fused(x_ptr, router_weight, *self.router, stream), "router_fused_out")
-        block._router_split_of = split_of
-        if self.gathered:
-            if self.route_rows is None:
-                if self.ranked:
-                    lib.check(lib.moe_dispatch_ranked_rows(*self.dispatch, stream), "dispatch")
-                else:
-                    lib.check(lib.moe_dispatch_rows(*self.dispatch, stream), "dispatch")
-            lib.check(lib.moe_grouped_gateup_swiglu_gathered_strided(x_ptr, *self.gateup, stream),
-                      "gateup_swiglu_out")
-        else:
-            if self.ranked:
-                lib.check(lib.moe_dispatch_ranked(x_ptr, *self.dispatch, stream), "dispatch")
-            else:
-                lib.check(lib.moe_dispatch(x_ptr, *self.dispatch, stream), "dispatch")
-            lib.check(lib.moe_grouped_gateup_swiglu_strided(*self.gateup, stream), "gateup_swiglu_out")
-        lib.check(lib.moe_grouped_gemm_strided(*self.down, stream), "grouped_gemm_out")
-        lib.check(lib.moe_combine(*self.combine, stream), "combine_out")
+        status = self.lib.moe_block_forward(self.args_address, x.data_ptr(), router_weight,
+                                            current_stream_handle(self.device_index))
+        if status:
+            self.lib.check(status, "forward")
+        if router_weight is not None:  # else the split it holds is the one it has on record
+            block._router_split_of = split_of
         return self.output
 
     def stage_calls(self, x):

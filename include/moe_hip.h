@@ -333,6 +333,61 @@ int moe_grouped_gateup_swiglu_gathered_strided(const void* x, const int32_t* row
                                                int64_t intermediate, int64_t experts, void* stream);
 
 /*
+ * One MoE block forward: the calls above in order on one stream, so that a
+ * caller which keeps its buffers makes one call per forward (a decoding step's
+ * five calls through a foreign-function interface cost more than its kernels).
+ * Each call makes its own checks; the first non-OK status is returned. The
+ * pointers and sizes are those calls' arguments of the same names. Routing:
+ * moe_route_rows when `one_pass` is non-zero, else moe_router_fused_ranked when
+ * tile_tokens > 0, else moe_router_fused; then the matching dispatch (the row table
+ * and the gathered gate/up GEMM when `gathered` or `one_pass` is non-zero), gate/up,
+ * down and combine. bf16. struct_bytes is sizeof(moe_block_args). router_w == NULL
+ * carries moe_router_fused's precondition. No counterpart in the reference.
+ */
+typedef struct moe_block_args {
+    int64_t struct_bytes;
+    const float* bias;
+    int32_t* ids32;
+    int64_t* ids64;
+    float* weights;
+    void* router_scratch;
+    int64_t router_scratch_bytes;
+    int32_t* counts;
+    int32_t* offsets;
+    int32_t* slots;
+    int32_t* inverse;
+    int32_t* row_src;
+    void* packed;
+    void* dispatch_scratch;
+    int64_t dispatch_scratch_bytes;
+    int32_t* ranks;
+    int32_t* tile_counts;
+    int64_t tile_counts_bytes;
+    int64_t tile_tokens;
+    void* sums;
+    int64_t sums_bytes;
+    const void* gate_up;
+    int64_t gate_up_row_stride;
+    const void* down;
+    int64_t down_row_stride;
+    void* activated;
+    void* expert_output;
+    void* output;
+    int64_t tokens;
+    int64_t hidden;
+    int64_t intermediate;
+    int64_t experts;
+    int64_t topk;
+    int64_t alignment;
+    int64_t packed_rows;
+    int64_t vectorized;
+    int64_t gathered;
+    int64_t one_pass;
+} moe_block_args;
+
+int moe_block_forward(const moe_block_args* args, const void* x, const float* router_w, void* stream);
+
+/*
  * Upper bound on the workgroups of the persistent grouped GEMM (both
  * moe_grouped_gemm and moe_grouped_gateup_swiglu): 0 (the default) runs one
  * per CU; n > 0 runs min(n, CUs), rounded down to a multiple of 8 (at least 8).

@@ -266,3 +266,21 @@ def test_route_rows_arguments_are_checked_before_launch():
     assert call(sums_bytes=sums - 1) not in (ok, invalid, unsupported)
     assert call(sums_ptr=None) not in (ok, unsupported) and call(sums_ptr=24) == invalid
     assert call(tokens=129, packed_rows=129 * 6) == unsupported and call(tokens=17, experts=16) == unsupported
+
+
+@stand_in_addresses
+def test_block_args_match_the_header_and_are_checked():
+    """BlockArgs restates moe_block_args field by field, and the call refuses another size."""
+    text = HEADER.read_text()
+    body = re.search(r"typedef struct moe_block_args \{(.*?)\}", text, flags=re.S).group(1)
+    fields = [(d.split()[-1].lstrip("*"), "*" in d) for d in body.split(";") if d.strip()]
+    assert [(name, kind is ctypes.c_void_p) for name, kind in _lib.BlockArgs._fields_] == fields
+    assert ctypes.sizeof(_lib.BlockArgs) == 8 * len(fields)
+    lib = _lib.load_library()
+    assert lib.moe_block_forward(None, 16, 16, None) == 1
+    args = _lib.BlockArgs(struct_bytes=8)
+    assert lib.moe_block_forward(ctypes.addressof(args), 16, 16, None) == 1
+    # Each stage makes its own checks: no tokens' buffers here.
+    args = _lib.BlockArgs(struct_bytes=ctypes.sizeof(_lib.BlockArgs), tokens=4, hidden=64, intermediate=64, experts=8,
+                          topk=2, alignment=8, packed_rows=96)
+    assert lib.moe_block_forward(ctypes.addressof(args), 16, 16, None) == 1

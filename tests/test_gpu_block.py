@@ -326,6 +326,28 @@ def test_padded_weight_rows_equal_contiguous_weights(cfg):
     assert torch.equal(block(x).clone(), twin(x))
 
 
+def test_native_forward_follows_replaced_parameters():
+    """The one-call forward is used while the tensors are the bound ones: a parameter set
+    over a buffer, a resized storage and a wrong input go back through the checks."""
+    cfg = MoEConfig(128, 192, 8, 2)
+    block = MoEBlock(cfg, device="cuda", implementation="cuda_fused", seed=3)
+    x = torch.randn(40, 128, device="cuda").bfloat16()
+    block(x)
+    down = (torch.randn(8, 128, 192, device="cuda") / 14).bfloat16()
+    block.down_weight = torch.nn.Parameter(down, requires_grad=False)
+    twin = MoEBlock(cfg, device="cuda", implementation="cuda_fused", seed=3)
+    twin.down_weight.copy_(down)
+    want = twin(x).clone()
+    for _ in range(3):
+        assert torch.equal(block(x), want)
+    assert block._launches[(40, x.device)].still_valid(block)
+    block.down_weight.data = torch.zeros_like(down)
+    assert torch.all(block(x) == 0)
+    for bad in (x[:, :64], x.float(), x.t().contiguous().t(), x.cpu()):
+        with pytest.raises(ValueError):
+            block(bad)
+
+
 def test_empty_batch():
     block = MoEBlock(MoEConfig(64, 128, 8, 2), device="cuda", implementation="cuda_fused")
     out = block(torch.empty(0, 64, device="cuda", dtype=torch.bfloat16))
