@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256) void topk_route_kernel(const float* __restrict
 
 constexpr int kRouterTokens = 16;
 constexpr int64_t kRankedPrefixMax = 4096;  // routing tiles x experts of a ranked route
-constexpr int kRouterSplitTokens = 64;  // split-k routing up to this many tokens (E <= 16)
+constexpr int kRouterSplitTokens = 64;  // split-k routing up to this many tokens (E <= 16, hidden past the direct kernel's)
 constexpr int kRouterSplitSlices = 16;
 constexpr int kRouterSplitTiles = kRouterSplitTokens / kRouterTokens;
 constexpr int64_t kRouterPartialBytes =
@@ -312,8 +312,8 @@ struct RouterShape {
 // b / slices and the k-slice b % slices of `per` stages, loads the whole slice
 // into its ring at once and writes the slice's partial logits to
 // partials[tile][slice][TB][EB]; router_reduce_kernel adds the slices in
-// slice order and selects. One token's routing at H=4096 otherwise streams its
-// 204 KB of weight planes through one CU, latency-bound (11 us). (A last-block
+// slice order and selects. Used past the hidden sizes of router_direct_kernel (one
+// token's planes are then 400 KB and more through one CU). (A last-block
 // reduction inside this kernel needs a device-scope release per block, an L2
 // write-back that costs more than the second launch.)
 template <int NT, int MT, bool SPLIT = false>
@@ -915,7 +915,7 @@ __device__ __forceinline__ void write_rows_layout(const int* ids, int n, int exp
 // E <= 16, hidden <= 8192, at most 16 tokens: the batch in one block of 16 waves
 // that split the 64-k steps, on router_direct_kernel's operands. Bound by the
 // latency of its loads, exchanges and code, not by bytes. H=4096, E=8, with the
-// layout: 6.9 us at one token and 7.9 at 16, where split-k partials, their sum
+// layout: 6.6 us at one token and 7.5 at 16, where split-k partials, their sum
 // and the pack kernel took 12.6 and 13.8. Two or more token tiles in the block
 // lost to one block each and a separate row-table dispatch (17 tokens: 10.0
 // against 9.7 us; 128 tokens of 512: 8.8 against 7.9).
