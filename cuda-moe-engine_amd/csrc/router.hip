@@ -172,14 +172,16 @@ __global__ __launch_bounds__(256) void router_split_kernel(const float* __restri
 // Rows of 128 bytes hold 8 chunks of 16 bytes; chunk c of row r sits at
 // physical chunk c ^ ((r >> 1) & 7), so 16 lanes reading 16 consecutive rows
 // at one chunk are conflict free.
-// The value of another lane of the same eight: the neighbour (STEP 0), the lane
-// two further (1), and for values equal inside each half of the eight the other
-// half's (2, a mirror). DPP moves take a few cycles where a shuffle goes through
-// LDS, and a selection has 6 * K of them one after another.
+// The value of lane sub ^ (1 << STEP) of the same eight. DPP moves take a few
+// cycles where a shuffle goes through LDS, and a selection has 6 * K of them one
+// after another. (No DPP control is an xor with 4: a mirror of the eight, sub ^ 7,
+// and the reversal of each four, sub ^ 3, make one.)
 template <int STEP>
 __device__ __forceinline__ int eight_lane_peer(int v) {
     constexpr int ctrl = STEP == 0 ? 0xB1 : STEP == 1 ? 0x4E : 0x141;  // quad_perm 1032, 2301, row_half_mirror
-    return __builtin_amdgcn_update_dpp(v, v, ctrl, 0xf, 0xf, false);
+    const int peer = __builtin_amdgcn_update_dpp(v, v, ctrl, 0xf, 0xf, false);
+    if constexpr (STEP < 2) return peer;
+    return __builtin_amdgcn_update_dpp(peer, peer, 0x1B, 0xf, 0xf, false);  // quad_perm 3210
 }
 
 // Top-k over one token's biased logits held by eight lanes (lane `sub` holds
@@ -188,8 +190,10 @@ __device__ __forceinline__ int eight_lane_peer(int v) {
 // lanes in three exchanges, then the winner is removed -- the
 // reference's iterative argmax with ties to the lower id. Lane j keeps round j's
 // winner, so the weights (write_route's, in its order: K = 1 and 2 are cases of
-// the general form, whose first term is exactly 1) take one exp, and a lane
-// each stores the ids and weights. With the rounds unrolled into register
+// the general form with a first term of 1, also for an infinite winner) take one
+// exp, and a lane each stores the ids and weights. Lane 0's round 0 is the one
+// that counts: a NaN keeps its own lane from seeing the others' winner there, and
+// is gone (removed, or passed over) from round 1 on. With the rounds unrolled into register
 // arrays that one lane turned into weights and stores, the selection was 6-8 KB
 // of straight-line code, and fetching it cost the small routers more than their
 // products. With the rank step below, H=2048, E=64, top-6 went from 30.8 to 19.1
@@ -224,8 +228,9 @@ __device__ __forceinline__ void select_eight_lanes(float (&v)[EPL], int sub, int
 #pragma unroll
         for (int j = 0; j < EPL; ++j) v[j] = (sub * EPL + j == bi) ? -INFINITY : v[j];
     }
-    const float rel = expf(value - first);
     const int lane0 = static_cast<int>(threadIdx.x & 63) - sub;
+    first = __shfl(first, lane0);
+    const float rel = topk <= 2 && sub == 0 ? 1.0f : expf(value - first);
     float total = 0.0f;
 #pragma unroll
     for (int j = 0; j < kMaxTopk; ++j) {

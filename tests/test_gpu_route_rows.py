@@ -65,3 +65,38 @@ def test_shapes_without_a_one_pass_route(ext):
     need = ext.lib.moe_route_rows_scratch_bytes
     assert need(17, 512, 16, 2) == -1 and need(1, 8200, 8, 2) == -1
     assert need(129, 512, 17, 2) == -1 and need(1, 4104, 17, 2) == -1 and need(128, 4096, 17, 8) > 0
+
+
+# One call per selection form: E <= 16 in one workgroup, by direct loads, and
+# E > 16. The logits are the biases (x is zero), so the selection is known exactly.
+@pytest.mark.parametrize("tokens,experts", [(3, 8), (16, 16), (200, 8), (3, 40), (200, 64)])
+@pytest.mark.parametrize("topk", [1, 2, 4, 7])
+@pytest.mark.parametrize("kind", ["plus_inf", "minus_inf", "nan"])
+def test_infinite_and_nan_logits(ext, tokens, experts, topk, kind):
+    hidden = 256
+    x = torch.zeros(tokens, hidden, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(experts, hidden, device="cuda")
+    bias = torch.arange(experts, 0, -1, dtype=torch.float32) / 16  # the lower expert is the larger
+    per_lane = 2 if experts <= 16 else 8
+    if kind == "plus_inf":  # a pinned expert
+        bias[experts - 1] = float("inf")
+    elif kind == "minus_inf":  # masked experts, at least topk others left in use
+        bias[: experts - topk] = float("-inf")
+    else:  # the first expert of the second lane: never the largest in a comparison
+        bias[per_lane] = float("nan")
+    order = torch.where(bias.isnan(), torch.full_like(bias, float("-inf")), bias)
+    want_ids = torch.sort(order, descending=True, stable=True).indices[:topk]
+    picked = bias[want_ids].double()
+    if topk <= 2 and kind == "plus_inf":
+        want = torch.tensor([1.0, 0.0], dtype=torch.float64)[:topk]
+    else:  # from top-3 on an infinite winner's own term is exp(inf - inf)
+        want = torch.exp(picked - picked[0])
+        want = want / want.sum()
+    ids32 = torch.empty(tokens, topk, device="cuda", dtype=torch.int32)
+    ids64, weights = ids32.long(), ids32.float()
+    scratch = torch.empty(ext.router_scratch_bytes(experts, hidden), dtype=torch.uint8, device="cuda")
+    ext.router_fused_out(x, w, bias.cuda(), ids32, ids64, weights, scratch=scratch)
+    assert torch.equal(ids64.cpu(), want_ids.expand(tokens, topk))
+    assert torch.equal(ids32.cpu().long(), ids64.cpu())
+    # 32-bit exp, sum and product: a few units in the last place.
+    torch.testing.assert_close(weights.cpu().double(), want.expand(tokens, topk), rtol=1e-6, atol=1e-9, equal_nan=True)
