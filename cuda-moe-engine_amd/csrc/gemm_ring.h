@@ -17,10 +17,11 @@
 //    experts' short last row tiles carried beside them; 32- and 64-column tiles
 //    for decode-sized launches.
 //  * K not a multiple of 64 runs the same kernels with the last stage
-//    zero-filled past K (TAIL). A register-staged kernel with one barrier per
-//    k-step served those before: at H=1000, I=2744, 12 experts, top-3, gate/up
-//    took 124.9 us and down 109.3 us at 777 tokens against 67.8 and 44.0 us
-//    now, and 43.8 and 95.4 us against 26.5 and 12.4 us at 7.
+//    zero-filled past K (TAIL) and the standalone activation's arithmetic in the
+//    epilogue. A register-staged kernel with one barrier per k-step served those
+//    before: at H=1000, I=2744, 12 experts, top-3, replayed, gate/up took 121.2 us
+//    and down 109.8 us at 777 tokens against 65.7 and 44.8 us now, and 43.1 and
+//    96.2 us against 23.6 and 13.5 us at 7.
 //  * The tile schedule is built on the device from offsets: no offsets are read
 //    on the host, and the persistent grid is one workgroup per CU.
 //  * Every output element is one MFMA chain in ascending k with one fp32
@@ -134,9 +135,17 @@ constexpr int ring_a_stages(uint32_t a_stage, uint32_t b_stage, uint32_t bytes, 
 
 __device__ __forceinline__ int ring_key(int row) { return (row >> 1) & 7; }
 
-// silu(g) * u for the fused epilogue: hardware exp2 and reciprocal
-// (v_exp_f32, v_rcp_f32; about 1 ulp each), g and u already rounded to bf16.
-__device__ __forceinline__ float swiglu_fast(float g, float u) {
+// silu(g) * u for the fused epilogue, g and u already rounded to bf16.
+// K a multiple of 64: hardware exp2 and reciprocal (v_exp_f32, v_rcp_f32; about
+// 1 ulp each). The exponent's rounding grows with |g|: up to 3.4e-6 before the
+// bf16 rounding at |g| of some tens, and g * u overflows on its own past 3.4e38.
+// Other K (EXACT): the standalone kernel's silu_f32 (within 2e-7, the product
+// formed last, so g = -1e30, u = 1e30 is -0), as these shapes had on the kernel
+// they ran on before. It costs about 35 VALU operations an element more: at
+// H=1000, I=2744, 12 experts, top-3, gate/up 51.9 -> 65.7 us at 777 tokens.
+template <bool EXACT>
+__device__ __forceinline__ float swiglu_act(float g, float u) {
+    if constexpr (EXACT) return silu_f32(g) * u;
     const float e = __builtin_amdgcn_exp2f(-g * 1.4426950408889634f);
     return (g * u) * __builtin_amdgcn_rcpf(1.0f + e);
 }
@@ -631,7 +640,7 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, char* lds, int ex
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const uint32_t gu = pack_bf16x2(acc[i][j][t], acc[i][j + FB / 2][t]);
-                    act[t] = swiglu_fast(__uint_as_float(gu << 16), __uint_as_float(gu & 0xffff0000u));
+                    act[t] = swiglu_act<TAIL>(__uint_as_float(gu << 16), __uint_as_float(gu & 0xffff0000u));
                 }
                 out[j] = make_uint2(pack_bf16x2(act[0], act[1]), pack_bf16x2(act[2], act[3]));
             } else {

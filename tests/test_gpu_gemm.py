@@ -9,10 +9,11 @@ that are not multiples of the column tile, decode-sized launches (at most 128
 rows, which take 32- and 64-column tiles), and the fused gate/up + SwiGLU
 epilogue against the kernels' own unfused pipeline (grouped GEMM -> bf16
 projection -> standalone SwiGLU). The two see the same bf16 gate and up values;
-the fused epilogue evaluates silu with the hardware exp2 and reciprocal
-(v_exp_f32, v_rcp_f32, about 1 ulp each) while the standalone kernel uses the
-correctly ordered fp32 sequence the oracle reproduces, so after the bf16
-rounding they may differ by one bf16 step in a few elements per 100 000.
+for K a multiple of 64 the fused epilogue evaluates silu with the hardware exp2
+and reciprocal (v_exp_f32, v_rcp_f32, about 1 ulp each) while the standalone
+kernel uses the correctly ordered fp32 sequence the oracle reproduces, so after
+the bf16 rounding they may differ by one bf16 step in a few elements per 100 000.
+For other K the fused epilogue runs the standalone sequence.
 """
 
 import numpy as np
@@ -20,7 +21,7 @@ import pytest
 import torch
 
 from oracle import moe_oracle as oracle
-from tests._helpers import assert_near_bit_exact, gpu, rel_l2, to_np
+from tests._helpers import assert_near_bit_exact, gpu, raw_bits, rel_l2, to_np
 
 pytestmark = gpu
 
@@ -313,8 +314,9 @@ PARTIAL_STAGE_CASES = [
 def test_partial_last_stage_equals_zero_padded(ext, counts, alignment, n, k):
     """K not a multiple of 64: the last 64-k stage is zero-filled past K, so the outputs
     equal, bit for bit, those of operands zero-padded to whole stages (the same MFMA
-    chains, plus products of zeros). The weights' row padding holds NaN, and one row
-    of A does, whose outputs alone may be NaN."""
+    chains, plus products of zeros); for gate/up, the standalone activation of that
+    projection, whose sequence the fused epilogue runs at these K. The weights' row
+    padding holds NaN, and one row of A does, whose outputs alone may be NaN."""
     experts = len(counts)
     a, offsets, rows = _inputs(counts, alignment, k, seed=5 * k + n)
     used = int(to_np(offsets)[-1])
@@ -326,13 +328,46 @@ def test_partial_last_stage_equals_zero_padded(ext, counts, alignment, n, k):
     for width, run in ((n, ext.grouped_gemm_out), (2 * n, ext.gateup_swiglu_out)):
         w = (torch.randn(experts, width, k, device="cuda", generator=g) / k**0.5).bfloat16()
         got = torch.full((rows, n), 3.0, device="cuda").bfloat16()
-        want = got.clone()
         run(a, _row_padded(w, 72), offsets, got)
-        run(a_full, torch.nn.functional.pad(w, (0, full - k)).contiguous(), offsets, want)
+        want = torch.full((rows, width), 3.0, device="cuda").bfloat16()
+        ext.grouped_gemm_out(a_full, torch.nn.functional.pad(w, (0, full - k)).contiguous(), offsets, want)
+        if width != n:
+            projection, want = want, torch.empty_like(got)
+            ext.swiglu_out(projection, offsets[-1:], want)
+            want[used:] = 3.0
         nan_rows = torch.isnan(got.float()).any(dim=1).nonzero().flatten().tolist()
         assert nan_rows == [used // 2]
         keep = torch.arange(rows, device="cuda") != used // 2
         assert torch.equal(got[keep], want[keep])
+
+
+@pytest.mark.parametrize("counts,k", [
+    ([3, 0, 5], 72),            # weight-streaming kernel, 64-row instance
+    ([90, 20], 200),            # 128-row instance
+    ([700, 40, 300], 136),      # persistent kernel
+    ([5] * 40, 8),              # persistent kernel, column pieces
+])
+def test_partial_stage_activation_over_the_whole_range(ext, counts, k):
+    """K not a multiple of 64: the fused epilogue gives the oracle's SwiGLU bit for bit
+    also where g * u overflows or exp(-g) does. One column of A is 1 and the others 0,
+    so the projections are the weights' first column exactly."""
+    inter = 136
+    offsets = torch.tensor(_offsets(counts, 8), device="cuda")
+    rows = int(offsets[-1])
+    a = torch.zeros(rows, k, device="cuda", dtype=torch.bfloat16)
+    a[:, 0] = 1
+    rng = np.random.default_rng(k)
+    values = rng.choice([-1e30, 1e30, -3e38, 3e38, 1e37, -1e-30, 0.0], (len(counts), 2, inter))
+    drawn = rng.standard_normal(values.shape) * 10.0 ** rng.uniform(-3, 2.3, values.shape)
+    values = np.where(rng.random(values.shape) < 0.5, values, drawn)
+    w = torch.zeros(len(counts), 2 * inter, k, device="cuda", dtype=torch.bfloat16)
+    w[:, :, 0] = torch.tensor(values.reshape(len(counts), -1), device="cuda").bfloat16()
+    got = torch.empty(rows, inter, device="cuda", dtype=torch.bfloat16)
+    ext.gateup_swiglu_out(a, w, offsets, got)
+    projection = np.repeat(to_np(w[:, :, 0]), np.diff(to_np(offsets)), axis=0)
+    want = torch.from_numpy(oracle.swiglu(projection, rows)).bfloat16()
+    assert torch.isnan(want).sum() == 0
+    np.testing.assert_array_equal(raw_bits(got), raw_bits(want))
 
 
 GATEUP_PIECES_CASES = [
