@@ -128,6 +128,9 @@ class LayerWorkspace:
     projection: torch.Tensor
     activated: torch.Tensor
     expert_output: torch.Tensor
+    # moe_route_rows' plane sums, where the shape needs any: a captured graph holds their
+    # address, so like every buffer here they live as long as the block.
+    plane_sums: torch.Tensor | None = None
 
 
 class MoEBlock(torch.nn.Module):
@@ -285,12 +288,15 @@ class MoEBlock(torch.nn.Module):
                 )
             rows = transport.capacity_rows
             # The fused gate/up kernel never materialises the [R, 2I] projection.
-            proj_rows = 0 if self.implementation == "cuda_fused" else rows
+            fused = self.implementation == "cuda_fused"
+            proj_rows = 0 if fused else rows
+            sums_bytes = (_one_pass_bytes(self._extension.lib, x.shape[0], cfg) or 0) if fused else 0
             self._workspaces[key] = LayerWorkspace(
                 transport,
                 torch.empty((proj_rows, 2 * cfg.intermediate), device=x.device, dtype=x.dtype),
                 torch.empty((rows, cfg.intermediate), device=x.device, dtype=x.dtype),
                 torch.empty((rows, cfg.hidden), device=x.device, dtype=x.dtype),
+                torch.empty(sums_bytes, device=x.device, dtype=torch.uint8) if sums_bytes else None,
             )
         return self._workspaces[key]
 
@@ -343,7 +349,7 @@ class MoEBlock(torch.nn.Module):
         fused = self.implementation == "cuda_fused"
         # The fused router does the dispatch's counting pass when the shape allows.
         ranked = fused and state.transport.rank_tile > 0
-        gathered = fused and (_one_pass_bytes(self._extension.lib, x, self.config) is not None
+        gathered = fused and (_one_pass_bytes(self._extension.lib, x.shape[0], self.config) is not None
                               or _gathers(x, self.config.topk))
         ids32, ids64, weights = self._route(x, state.transport if ranked else None)
         transport = state.transport
@@ -368,9 +374,9 @@ class MoEBlock(torch.nn.Module):
         return state.transport.output
 
 
-def _can_gather(x):
-    """Whether the gate/up GEMM can read its rows from x (hidden a multiple of 64, x below 2 GiB)."""
-    return x.shape[1] % 64 == 0 and x.numel() * x.element_size() < 2**31
+def _can_gather(tokens, hidden):
+    """Whether the gate/up GEMM can read its rows from bf16 x (hidden a multiple of 64, x below 2 GiB)."""
+    return hidden % 64 == 0 and tokens * hidden * 2 < 2**31
 
 
 def _gathers(x, topk):
@@ -384,16 +390,16 @@ def _gathers(x, topk):
     that configuration's Zipf routing the gathered GEMM is itself faster than
     the packed one (560 against 638 us): it reads x's 33.6 MB where the packed
     kernel reads a 201 MB copy."""
-    return topk >= 3 and _can_gather(x)
+    return topk >= 3 and _can_gather(*x.shape)
 
 
-def _one_pass_bytes(lib, x, cfg):
+def _one_pass_bytes(lib, tokens, cfg):
     """Plane-sum bytes of the small-batch route that also writes the row table
     (``moe_route_rows``), or None where the shape has none. It replaces the router
     and the dispatch whatever top-k is: H=4096, E=8, top-2: 12.6 -> 6.6 us at one
     token, 13.8 -> 7.5 at 16; H=2048, E=64, top-6, 48 tokens: 33.6 -> 10.5 us."""
-    need = lib.moe_route_rows_scratch_bytes(x.shape[0], cfg.hidden, cfg.experts, cfg.topk)
-    return need if need >= 0 and _can_gather(x) else None
+    need = lib.moe_route_rows_scratch_bytes(tokens, cfg.hidden, cfg.experts, cfg.topk)
+    return need if need >= 0 and _can_gather(tokens, cfg.hidden) else None
 
 
 class _FusedLaunches:
@@ -433,7 +439,7 @@ class _FusedLaunches:
         # has one, and the row table instead of the packed copy whenever the
         # gate/up GEMM gathers, as in forward().
         self.ranked = t.rank_tile > 0
-        sums_bytes = _one_pass_bytes(self.lib, x, cfg)
+        sums_bytes = _one_pass_bytes(self.lib, tokens, cfg)
         self.gathered = sums_bytes is not None or _gathers(x, cfg.topk)
         # The weights' row strides (contiguous, or gate/up rows padded); anything
         # else was refused by the validating forward that built these launches.
@@ -441,10 +447,6 @@ class _FusedLaunches:
         down_stride = weight_row_stride(block.down_weight)
         if gate_up_stride is None or down_stride is None:
             raise RuntimeError("expert weights must be contiguous or row-padded")
-        # Small batches: routing and the row-table dispatch in one pass (every
-        # output as the two calls write it), its plane sums owned by these launches.
-        if sums_bytes is not None:
-            self.sums = torch.empty(max(sums_bytes, 4), dtype=torch.uint8, device=x.device)
         index = (ids32.data_ptr(), t.counts.data_ptr(), t.offsets.data_ptr(), t.slots.data_ptr())
         if self.ranked:
             self.router += (t.tile_ranks.data_ptr(), t.tile_counts.data_ptr(), t.tile_counts.numel() * 4)
@@ -485,7 +487,7 @@ class _FusedLaunches:
             struct_bytes=ctypes.sizeof(_lib.BlockArgs), router_scratch_bytes=scratch.numel() * scratch.element_size(),
             dispatch_scratch_bytes=t.scratch.numel() * t.scratch.element_size(),
             tile_counts_bytes=t.tile_counts.numel() * 4, tile_tokens=t.rank_tile,
-            sums_bytes=self.sums.numel() if sums_bytes is not None else 0, gate_up_row_stride=gate_up_stride,
+            sums_bytes=0 if state.plane_sums is None else state.plane_sums.numel(), gate_up_row_stride=gate_up_stride,
             down_row_stride=down_stride, tokens=tokens, hidden=hidden, intermediate=cfg.intermediate,
             experts=cfg.experts, topk=cfg.topk, alignment=t.alignment, packed_rows=rows,
             vectorized=int(bool(t.vectorized)), gathered=int(self.gathered), one_pass=int(sums_bytes is not None))
@@ -494,7 +496,7 @@ class _FusedLaunches:
                 ("router_scratch", scratch), ("counts", t.counts), ("offsets", t.offsets), ("slots", t.slots),
                 ("inverse", t.inverse), ("row_src", t.row_src), ("packed", t.packed), ("dispatch_scratch", t.scratch),
                 ("ranks", t.tile_ranks), ("tile_counts", t.tile_counts),
-                ("sums", self.sums if sums_bytes is not None else None), ("gate_up", block.gate_up_weight),
+                ("sums", state.plane_sums), ("gate_up", block.gate_up_weight),
                 ("down", block.down_weight), ("activated", state.activated), ("expert_output", state.expert_output),
                 ("output", t.output)):
             setattr(args, name, None if tensor is None else tensor.data_ptr())

@@ -112,3 +112,31 @@ def test_forward_graph_replays_skip_the_split_until_the_weights_change():
     finally:
         block._extension.router_split_out = real
     torch.cuda.synchronize()
+
+
+def test_plane_sums_of_a_captured_forward_outlive_its_launches():
+    """E > 16 at few tokens: the one-pass route's plane sums keep their address when a
+    replaced router weight rebuilds the launches, so an earlier graph, which recorded
+    that address, writes to memory the block still owns."""
+    cfg = MoEConfig(512, 256, 64, 6)
+    block = MoEBlock(cfg, device="cuda", implementation="cuda_fused", seed=0)
+    twin = MoEBlock(cfg, device="cuda", implementation="cuda_fused", seed=0)
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn(48, cfg.hidden, device="cuda", generator=gen).bfloat16()
+    graph = capture_forward(block, x)
+    before = block._launches[(48, x.device)]
+    assert before.args.one_pass == 1 and before.args.sums and before.args.sums_bytes == 48 * 3 * 64 * 4
+    new_w = torch.randn(cfg.experts, cfg.hidden, device="cuda", generator=gen) / cfg.hidden**0.5
+    block.router_weight = new_w
+    block(x)
+    after = block._launches[(48, x.device)]
+    assert after is not before and after.args.sums == before.args.sums
+    del before
+    twin.router_weight = new_w.clone()
+    expected = twin(x).clone()
+    for _ in range(3):
+        with torch.inference_mode():
+            graph.output.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(graph.output, expected)
