@@ -79,18 +79,17 @@ def make_weights(config, device, dtype, seed=42):
     return MoEWeights(router, gate_up, down)
 
 
-# Elements of padding after each expert weight row whose length is a multiple of
-# WEIGHT_ROW_CONFLICT bytes, for the fused block. The GEMMs read every row of a
-# tile, on every CU, at the same k offset at once, and rows a multiple of 4 KiB
-# apart then fall on the same memory channels. Measured, padded against
-# contiguous rows: gate/up at H=2048, I=4096, 16 experts, 128 rows 121.6 -> 93.0
-# us (4.4 -> 5.8 TB/s) and at H=2048, I=1408, 64 experts, 288 rows 139.2 -> 125.2;
-# at H=4096, I=14336, 8 experts, 2 rows 90.0 -> 80.3 and 32 rows 338 -> 302; down
-# at I=14336 (7 x 4 KiB) with 32 rows 182 -> 158 and 666 rows 217 -> 206. Full
-# prefill is unchanged (4096 tokens at H=4096: 1447 and 1441 us). Rows of 2 KiB
-# multiples gained 1-8% at H=1024 with few rows and nothing with many, and stay
-# contiguous; so do rows of other lengths. The results are the same bit for bit
-# (each output is the same MFMA chain).
+# Elements of padding after each row of a row-padded expert weight. The GEMMs read
+# every row of a tile, on every CU, at the same k offset at once, and rows a
+# multiple of WEIGHT_ROW_CONFLICT bytes apart then fall on the same memory
+# channels. Measured, padded against contiguous rows: gate/up at H=2048, I=4096,
+# 16 experts, 128 rows 121.6 -> 93.0 us (4.4 -> 5.8 TB/s) and at H=2048, I=1408, 64
+# experts, 288 rows 139.2 -> 125.2; at H=4096, I=14336, 8 experts, 2 rows 90.0 ->
+# 80.3 and 32 rows 338 -> 302; down at I=14336 (7 x 4 KiB) with 32 rows 182 -> 158
+# and 666 rows 217 -> 206. Full prefill is unchanged (4096 tokens at H=4096: 1447
+# and 1441 us). Rows of 2 KiB multiples gained 1-8% at H=1024 with few rows and
+# nothing with many; rows of other lengths do not conflict. The results are the
+# same bit for bit (each output is the same MFMA chain).
 GATE_UP_ROW_PADDING = 64
 WEIGHT_ROW_CONFLICT = 4096
 
@@ -103,8 +102,10 @@ def _row_padded(weight):
 
 
 def padded_gate_up(weight):
-    """``weight`` ([E, 2I, H]) as a ``[:, :, :H]`` view of row-padded storage when
-    its rows are a power of two bytes of at least 8 KiB long, else contiguous."""
+    """``weight`` ([E, 2I, H]) as a ``[:, :, :H]`` view of row-padded storage when its
+    rows are a power of two bytes of at least 8 KiB, else contiguous: the layout the
+    fused block gives its gate/up weights. Every other weight keeps the storage it
+    was given, which its owner may share between blocks or update in place."""
     row_bytes = weight.shape[2] * weight.element_size()
     if row_bytes < 8192 or row_bytes & (row_bytes - 1):
         return weight.contiguous()
@@ -114,7 +115,9 @@ def padded_gate_up(weight):
 def padded_weight(weight):
     """``weight`` ([E, N, K]) as a ``[:, :, :K]`` view of row-padded storage when its
     rows are a multiple of WEIGHT_ROW_CONFLICT bytes and one expert stays below the
-    GEMMs' 4 GiB with the padding, else contiguous."""
+    GEMMs' 4 GiB with the padding, else contiguous. For a program that has no other
+    use of the tensor: ``block.down_weight = padded_weight(block.down_weight)`` (and
+    ``gate_up_weight``) moves a fused block's weights to storage of their own."""
     _, n, k = weight.shape
     size = weight.element_size()
     if k * size % WEIGHT_ROW_CONFLICT or n * (k + GATE_UP_ROW_PADDING) * size >= 2**32:
@@ -173,11 +176,11 @@ class MoEBlock(torch.nn.Module):
         if weights.router.shape != (cfg.experts, cfg.hidden):
             raise ValueError("router weights do not match the block configuration")
         self.register_buffer("router_weight", weights.router.contiguous())
-        # The fused block keeps conflicting weight rows padded (WEIGHT_ROW_CONFLICT); its
-        # tensors are views of that storage, so in-place updates of them reach the kernels.
-        laid_out = padded_weight if implementation == "cuda_fused" else torch.Tensor.contiguous
-        self.register_buffer("gate_up_weight", laid_out(weights.gate_up))
-        self.register_buffer("down_weight", laid_out(weights.down))
+        # The fused block pads power-of-two gate/up rows (padded_gate_up); the tensor is a
+        # view of that storage, so in-place updates of it reach the kernels.
+        gate_up = padded_gate_up(weights.gate_up) if implementation == "cuda_fused" else weights.gate_up.contiguous()
+        self.register_buffer("gate_up_weight", gate_up)
+        self.register_buffer("down_weight", weights.down.contiguous())
         self.register_buffer("routing_bias", torch.zeros(cfg.experts, device=device))
         self._workspaces = {}
         self._route_buffers = {}

@@ -107,7 +107,7 @@ def test_fused_block_pads_power_of_two_gate_up_rows():
     assert padded_gate_up(torch.zeros(1, 2, 2048)).stride(1) == 2048 + GATE_UP_ROW_PADDING
 
 
-def test_fused_block_pads_weight_rows_that_conflict():
+def test_padded_weight_pads_rows_that_conflict():
     from moe_dispatch._extension import weight_row_stride
     from moe_dispatch.layer import GATE_UP_ROW_PADDING, padded_weight
 

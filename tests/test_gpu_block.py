@@ -28,7 +28,7 @@ import numpy as np
 import pytest
 import torch
 
-from moe_dispatch.layer import GATE_UP_ROW_PADDING, MoEBlock, MoEConfig
+from moe_dispatch.layer import GATE_UP_ROW_PADDING, MoEBlock, MoEConfig, make_weights, padded_weight
 from oracle import moe_oracle as oracle
 from tests._helpers import LazyExpertWeights, assert_near_bit_exact, gpu, rel_l2, route_margin, to_np
 
@@ -308,11 +308,13 @@ def test_padded_gate_up_rows_equal_contiguous_weights(cfg):
 
 @pytest.mark.parametrize("cfg", [MoEConfig(2048, 256, 8, 2), MoEConfig(128, 4096, 8, 2), MoEConfig(2048, 2048, 16, 6)])
 def test_padded_weight_rows_equal_contiguous_weights(cfg):
-    """Gate/up or down rows of a multiple of 4 KiB are kept padded: the forward equals that
-    of a twin with contiguous copies, bit for bit, and in-place updates reach the kernels."""
+    """Gate/up or down rows of a multiple of 4 KiB moved to row-padded storage: the forward
+    equals that of a twin with contiguous copies, bit for bit, and in-place updates reach
+    the kernels."""
     block = MoEBlock(cfg, device="cuda", implementation="cuda_fused", seed=3)
     twin = MoEBlock(cfg, device="cuda", implementation="cuda_fused", seed=3)
     for name, k in (("gate_up_weight", cfg.hidden), ("down_weight", cfg.intermediate)):
+        setattr(block, name, padded_weight(getattr(block, name)))
         assert getattr(block, name).stride(1) == (k + GATE_UP_ROW_PADDING if k % 2048 == 0 else k)
         setattr(twin, name, getattr(block, name).contiguous())
     gen = torch.Generator(device="cuda").manual_seed(5)
@@ -324,6 +326,31 @@ def test_padded_weight_rows_equal_contiguous_weights(cfg):
     twin.down_weight.copy_(new)
     x = torch.randn(300, cfg.hidden, device="cuda", generator=gen).bfloat16()
     assert torch.equal(block(x).clone(), twin(x))
+
+
+@pytest.mark.parametrize("cfg", [MoEConfig(2048, 256, 8, 2), MoEConfig(4096, 2048, 8, 2), MoEConfig(6144, 512, 4, 1)])
+def test_given_weights_are_shared(cfg):
+    """A fused block keeps the storage of the weights it is given (gate/up rows of a power
+    of two bytes of at least 8 KiB aside, which it pads): no second copy, and the owner's
+    in-place updates reach the kernels, also between blocks that share them."""
+    weights = make_weights(cfg, "cuda", torch.bfloat16, 3)
+    blocks = [MoEBlock(cfg, device="cuda", implementation="cuda_fused", weights=weights) for _ in range(2)]
+    shared = ["router", "down"] + (["gate_up"] if cfg.hidden != 4096 else [])
+    for block in blocks:
+        for name in shared:
+            tensor = getattr(block, name + "_weight")
+            assert tensor.data_ptr() == getattr(weights, name).data_ptr() and tensor.is_contiguous(), name
+    x = torch.randn(20, cfg.hidden, device="cuda").bfloat16()
+    first = [block(x).clone() for block in blocks]
+    for name in shared[1:]:
+        getattr(weights, name).mul_(-0.5)
+    twin = MoEBlock(cfg, device="cuda", implementation="cuda_fused", weights=weights)
+    if "gate_up" not in shared:
+        twin.gate_up_weight = blocks[0].gate_up_weight
+    want = twin(x).clone()
+    assert not torch.equal(want, first[0])
+    for block in blocks:
+        assert torch.equal(block(x), want)
 
 
 def test_native_forward_follows_replaced_parameters():
