@@ -687,6 +687,14 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, char* lds, int ex
 // rows 115 -> 104; H=512, I=1024, 8192 rows 28 -> 25. Halves of its short tiles
 // after rounds of full ones lose, though (H=1024, I=2048, 16 experts, 8192 rows: in
 // the forward 82 -> 85 us; they are HBM-bound whole, and a half reads A again).
+// Short tiles alone (no full ones) gain as halves after whole rounds of theirs too,
+// but weight rows a multiple of kConflictBytes apart fall on the same memory
+// channels, and more CUs reading them can lose once the last round is nearly half
+// full: H=2048, I=1408, 64 experts, two rounds and 82 / 93 / 115 / 126 tiles 132 ->
+// 129, 131 -> 131, 135 -> 140, 136 -> 143 us whole -> halves (121 -> 116 with padded
+// rows); H=4096, I=1536, 32 experts, one round and 128 163 -> 169 (145 -> 135
+// padded). Others gain 2-3% (H=2048, I=768 or 1024, one round and 128), and where
+// the weights lie moves such rows by as much. They are split up to 3/8 of the slots.
 //
 // For the plain GEMM, when phase 1 fills at most half of the slots of one round
 // beside a phase 2, its tiles run as halves (the two halves of a tile in
@@ -696,6 +704,8 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, char* lds, int ex
 // more of the plan live through the k-loop and spilled: H=4096, I=14336, 4096
 // tokens 1460 -> 1587 us.) Every tile or piece runs its whole k chain in order on one
 // workgroup, so results do not depend on the schedule or on G.
+constexpr int64_t kConflictBytes = 4096;
+
 struct RingPhase {
     int count;   // tiles
     int main;    // tiles mapped XCD-contiguously
@@ -706,12 +716,13 @@ struct RingPhase {
 
 // Short tiles (phase 2) split four ways when that still fits the slots: their
 // cost is streaming the weight slab, which more CUs pull faster.
-__device__ __forceinline__ RingPhase ring_phase(int count, int grid, bool pieces, bool short_tiles, bool halves) {
+// `halves`: the most tiles of a last round that split in two.
+__device__ __forceinline__ RingPhase ring_phase(int count, int grid, bool pieces, bool short_tiles, int halves) {
     RingPhase ph;
     ph.count = count;
     const int rem = count % grid;
     const bool quarters = short_tiles && 4 * rem <= grid;
-    const bool split = pieces && rem > 0 && (quarters || (halves && 2 * rem <= grid));
+    const bool split = pieces && rem > 0 && (quarters || rem <= halves);
     ph.ways = quarters ? 4 : 2;
     ph.main = split ? count - rem : count;
     ph.blocks = (ph.main + kNumXcd - 1) / kNumXcd * kNumXcd;
@@ -736,7 +747,7 @@ struct RingPlan {
 };
 
 // grid is a positive multiple of 8.
-__device__ __forceinline__ RingPlan ring_plan(int n1, int n2, int grid, bool swiglu, bool pieces) {
+__device__ __forceinline__ RingPlan ring_plan(int n1, int n2, int grid, bool swiglu, bool pieces, bool conflict) {
     RingPlan pl{};
     pl.n1 = n1;
     pl.n2 = n2;
@@ -753,7 +764,14 @@ __device__ __forceinline__ RingPlan ring_plan(int n1, int n2, int grid, bool swi
         pl.slots = rounds * grid - kNumXcd * pl.per1;
         pl.carried = min(n2, 2 * pl.slots);
     }
-    pl.rest = ring_phase(n2 > 0 ? n2 - pl.carried : n1, grid, pieces, n2 > 0, !swiglu || n1 == 0 || n2 == 0);
+    int halves = grid / 2;
+    if (swiglu && n2 > 0) {
+        if (n1 > 0)
+            halves = 0;
+        else if (conflict && n2 > grid)
+            halves = 3 * grid / 8;
+    }
+    pl.rest = ring_phase(n2 > 0 ? n2 - pl.carried : n1, grid, pieces, n2 > 0, halves);
     pl.virtual_blocks = pl.rounds * grid + pl.rest.blocks + pl.rest.pieces;
     return pl;
 }
@@ -1064,7 +1082,8 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_persistent_kernel(G
     // as column pieces on every CU (781 -> 800 us at H=4096, I=14336).
     const RingTable table = ring_table(p, SWIGLU && p.k >= 2048);
     const int grid = static_cast<int>(gridDim.x);
-    const RingPlan plan = ring_plan(table.n_full, table.n_part, grid, SWIGLU, PIECES);
+    const RingPlan plan =
+        ring_plan(table.n_full, table.n_part, grid, SWIGLU, PIECES, p.ldb * 2 % kConflictBytes == 0);
     // The next tile of this workgroup at or after tile `sub` of virtual workgroup q.
     auto next = [&](int& q, int& sub) {
         RingWork w{false, 0, 0, 0, 0, 0};

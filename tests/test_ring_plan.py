@@ -1,13 +1,14 @@
 """The persistent grouped GEMM's tile plan, restated and checked on the CPU.
 
-grouped_gemm_persistent_kernel (cuda-moe-engine_amd/csrc/gemm.hip: ring_plan,
+grouped_gemm_persistent_kernel (cuda-moe-engine_amd/csrc/gemm_ring.h: ring_plan,
 ring_slot) walks virtual workgroups q = blockIdx.x + i*G in rounds of G. Full
 row tiles (phase 1) run in 8 XCD-contiguous ranges, cpr per XCD and round;
 the other slots of the rounds carry one or two of the experts' short last row
 tiles (phase 2); phase-2 tiles the rounds do not take, or phase 1 when there is
 no phase 2, run after the rounds with an optional split of a short last round
-into 128-column pieces (plain GEMM only); a phase 1 that fills at most half of
-one round beside a phase 2 runs in the rounds as 128-column halves (plain GEMM
+into column halves or quarters (the plain GEMM, and the gate/up kernel that
+splits tiles); a phase 1 that fills at most half of
+one round beside a phase 2 runs in the rounds as column halves (plain GEMM
 only). The gate/up GEMM at K >= 2048 cuts each expert of more than 128 rows
 into ceil(rows/256) balanced row tiles, all in phase 1. This restates those
 formulas and checks that every tile (or both halves of a split tile) is
@@ -46,18 +47,19 @@ def balanced_for(swiglu, k):
     return swiglu and k >= 2048
 
 
-def ring_phase(count, grid, allow_split, short_tiles=False, halves=True):
+def ring_phase(count, grid, allow_split, short_tiles, halves):
     rem = count % grid
     ways = 4 if short_tiles and 4 * rem <= grid else 2
-    split = allow_split and rem > 0 and (ways == 4 or (halves and 2 * rem <= grid))
+    split = allow_split and rem > 0 and (ways == 4 or rem <= halves)
     main = count - rem if split else count
     return {"main": main, "blocks": (main + XCD - 1) // XCD * XCD, "pieces": ways * rem if split else 0,
             "ways": ways}
 
 
-def ring_plan(n1, n2, grid, allow_split, gateup_pieces=False):
+def ring_plan(n1, n2, grid, allow_split, gateup_pieces=False, conflict=False):
     """The plan of the plain GEMM (allow_split), of the gate/up kernel without pieces
-    (not allow_split), or with gateup_pieces of the gate/up kernel that splits tiles."""
+    (not allow_split), or with gateup_pieces of the gate/up kernel that splits tiles
+    (conflict: its weight rows are a multiple of 4 KiB apart)."""
     half1 = allow_split and not gateup_pieces and n2 > 0 and n1 > 0 and 2 * n1 <= grid
     pl = {"n1": n1, "n2": n2, "half1": half1, "u1": 2 * n1 if half1 else n1, "per1": 0, "cpr": 0, "rounds": 0,
           "full_rounds": 0, "last_cols": 0, "slots": 0, "carried": 0}
@@ -70,8 +72,10 @@ def ring_plan(n1, n2, grid, allow_split, gateup_pieces=False):
         slots = rounds * grid - XCD * per1
         pl.update(per1=per1, rounds=rounds, cpr=cpr, full_rounds=per1 // cpr,
                   last_cols=per1 - (per1 // cpr) * cpr, slots=slots, carried=min(n2, 2 * slots))
-    pl["rest"] = ring_phase(n2 - pl["carried"] if n2 > 0 else n1, grid, allow_split, n2 > 0,
-                            not gateup_pieces or n1 == 0 or n2 == 0)
+    halves = grid // 2
+    if gateup_pieces and n2 > 0:
+        halves = 0 if n1 > 0 else 3 * grid // 8 if conflict and n2 > grid else halves
+    pl["rest"] = ring_phase(n2 - pl["carried"] if n2 > 0 else n1, grid, allow_split, n2 > 0, halves)
     pl["virtual_blocks"] = pl["rounds"] * grid + pl["rest"]["blocks"] + pl["rest"]["pieces"]
     return pl
 
@@ -114,9 +118,9 @@ def ring_slot(pl, grid, q, sub):
     return None
 
 
-def walk(n1, n2, grid, allow_split, gateup_pieces=False):
+def walk(n1, n2, grid, allow_split, gateup_pieces=False, conflict=False):
     """Per workgroup, the (phase, tile, piece) sequence it runs."""
-    pl = ring_plan(n1, n2, grid, allow_split, gateup_pieces)
+    pl = ring_plan(n1, n2, grid, allow_split, gateup_pieces, conflict)
     runs = []
     for wg in range(grid):
         seq = []
@@ -129,8 +133,8 @@ def walk(n1, n2, grid, allow_split, gateup_pieces=False):
     return pl, runs
 
 
-def check_cover(n1, n2, grid, allow_split, gateup_pieces=False):
-    pl, runs = walk(n1, n2, grid, allow_split, gateup_pieces)
+def check_cover(n1, n2, grid, allow_split, gateup_pieces=False, conflict=False):
+    pl, runs = walk(n1, n2, grid, allow_split, gateup_pieces, conflict)
     seen = {}
     for seq in runs:
         for _, (phase, tile, piece) in seq:
@@ -288,12 +292,19 @@ def test_gateup_pieces_plans():
     rng = random.Random(11)
     for _ in range(200):
         grid = 8 * rng.randint(1, 32)
-        check_cover(rng.choice([0, rng.randint(0, 900)]), rng.choice([0, rng.randint(0, 900)]), grid, True, True)
+        check_cover(rng.choice([0, rng.randint(0, 900)]), rng.choice([0, rng.randint(0, 900)]), grid, True, True,
+                    rng.random() < 0.5)
     # H=4096, I=14336, 8 experts of at most 128 rows: three rounds and 256 halves.
     pl, _ = check_cover(0, 8 * 112, 256, True, True)
     assert (pl["rest"]["main"], pl["rest"]["pieces"], pl["rest"]["ways"]) == (768, 256, 2)
     # H=2048, I=1408: six active experts as 132 halves, 51 as two rounds and 196 quarters.
     assert check_cover(0, 66, 256, True, True)[0]["rest"]["pieces"] == 132
     assert check_cover(0, 561, 256, True, True)[0]["rest"]["pieces"] == 196
+    # Rows a multiple of 4 KiB apart: 57 and 58 experts (115 and 126 tiles after two
+    # rounds) stay whole, 54 (82 tiles) split, and so do 66 tiles without a full round.
+    for active, pieces in ((57, 0), (58, 0), (54, 164), (6, 132), (51, 196)):
+        assert check_cover(0, 11 * active, 256, True, True, conflict=True)[0]["rest"]["pieces"] == pieces
+        if active in (57, 58):
+            assert check_cover(0, 11 * active, 256, True, True)[0]["rest"]["pieces"] == 2 * (11 * active - 512)
     # H=1024, I=2048, 8192 rows: 128 short tiles after full rounds stay whole.
     assert check_cover(512, 128, 256, True, True)[0]["rest"]["pieces"] == 0
