@@ -925,9 +925,12 @@ __device__ __forceinline__ void write_rows_layout(const int* ids, int n, int exp
 // and the pack kernel took 12.6 and 13.8. Two or more token tiles in the block
 // lost to one block each and a separate row-table dispatch (17 tokens: 10.0
 // against 9.7 us; 128 tokens of 512: 8.8 against 7.9).
+// Steps of loads in flight: 1024 threads leave 128 VGPRs a lane, which three
+// steps of five fragments overrun (33 spilled: H=8192, E=12, 16 tokens routed in
+// 18.0 us, 11.3 with two steps).
 template <int F>
-constexpr int small_depth() {  // 1024 threads leave 128 VGPRs a lane
-    return 22 / (2 + F);
+constexpr int small_depth() {
+    return F == 5 ? 2 : 22 / (2 + F);
 }
 
 template <int PER, int F>
