@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256) void topk_route_kernel(const float* __restrict
 
 constexpr int kRouterTokens = 16;
 constexpr int64_t kRankedPrefixMax = 4096;  // routing tiles x experts of a ranked route
-constexpr int kRouterSplitTokens = 64;  // split-k routing up to this many tokens (E <= 16, hidden past the direct kernel's)
+constexpr int kRouterSplitTokens = 64;  // split-k routing up to this many tokens (E <= 16, large hidden)
 constexpr int kRouterSplitSlices = 16;
 constexpr int kRouterSplitTiles = kRouterSplitTokens / kRouterTokens;
 constexpr int64_t kRouterPartialBytes =
@@ -318,8 +318,8 @@ struct RouterShape {
 // b / slices and the k-slice b % slices of `per` stages, loads the whole slice
 // into its ring at once and writes the slice's partial logits to
 // partials[tile][slice][TB][EB]; router_reduce_kernel adds the slices in
-// slice order and selects. Used past the hidden sizes of router_direct_kernel (one
-// token's planes are then 400 KB and more through one CU). (A last-block
+// slice order and selects. Used where a block of router_direct_kernel would move
+// 300 KB and more of planes through one CU (launch_router_fused). (A last-block
 // reduction inside this kernel needs a device-scope release per block, an L2
 // write-back that costs more than the second launch.)
 template <int NT, int MT, bool SPLIT = false>
@@ -1259,7 +1259,11 @@ int64_t router_rank_tile(int64_t tokens, int64_t experts) {
     return tile;
 }
 
-// Whether a batch routes in one block (route_small_kernel).
+// Whether a batch routes in one block (route_small_kernel). The router without the
+// row table takes it at the same sizes, so that both give the same bits; alone it is
+// 0.6-0.8 us slower than router_direct_kernel below 1024 hidden (E=8: 3.5 and 4.2 us)
+// and up to 3 us slower than split k at E > 8, H > 4096 (E=16, H=8192, 16 tokens 9.2 and
+// 12.1), which the saved dispatch gives back in a forward (7.7 and 5.9, 13.5 and 14.0).
 static bool small_route(int64_t tokens, int64_t hidden, int64_t experts) {
     return experts <= kDirectMaxExperts && tokens > 0 && tokens <= kRouterTokens && hidden <= 8192;
 }
@@ -1357,8 +1361,14 @@ int launch_router_fused(const uint16_t* x, const float* router_w, const float* b
     }
     const int k_stages = (hidden + 63) / 64;
     constexpr int kSplitMaxPer = RouterShape<1, 1>::STAGES;  // a slice fits the ring at once
-    if (experts <= 16 && tokens <= kRouterSplitTokens && k_stages > kDirectWaves * kDirectMaxPer &&
-        k_stages <= kRouterSplitSlices * kSplitMaxPer) {
+    // 17 to 64 tokens: split k past router_direct_kernel's hidden sizes, and with four
+    // or more weight fragments (E > 8) already from its last doubling on (H > 4096),
+    // where a block of it reads 0.3 MB and more. E=16: H=4096 9.0 us split, 8.1 direct;
+    // H=5120 9.4 and 12.6, H=8192 10.6 and 12.5; E=10: 8.3 and 6.6, 8.2 and 9.6, 9.5 and
+    // 9.9. E=8 (three fragments) 8.2 and 6.1, 8.4 and 8.8, 9.5 and 9.0.
+    const bool split = k_stages > kDirectWaves * kDirectMaxPer ||
+                       (k_stages > kDirectWaves * kDirectMaxPer / 2 && router_fragments(experts) > 3);
+    if (experts <= 16 && tokens <= kRouterSplitTokens && split && k_stages <= kRouterSplitSlices * kSplitMaxPer) {
         // Split k: slices of about 8 stages (64 KiB of loads per workgroup),
         // none empty.
         const int per = (k_stages + min(kRouterSplitSlices, (k_stages + 7) / 8) - 1) /

@@ -29,7 +29,7 @@ CASES = [
     # tokens, hidden, experts, topk, alignment
     (300, 512, 8, 2, 8),      # VGPR-load router, ragged last tile
     (1000, 1024, 16, 2, 1),   # VGPR-load router, E = 16
-    (40, 2048, 8, 2, 8),      # split-k router (T <= 64) and its selection kernel
+    (40, 2048, 8, 2, 8),      # VGPR-load router, a ragged last token tile
     (130, 8200, 8, 2, 1),     # LDS ring router, E <= 16
     (200, 256, 32, 4, 8),     # many-expert VGPR-load router, E = 32: 32-token tiles
     (100, 128, 64, 6, 1),     # many-expert VGPR-load router, E = 64

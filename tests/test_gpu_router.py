@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 import torch
 
+from moe_dispatch.workspace import CudaWorkspace
 from oracle import moe_oracle as oracle
 from tests._helpers import gpu, route_margin, to_np
 
@@ -68,9 +69,9 @@ def test_zero_logits_known_answer_and_empty_batch(ext):
     "tokens,hidden,experts,topk",
     [(1, 512, 8, 2), (33, 512, 8, 1), (257, 1024, 16, 2), (300, 2048, 64, 6), (64, 4096, 8, 2),
      (100, 136, 5, 3), (1000, 72, 32, 4), (8192, 2048, 64, 6),
-     # Split-k routing (tokens <= 64, E <= 16, 16..256 stages of 64 hidden):
-     # one token; a ragged last stage inside the last slice; the largest split
-     # (16 slices of 16 stages); one stage past it (the single-workgroup path).
+     # Up to 16 tokens, E <= 16: one workgroup (route_small_kernel). Split-k routing
+     # (17 to 64 tokens, and fewer past 8192 hidden): the largest split (16 slices of
+     # 16 stages); one stage past it (the single-workgroup path).
      (1, 4096, 8, 2), (16, 4096, 16, 6), (33, 2040, 12, 3), (50, 16384, 4, 2), (3, 16448, 8, 2),
      # E <= 16 past the split sizes: the VGPR-load kernel with 1 to 6 weight fragments
      # (E = 2, 3, 8, 10, 12, 16) and 2, 8 and 16 steps of 64 hidden per wave (ragged
@@ -114,8 +115,7 @@ def test_fused_router_matches_oracle(ext, tokens, hidden, experts, topk):
 def test_fused_router_ties_go_to_lower_expert(ext, experts, topk, tokens, hidden):
     """Zero activations make every logit exactly 0, so the selection is decided by a
     bias full of repeated values: the fused top-k must keep the lower expert id on
-    every tie, like the reference (``csrc/dispatch.cu:331-333``). 40 x 2048 with
-    E <= 16 takes the split-k path and its separate selection kernel."""
+    every tie, like the reference (``csrc/dispatch.cu:331-333``)."""
     x = torch.zeros(tokens, hidden, device="cuda", dtype=torch.bfloat16)
     w = torch.randn(experts, hidden, device="cuda") / hidden**0.5
     levels = torch.tensor([0.0, 1.0, 2.0, 0.5], device="cuda")
@@ -132,8 +132,7 @@ def test_fused_router_ties_go_to_lower_expert(ext, experts, topk, tokens, hidden
 @pytest.mark.parametrize("tokens,hidden", [(300, 512), (8, 4096)])
 def test_fused_router_reuses_a_held_split(ext, tokens, hidden):
     """router_weight=None routes with the split the scratch already holds: the same
-    logits, ids and weights as passing the weights again, on new tokens (8 x 4096:
-    the split-k path, whose partial logits follow the planes in the scratch)."""
+    logits, ids and weights as passing the weights again, on new tokens."""
     experts, topk = 16, 2
     gen = torch.Generator(device="cuda").manual_seed(5)
     w = torch.randn(experts, hidden, device="cuda", generator=gen) / hidden**0.5
@@ -155,3 +154,40 @@ def test_fused_router_reuses_a_held_split(ext, tokens, hidden):
     fresh = route(x, w)
     for a, b in zip(reused, fresh):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,topk,split", [
+    # From 17 tokens on; E > 8 from 4097 hidden, fewer experts past the direct kernel's 8192.
+    (17, 4104, 16, 4, True), (64, 8192, 9, 2, True), (33, 6152, 12, 3, True), (20, 8200, 4, 2, True),
+    (64, 4096, 16, 4, False), (64, 8192, 8, 2, False), (65, 8192, 16, 2, False), (16, 8192, 16, 8, False),
+])
+def test_split_k_routing_is_used_where_it_is_faster(ext, tokens, hidden, experts, topk, split):
+    """Split k leaves its slices' partial logits in the scratch, between the planes and
+    their copy in operand order; the other routers leave that part alone. Ids and weights
+    equal the oracle's selection from the kernel's own logits, ranked as well."""
+    gen = torch.Generator(device="cuda").manual_seed(tokens + hidden + experts)
+    x = torch.randn(tokens, hidden, device="cuda", generator=gen).bfloat16()
+    w = torch.randn(experts, hidden, device="cuda", generator=gen) / hidden**0.5
+    bias = torch.randn(experts, device="cuda", generator=gen) * 0.1
+    scratch = torch.full((ext.router_scratch_bytes(experts, hidden),), 0x5A, dtype=torch.uint8, device="cuda")
+    ids32 = torch.empty(tokens, topk, device="cuda", dtype=torch.int32)
+    ids64, weights = ids32.long(), torch.empty(tokens, topk, device="cuda")
+    logits = torch.empty(tokens, experts, device="cuda")
+    ext.router_fused_out(x, w, bias, ids32, ids64, weights, logits, scratch=scratch)
+    start = (6 * experts * hidden + 255) // 256 * 256
+    assert bool((scratch[start:start + 65536] != 0x5A).any()) == split
+    ref = oracle.router_logits(to_np(x), to_np(w))
+    scale = np.linalg.norm(to_np(x), axis=1)[:, None] * np.linalg.norm(to_np(w), axis=1)[None, :]
+    assert np.all(np.abs(to_np(logits) - ref) <= 1e-6 * scale + 1e-7)
+    ids_ref, w_ref, _ = oracle.topk_route(to_np(logits), to_np(bias), topk)
+    np.testing.assert_array_equal(to_np(ids32), ids_ref)
+    np.testing.assert_allclose(to_np(weights), w_ref, rtol=2e-6, atol=2e-6)
+    ws = CudaWorkspace(tokens, hidden, experts, topk, torch.bfloat16, extension=ext)
+    again = [torch.empty_like(t) for t in (ids32, ids64, weights)]
+    ext.router_fused_ranked_out(x, None, bias, *again, ws.tile_ranks, ws.tile_counts, scratch=scratch)
+    for a, b in zip(again, (ids32, ids64, weights)):
+        assert torch.equal(a, b)
+    ws.dispatch_ranked(x, ids32)
+    other = CudaWorkspace(tokens, hidden, experts, topk, torch.bfloat16, extension=ext)
+    other.dispatch(x, ids32)
+    assert torch.equal(ws.inverse, other.inverse) and torch.equal(ws.packed, other.packed)
