@@ -308,3 +308,37 @@ def test_gateup_pieces_plans():
             assert check_cover(0, 11 * active, 256, True, True)[0]["rest"]["pieces"] == 2 * (11 * active - 512)
     # H=1024, I=2048, 8192 rows: 128 short tiles after full rounds stay whole.
     assert check_cover(512, 128, 256, True, True)[0]["rest"]["pieces"] == 0
+
+
+def narrow_shift(shift, groups, n_out, a_rows, grid, one_round_stops=True):
+    """The plain weight-streaming GEMM's column width (log2) for `groups` row tiles."""
+    def tiles_of(s):
+        return groups * ((n_out + (1 << s) - 1) >> s)
+
+    tiles = tiles_of(shift)
+    if one_round_stops and tiles <= grid:
+        return shift
+    rounds = -(-tiles // grid)
+    while shift < 7 and (rounds > 1 or not one_round_stops):
+        wide_tiles = tiles_of(shift + 1)
+        wide_rounds = -(-wide_tiles // grid)
+        now, wide = rounds * (a_rows + (1 << shift)), wide_rounds * (a_rows + (2 << shift))
+        empty = 10 * tiles < 8 * rounds * grid
+        if not (10 * wide <= 7 * now or (empty and wide < now)):
+            break
+        tiles, rounds, shift = wide_tiles, wide_rounds, shift + 1
+    return shift
+
+
+def test_launches_of_one_round_keep_the_narrowest_columns():
+    """The width rule stops at one round of tiles, and before its divisions when the
+    narrowest tiles already fit one: the widths are those of the rule without the stop."""
+    rng = random.Random(5)
+    widened = 0
+    for _ in range(20000):
+        case = (rng.choice([5, 6]), rng.randint(1, 80), 8 * rng.randint(1, 2000), rng.choice([64, 128]),
+                rng.choice([1, 64, 255, 256, 304]))
+        width = narrow_shift(*case)
+        assert width == narrow_shift(*case, one_round_stops=False), case
+        widened += width > case[0]
+    assert widened > 1000
