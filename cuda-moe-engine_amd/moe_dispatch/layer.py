@@ -131,8 +131,9 @@ class LayerWorkspace:
     projection: torch.Tensor
     activated: torch.Tensor
     expert_output: torch.Tensor
-    # moe_route_rows' plane sums, where the shape needs any: a captured graph holds their
-    # address, so like every buffer here they live as long as the block.
+    one_pass: bool = False  # the fused forward routes through moe_route_rows
+    # Its plane sums, where the shape needs any: a captured graph holds their address,
+    # so like every buffer here they live as long as the block.
     plane_sums: torch.Tensor | None = None
 
 
@@ -293,12 +294,13 @@ class MoEBlock(torch.nn.Module):
             # The fused gate/up kernel never materialises the [R, 2I] projection.
             fused = self.implementation == "cuda_fused"
             proj_rows = 0 if fused else rows
-            sums_bytes = (_one_pass_bytes(self._extension.lib, x.shape[0], cfg) or 0) if fused else 0
+            sums_bytes = _one_pass_bytes(self._extension.lib, x.shape[0], cfg) if fused else None
             self._workspaces[key] = LayerWorkspace(
                 transport,
                 torch.empty((proj_rows, 2 * cfg.intermediate), device=x.device, dtype=x.dtype),
                 torch.empty((rows, cfg.intermediate), device=x.device, dtype=x.dtype),
                 torch.empty((rows, cfg.hidden), device=x.device, dtype=x.dtype),
+                sums_bytes is not None,
                 torch.empty(sums_bytes, device=x.device, dtype=torch.uint8) if sums_bytes else None,
             )
         return self._workspaces[key]
@@ -352,8 +354,7 @@ class MoEBlock(torch.nn.Module):
         fused = self.implementation == "cuda_fused"
         # The fused router does the dispatch's counting pass when the shape allows.
         ranked = fused and state.transport.rank_tile > 0
-        gathered = fused and (_one_pass_bytes(self._extension.lib, x.shape[0], self.config) is not None
-                              or _gathers(x, self.config.topk))
+        gathered = fused and (state.one_pass or _gathers(x, self.config.topk))
         ids32, ids64, weights = self._route(x, state.transport if ranked else None)
         transport = state.transport
         if gathered:
@@ -405,6 +406,9 @@ def _one_pass_bytes(lib, tokens, cfg):
     return need if need >= 0 and _can_gather(tokens, cfg.hidden) else None
 
 
+_BLOCK_ARGS_BYTES = ctypes.sizeof(_lib.BlockArgs)
+
+
 class _FusedLaunches:
     """The C-ABI calls of one validated cuda_fused forward, for reuse.
 
@@ -432,79 +436,41 @@ class _FusedLaunches:
         self.device_index = x.device.index if x.device.index is not None else torch.cuda.current_device()
         self.fingerprint = self._fingerprint(block)
         self.keep = (ids32, ids64, weights, t, state)  # the buffers below stay allocated
+        self.output = t.output
         tokens, hidden = x.shape
-        rows = t.packed.shape[0]
         scratch = block._router_scratch
-        self.router = (block.routing_bias.data_ptr(), ids32.data_ptr(), ids64.data_ptr(), weights.data_ptr(),
-                       None, scratch.data_ptr(), scratch.numel() * scratch.element_size(),
-                       tokens, hidden, cfg.experts, cfg.topk)
         # A ranked route (the router counts for the dispatch) whenever the shape
         # has one, and the row table instead of the packed copy whenever the
         # gate/up GEMM gathers, as in forward().
         self.ranked = t.rank_tile > 0
-        sums_bytes = _one_pass_bytes(self.lib, tokens, cfg)
-        self.gathered = sums_bytes is not None or _gathers(x, cfg.topk)
+        self.gathered = state.one_pass or _gathers(x, cfg.topk)
         # The weights' row strides (contiguous, or gate/up rows padded); anything
         # else was refused by the validating forward that built these launches.
         gate_up_stride = weight_row_stride(block.gate_up_weight)
         down_stride = weight_row_stride(block.down_weight)
         if gate_up_stride is None or down_stride is None:
             raise RuntimeError("expert weights must be contiguous or row-padded")
-        index = (ids32.data_ptr(), t.counts.data_ptr(), t.offsets.data_ptr(), t.slots.data_ptr())
-        if self.ranked:
-            self.router += (t.tile_ranks.data_ptr(), t.tile_counts.data_ptr(), t.tile_counts.numel() * 4)
-            ranked_table = (t.tile_ranks.data_ptr(), t.tile_counts.data_ptr(), t.tile_counts.numel() * 4, t.rank_tile)
-        if self.gathered:
-            after = (t.inverse.data_ptr(), t.row_src.data_ptr())
-            if self.ranked:
-                self.dispatch = index + after + ranked_table + (tokens, cfg.experts, cfg.topk, t.alignment, rows)
-            else:
-                self.dispatch = index + after + (t.scratch.data_ptr(), t.scratch.numel() * t.scratch.element_size(),
-                                                 tokens, cfg.experts, cfg.topk, t.alignment, rows)
-            # moe_grouped_gateup_swiglu_gathered_strided after x.
-            self.gateup = (t.row_src.data_ptr(), tokens, block.gate_up_weight.data_ptr(), gate_up_stride,
-                           state.activated.data_ptr(), t.offsets.data_ptr(), rows, hidden, cfg.intermediate,
-                           cfg.experts)
-        else:
-            packed = (t.packed.data_ptr(), t.inverse.data_ptr())
-            if self.ranked:
-                self.dispatch = (_lib.DTYPE_BF16,) + index + packed + ranked_table + (
-                    tokens, hidden, cfg.experts, cfg.topk, t.alignment, rows, int(bool(t.vectorized)))
-            else:
-                self.dispatch = (_lib.DTYPE_BF16,) + index + packed + (
-                    t.scratch.data_ptr(), t.scratch.numel() * t.scratch.element_size(), tokens, hidden, cfg.experts,
-                    cfg.topk, t.alignment, rows, int(bool(t.vectorized)))
-            self.gateup = (t.packed.data_ptr(), block.gate_up_weight.data_ptr(), gate_up_stride,
-                           state.activated.data_ptr(), t.offsets.data_ptr(), rows, hidden, cfg.intermediate,
-                           cfg.experts)
-        self.down = (state.activated.data_ptr(), block.down_weight.data_ptr(), down_stride,
-                     state.expert_output.data_ptr(), t.offsets.data_ptr(), rows, hidden, cfg.intermediate,
-                     cfg.experts)
-        self.combine = (state.expert_output.data_ptr(), _lib.DTYPE_BF16, t.inverse.data_ptr(), weights.data_ptr(),
-                        t.output.data_ptr(), tokens, hidden, cfg.topk, rows)
-        self.output = t.output
         if x.dtype != torch.bfloat16:
             raise RuntimeError("cuda_fused launches are bf16")
-        # The whole forward as one call (moe_block_forward).
-        args = _lib.BlockArgs(
-            struct_bytes=ctypes.sizeof(_lib.BlockArgs), router_scratch_bytes=scratch.numel() * scratch.element_size(),
-            dispatch_scratch_bytes=t.scratch.numel() * t.scratch.element_size(),
+        sums = state.plane_sums
+        # The whole forward as one call (moe_block_forward). Every new token count pays for
+        # this: one constructor call (a setattr per field takes three times as long).
+        self.args = _lib.BlockArgs(
+            struct_bytes=_BLOCK_ARGS_BYTES, bias=block.routing_bias.data_ptr(), ids32=ids32.data_ptr(),
+            ids64=ids64.data_ptr(), weights=weights.data_ptr(), router_scratch=scratch.data_ptr(),
+            router_scratch_bytes=scratch.numel(), counts=t.counts.data_ptr(), offsets=t.offsets.data_ptr(),
+            slots=t.slots.data_ptr(), inverse=t.inverse.data_ptr(), row_src=t.row_src.data_ptr(),
+            packed=t.packed.data_ptr(), dispatch_scratch=t.scratch.data_ptr(), dispatch_scratch_bytes=t.scratch.numel(),
+            ranks=t.tile_ranks.data_ptr(), tile_counts=t.tile_counts.data_ptr(),
             tile_counts_bytes=t.tile_counts.numel() * 4, tile_tokens=t.rank_tile,
-            sums_bytes=0 if state.plane_sums is None else state.plane_sums.numel(), gate_up_row_stride=gate_up_stride,
-            down_row_stride=down_stride, tokens=tokens, hidden=hidden, intermediate=cfg.intermediate,
-            experts=cfg.experts, topk=cfg.topk, alignment=t.alignment, packed_rows=rows,
-            vectorized=int(bool(t.vectorized)), gathered=int(self.gathered), one_pass=int(sums_bytes is not None))
-        for name, tensor in (
-                ("bias", block.routing_bias), ("ids32", ids32), ("ids64", ids64), ("weights", weights),
-                ("router_scratch", scratch), ("counts", t.counts), ("offsets", t.offsets), ("slots", t.slots),
-                ("inverse", t.inverse), ("row_src", t.row_src), ("packed", t.packed), ("dispatch_scratch", t.scratch),
-                ("ranks", t.tile_ranks), ("tile_counts", t.tile_counts),
-                ("sums", state.plane_sums), ("gate_up", block.gate_up_weight),
-                ("down", block.down_weight), ("activated", state.activated), ("expert_output", state.expert_output),
-                ("output", t.output)):
-            setattr(args, name, None if tensor is None else tensor.data_ptr())
-        self.args = args
-        self.args_address = ctypes.addressof(args)
+            sums=None if sums is None else sums.data_ptr(), sums_bytes=0 if sums is None else sums.numel(),
+            gate_up=block.gate_up_weight.data_ptr(), gate_up_row_stride=gate_up_stride,
+            down=block.down_weight.data_ptr(), down_row_stride=down_stride, activated=state.activated.data_ptr(),
+            expert_output=state.expert_output.data_ptr(), output=t.output.data_ptr(), tokens=tokens, hidden=hidden,
+            intermediate=cfg.intermediate, experts=cfg.experts, topk=cfg.topk, alignment=t.alignment,
+            packed_rows=t.capacity_rows, vectorized=bool(t.vectorized), gathered=self.gathered,
+            one_pass=state.one_pass)
+        self.args_address = ctypes.addressof(self.args)
 
     @classmethod
     def _fingerprint(cls, block):
@@ -543,22 +509,40 @@ class _FusedLaunches:
         """Each stage of __call__ as a zero-argument callable on the current
         stream (the router with the split it holds), for per-stage timing. A
         small batch's one-pass route is timed as its two stages' own calls."""
-        lib, x_ptr = self.lib, x.data_ptr()
+        lib, a, x_ptr = self.lib, self.args, x.data_ptr()
 
         def bind(name, *args):
             def run():
                 lib.check(getattr(lib, name)(*args, current_stream_handle(self.device_index)), name)
             return run
 
-        router = "moe_router_fused_ranked" if self.ranked else "moe_router_fused"
-        if self.gathered:
-            dispatch = bind("moe_dispatch_ranked_rows" if self.ranked else "moe_dispatch_rows", *self.dispatch)
-            gateup = bind("moe_grouped_gateup_swiglu_gathered_strided", x_ptr, *self.gateup)
+        router = (x_ptr, None, a.bias, a.ids32, a.ids64, a.weights, None, a.router_scratch, a.router_scratch_bytes,
+                  a.tokens, a.hidden, a.experts, a.topk)
+        index = (a.ids32, a.counts, a.offsets, a.slots)
+        table = (a.ranks, a.tile_counts, a.tile_counts_bytes, a.tile_tokens)
+        counted = (a.dispatch_scratch, a.dispatch_scratch_bytes)
+        layout = (a.experts, a.topk, a.alignment, a.packed_rows)
+        if self.ranked:
+            router = bind("moe_router_fused_ranked", *router, a.ranks, a.tile_counts, a.tile_counts_bytes)
         else:
-            dispatch = bind("moe_dispatch_ranked" if self.ranked else "moe_dispatch", x_ptr, *self.dispatch)
-            gateup = bind("moe_grouped_gateup_swiglu_strided", *self.gateup)
-        return {"router": bind(router, x_ptr, None, *self.router), "dispatch": dispatch, "gateup_swiglu": gateup,
-                "down": bind("moe_grouped_gemm_strided", *self.down), "combine": bind("moe_combine", *self.combine)}
+            router = bind("moe_router_fused", *router)
+        if self.gathered:
+            rows = index + (a.inverse, a.row_src) + (table if self.ranked else counted)
+            dispatch = bind("moe_dispatch_ranked_rows" if self.ranked else "moe_dispatch_rows", *rows, a.tokens, *layout)
+            gateup = bind("moe_grouped_gateup_swiglu_gathered_strided", x_ptr, a.row_src, a.tokens, a.gate_up,
+                          a.gate_up_row_stride, a.activated, a.offsets, a.packed_rows, a.hidden, a.intermediate,
+                          a.experts)
+        else:
+            rows = index + (a.packed, a.inverse) + (table if self.ranked else counted)
+            dispatch = bind("moe_dispatch_ranked" if self.ranked else "moe_dispatch", x_ptr, _lib.DTYPE_BF16, *rows,
+                            a.tokens, a.hidden, *layout, a.vectorized)
+            gateup = bind("moe_grouped_gateup_swiglu_strided", a.packed, a.gate_up, a.gate_up_row_stride, a.activated,
+                          a.offsets, a.packed_rows, a.hidden, a.intermediate, a.experts)
+        down = bind("moe_grouped_gemm_strided", a.activated, a.down, a.down_row_stride, a.expert_output, a.offsets,
+                    a.packed_rows, a.hidden, a.intermediate, a.experts)
+        combine = bind("moe_combine", a.expert_output, _lib.DTYPE_BF16, a.inverse, a.weights, a.output, a.tokens,
+                       a.hidden, a.topk, a.packed_rows)
+        return {"router": router, "dispatch": dispatch, "gateup_swiglu": gateup, "down": down, "combine": combine}
 
 
 @torch.inference_mode()

@@ -530,3 +530,23 @@ def test_config5_full_size_zipf_skew():
     counts = _check_block_sampled(cfg, 8192, bias=oracle.zipf_bias(64), full_span=True)
     assert int((counts == 0).sum()) >= 3
     assert int((counts > 0.15 * 8192 * 6).sum()) >= 2
+
+
+def test_first_forward_of_a_token_count_asks_the_library_once(monkeypatch):
+    """A new token count pays for its buffers, its operators and one argument struct: one
+    query of the one-pass route, and no argument tuples for the stages (stage_calls
+    makes those for whoever times them)."""
+    cfg = MoEConfig(512, 256, 64, 6)
+    block = MoEBlock(cfg, device="cuda", implementation="cuda_fused", seed=0)
+    lib = block._extension.lib
+    real, calls = lib.moe_route_rows_scratch_bytes, []
+    monkeypatch.setattr(lib, "moe_route_rows_scratch_bytes", lambda *a: calls.append(a) or real(*a))
+    for tokens in (5, 300):
+        x = torch.randn(tokens, cfg.hidden, device="cuda").bfloat16()
+        calls.clear()
+        block(x)
+        block(x)
+        assert calls == [(tokens, cfg.hidden, cfg.experts, cfg.topk)]
+        launches = block._launches[(tokens, x.device)]
+        pairs = {name: value for name, value in vars(launches).items() if isinstance(value, tuple)}
+        assert set(pairs) == {"fingerprint", "keep"}, set(pairs)
