@@ -134,7 +134,8 @@ def time_graph(fn, reps, warmup):
 def time_stages(block, x, steps, warmup):
     """Per-stage GPU time: the forward's own C-ABI calls (the block's pre-bound
     launches, router split already done), each repeated back to back in a graph
-    (every stage is idempotent given the previous stage's outputs)."""
+    (every stage is idempotent given the previous stage's outputs). A small
+    batch's forward has one ``route`` stage where others have router and dispatch."""
     import torch
 
     with torch.inference_mode():
@@ -578,7 +579,8 @@ def main(argv=None):
         "stages_us": {k: round(v["mean_us"], 2) for k, v in stages.items()},
         "expert_tflops": round(expert_tflops, 1),
         "expert_mfma_frac": round(expert_tflops / BF16_PEAK_TFLOPS, 4),
-        "dispatch_gbs": round(disp_bytes / (stages["dispatch"]["mean_us"] * 1e-6) / 1e9, 1),
+        "dispatch_gbs": (round(disp_bytes / (stages["dispatch"]["mean_us"] * 1e-6) / 1e9, 1)
+                         if "dispatch" in stages else None),
         "combine_gbs": round(comb_bytes / (stages["combine"]["mean_us"] * 1e-6) / 1e9, 1),
         "expert_counts": counts.tolist(),
         "roofline": gateup_roofline(args.config, counts, block.workspace(x).transport.packed.shape[0],

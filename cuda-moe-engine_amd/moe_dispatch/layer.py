@@ -507,8 +507,8 @@ class _FusedLaunches:
 
     def stage_calls(self, x):
         """Each stage of __call__ as a zero-argument callable on the current
-        stream (the router with the split it holds), for per-stage timing. A
-        small batch's one-pass route is timed as its two stages' own calls."""
+        stream (the router with the split it holds), for per-stage timing: router
+        and dispatch, or for a small batch the one-pass ``route`` in their place."""
         lib, a, x_ptr = self.lib, self.args, x.data_ptr()
 
         def bind(name, *args):
@@ -516,33 +516,40 @@ class _FusedLaunches:
                 lib.check(getattr(lib, name)(*args, current_stream_handle(self.device_index)), name)
             return run
 
-        router = (x_ptr, None, a.bias, a.ids32, a.ids64, a.weights, None, a.router_scratch, a.router_scratch_bytes,
-                  a.tokens, a.hidden, a.experts, a.topk)
         index = (a.ids32, a.counts, a.offsets, a.slots)
-        table = (a.ranks, a.tile_counts, a.tile_counts_bytes, a.tile_tokens)
-        counted = (a.dispatch_scratch, a.dispatch_scratch_bytes)
         layout = (a.experts, a.topk, a.alignment, a.packed_rows)
-        if self.ranked:
-            router = bind("moe_router_fused_ranked", *router, a.ranks, a.tile_counts, a.tile_counts_bytes)
+        stages = {}
+        if a.one_pass:
+            stages["route"] = bind("moe_route_rows", x_ptr, None, a.bias, a.ids32, a.ids64, a.weights, a.router_scratch,
+                                   a.router_scratch_bytes, *index[1:], a.inverse, a.row_src, a.sums, a.sums_bytes,
+                                   a.tokens, a.hidden, *layout)
         else:
-            router = bind("moe_router_fused", *router)
+            table = (a.dispatch_scratch, a.dispatch_scratch_bytes)
+            router = (x_ptr, None, a.bias, a.ids32, a.ids64, a.weights, None, a.router_scratch, a.router_scratch_bytes,
+                      a.tokens, a.hidden, a.experts, a.topk)
+            name = ""
+            if self.ranked:
+                name, table = "_ranked", (a.ranks, a.tile_counts, a.tile_counts_bytes, a.tile_tokens)
+                router += table[:3]
+            stages["router"] = bind("moe_router_fused" + name, *router)
+            if self.gathered:
+                stages["dispatch"] = bind(f"moe_dispatch{name}_rows", *index, a.inverse, a.row_src, *table, a.tokens,
+                                          *layout)
+            else:
+                stages["dispatch"] = bind("moe_dispatch" + name, x_ptr, _lib.DTYPE_BF16, *index, a.packed, a.inverse,
+                                          *table, a.tokens, a.hidden, *layout, a.vectorized)
+        gemm = (a.activated, a.offsets, a.packed_rows, a.hidden, a.intermediate, a.experts)
         if self.gathered:
-            rows = index + (a.inverse, a.row_src) + (table if self.ranked else counted)
-            dispatch = bind("moe_dispatch_ranked_rows" if self.ranked else "moe_dispatch_rows", *rows, a.tokens, *layout)
-            gateup = bind("moe_grouped_gateup_swiglu_gathered_strided", x_ptr, a.row_src, a.tokens, a.gate_up,
-                          a.gate_up_row_stride, a.activated, a.offsets, a.packed_rows, a.hidden, a.intermediate,
-                          a.experts)
+            stages["gateup_swiglu"] = bind("moe_grouped_gateup_swiglu_gathered_strided", x_ptr, a.row_src, a.tokens,
+                                           a.gate_up, a.gate_up_row_stride, *gemm)
         else:
-            rows = index + (a.packed, a.inverse) + (table if self.ranked else counted)
-            dispatch = bind("moe_dispatch_ranked" if self.ranked else "moe_dispatch", x_ptr, _lib.DTYPE_BF16, *rows,
-                            a.tokens, a.hidden, *layout, a.vectorized)
-            gateup = bind("moe_grouped_gateup_swiglu_strided", a.packed, a.gate_up, a.gate_up_row_stride, a.activated,
-                          a.offsets, a.packed_rows, a.hidden, a.intermediate, a.experts)
-        down = bind("moe_grouped_gemm_strided", a.activated, a.down, a.down_row_stride, a.expert_output, a.offsets,
-                    a.packed_rows, a.hidden, a.intermediate, a.experts)
-        combine = bind("moe_combine", a.expert_output, _lib.DTYPE_BF16, a.inverse, a.weights, a.output, a.tokens,
-                       a.hidden, a.topk, a.packed_rows)
-        return {"router": router, "dispatch": dispatch, "gateup_swiglu": gateup, "down": down, "combine": combine}
+            stages["gateup_swiglu"] = bind("moe_grouped_gateup_swiglu_strided", a.packed, a.gate_up,
+                                           a.gate_up_row_stride, *gemm)
+        stages["down"] = bind("moe_grouped_gemm_strided", a.activated, a.down, a.down_row_stride, a.expert_output,
+                              *gemm[1:])
+        stages["combine"] = bind("moe_combine", a.expert_output, _lib.DTYPE_BF16, a.inverse, a.weights, a.output,
+                                 a.tokens, a.hidden, a.topk, a.packed_rows)
+        return stages
 
 
 @torch.inference_mode()

@@ -550,3 +550,32 @@ def test_first_forward_of_a_token_count_asks_the_library_once(monkeypatch):
         launches = block._launches[(tokens, x.device)]
         pairs = {name: value for name, value in vars(launches).items() if isinstance(value, tuple)}
         assert set(pairs) == {"fingerprint", "keep"}, set(pairs)
+
+
+@pytest.mark.parametrize("cfg,tokens,first", [
+    (MoEConfig(512, 256, 64, 6), 40, ["route"]),              # one-pass route with plane sums
+    (MoEConfig(512, 256, 8, 2), 7, ["route"]),                # one-pass route in one workgroup
+    (MoEConfig(512, 256, 8, 2), 200, ["router", "dispatch"]),  # ranked, packed
+    (MoEConfig(512, 256, 8, 4), 200, ["router", "dispatch"]),  # ranked, gathered
+    (MoEConfig(128, 64, 64, 2), 3000, ["router", "dispatch"]),  # counted, packed
+    (MoEConfig(128, 64, 64, 6), 3000, ["router", "dispatch"]),  # counted, gathered
+])
+def test_stage_calls_are_the_forwards_own(monkeypatch, cfg, tokens, first):
+    """The timed stages make the calls that the forward makes, in its order and with its
+    arguments: run one after another on cleared buffers they give its output."""
+    block = MoEBlock(cfg, device="cuda", implementation="cuda_fused", seed=0)
+    x = torch.randn(tokens, cfg.hidden, device="cuda").bfloat16()
+    block(x)
+    want = block(x).clone()
+    launches = block._launches[(tokens, x.device)]
+    assert (launches.args.one_pass == 1) == (first == ["route"])
+    stages = launches.stage_calls(x)
+    assert list(stages) == first + ["gateup_swiglu", "down", "combine"]
+    state = block.workspace(x)
+    with torch.inference_mode():
+        buffers = [t for t in vars(state.transport).values() if isinstance(t, torch.Tensor)]
+        for t in buffers + [state.activated, state.expert_output, *block._route_buffers[(tokens, x.device)]]:
+            t.zero_()
+    for run in stages.values():
+        run()
+    assert torch.equal(launches.output, want)
