@@ -47,14 +47,14 @@ GEMM_CASES = [
     ([1024, 1030, 998, 1051], 8, 264, 200),
     ([33] * 16, 1, 128, 1024),
     ([2000, 0], 8, 1024, 512),
-    # at most 128 rows in all: the 32-column decode tiles (K % 64 == 0; K=96 takes the generic path)
+    # at most 128 rows in all: the decode tiles (K=96: with a partial last stage)
     ([90, 20, 0], 8, 200, 96),
     ([1, 0, 1], 1, 1000, 64),
     ([90, 20, 0], 8, 200, 128),
     ([7, 0, 40], 1, 96, 192),
     ([2, 2], 1, 4096, 1024),
-    # generic path (K % 64 != 0) with one or two column tiles: 9 row tiles of one
-    # expert need every one of the 8 * ceil(9 / 8) workgroup slots
+    # K % 64 != 0 on the wide tiles, with one column tile: nine row tiles of one expert;
+    # full and short ones
     ([2304], 8, 256, 200),
     ([1500, 100, 3, 0], 8, 256, 1000),
 ]
@@ -255,7 +255,7 @@ STRIDED_CASES = [
     ([60, 40, 20], 8, 512, 2048, 64),            # weight-streaming kernel, 128-row instance
     ([700, 3, 0, 260, 1100], 8, 384, 1024, 64),  # persistent kernel: full, short and split tiles
     ([300, 420, 520, 700, 1034, 100], 8, 128, 512, 8),
-    ([1500, 100, 3, 0], 8, 256, 200, 8),         # generic kernel (K % 64 != 0)
+    ([1500, 100, 3, 0], 8, 256, 200, 8),         # partial last stage (K % 64 != 0)
 ]
 
 
@@ -412,17 +412,25 @@ def test_gateup_pieces_do_not_change_results(ext, counts, alignment, inter, k, g
     assert torch.all(outs[0][used:] == 3.0)
 
 
-@pytest.mark.parametrize("counts,n", [
-    ([2, 2], 4096),            # 32 columns (256 CUs: one tile each)
-    ([1, 3, 2, 2], 8192),      # 64 columns
-    ([1, 0, 3, 2, 1], 8200),   # 64 columns, a last tile of 8
-    ([100] * 8, 4104),         # 128 columns, 128-row tiles
-    ([20, 1, 0, 5, 60], 4096), # 128 columns, 64-row tiles
-    ([100, 10] * 4, 1000),     # 64 columns, tall and short tiles
-])
-def test_weight_streaming_widths(ext, counts, n):
-    """The plain weight-streaming GEMM at each column width, against the oracle."""
-    k = 192
+WIDTH_CASES = [
+    # counts per expert, n, rows of the instance (64: at most 64 rows in all), columns per
+    # tile at 256 workgroups (tests/test_ring_plan.py checks both from the rule)
+    ([2, 2], 4096, 64, 32),             # one round of the narrowest tiles
+    ([1, 2, 3, 1], 4096, 64, 64),       # two full rounds
+    ([1, 3, 2, 2, 40], 3832, 64, 128),  # three rounds, the last one short; a last tile of 120 columns
+    ([20, 1, 0, 5, 60], 4096, 128, 64),
+    ([20, 1, 30, 5, 60], 3832, 128, 128),
+    ([100, 10] * 4, 1000, 128, 64),     # tall and short row tiles
+    ([100, 10] * 4, 4096, 128, 128),
+    ([100] * 8, 4104, 128, 128),
+]
+
+
+@pytest.mark.parametrize("counts,n,instance,columns", WIDTH_CASES)
+def test_weight_streaming_widths(ext, counts, n, instance, columns):
+    """The plain weight-streaming GEMM at each column width of both its instances,
+    against the oracle. Ten k stages: more than any of these rings holds."""
+    k = 640
     a, offsets, rows = _inputs(counts, 1, k, seed=n)
     g = torch.Generator(device="cuda").manual_seed(n)
     b = (torch.randn(len(counts), n, k, device="cuda", generator=g) / k**0.5).bfloat16()

@@ -342,3 +342,21 @@ def test_launches_of_one_round_keep_the_narrowest_columns():
         assert width == narrow_shift(*case, one_round_stops=False), case
         widened += width > case[0]
     assert widened > 1000
+
+
+def test_width_cases_reach_every_width():
+    """The GPU width test's cases run the instance and the column width they name on 256
+    CUs: the launcher's choice of instance, then the device's of the width."""
+    from tests.test_gpu_gemm import WIDTH_CASES
+
+    for counts, n, instance, columns in WIDTH_CASES:
+        rows = sum(counts) + 5  # the test's spare rows
+        experts = len(counts)
+        wide_tiles = experts * -(-(-(-rows // experts)) // 256) * -(-n // 256)
+        assert rows <= 128 or (rows <= 128 * experts and wide_tiles < 256)
+        assert instance == (64 if rows <= 64 else 128)
+        groups = sum(-(-c // instance) for c in counts)
+        a_rows = 128 if instance == 128 and max(counts) > 64 else 64
+        assert columns == 1 << narrow_shift(5 if instance == 64 else 6, groups, n, a_rows, 256), (counts, n)
+    reached = {(instance, columns) for _, _, instance, columns in WIDTH_CASES}
+    assert reached == {(64, 32), (64, 64), (64, 128), (128, 64), (128, 128)}
