@@ -237,8 +237,8 @@ static int check_dispatch(const void* x, int dtype, const int32_t* ids, int32_t*
 
 static int check_dispatch_alignment(const void* x, int dtype, void* packed, const int32_t* ids, int32_t* counts,
                                     int32_t* offsets, int32_t* slots, int32_t* inverse, const void* table) {
-    // Rows are copied with the widest access that the row size and both base
-    // addresses allow (launch_dispatch), down to one element.
+    // Rows of at least 16 bytes are copied as 16-byte vectors at any element's
+    // address (the last one may overlap the one before), shorter ones by elements.
     const uintptr_t elem = static_cast<uintptr_t>(dtype_size(dtype));
     MOE_REQUIRE(aligned_to(x, elem) && aligned_to(packed, elem), MOE_ERR_INVALID_ARGUMENT,
                 "x and packed must be aligned to their element size");
@@ -401,7 +401,7 @@ int moe_combine(const void* expert_output, int dtype, const int32_t* inverse,
     MOE_REQUIRE(packed_rows >= tokens * topk, MOE_ERR_INVALID_ARGUMENT, "shape/dtype mismatch");
     if (tokens == 0) return MOE_OK;
     MOE_REQUIRE(expert_output && inverse && weights && output, MOE_ERR_INVALID_ARGUMENT, "null pointer");
-    // 16-byte vectors when both row arrays allow them (launch_combine), else elements.
+    // 16-byte vectors at any element's address, elements for rows shorter than one (launch_combine).
     const uintptr_t elem = static_cast<uintptr_t>(dtype_size(dtype));
     MOE_REQUIRE(aligned_to(expert_output, elem) && aligned_to(output, elem), MOE_ERR_INVALID_ARGUMENT,
                 "expert output and output must be aligned to their element size");

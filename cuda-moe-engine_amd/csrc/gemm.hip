@@ -93,7 +93,9 @@ static int launch_gemm_t(GemmParams p, int64_t rows, hipStream_t stream) {
     // cold takes 2-3 us longer: forwards at H=1024, I=2048, 16 experts, 8192 rows
     // 153 -> 156 us with it, at H=2048, I=1408, 64 experts, 288 rows 219.7 ->
     // 221.4; against 603 -> 550 (with the down GEMM's widths) at H=4096, I=14336, 8
-    // experts, 666 rows, whose 896 tiles fill three and a half rounds.
+    // experts, 666 rows, whose 896 tiles fill three and a half rounds. (`rows` is the
+    // buffer's padded capacity: E=64, top-6 counts as few rows up to 47 tokens at
+    // alignment 8 and never from 16 on, where one token takes 17.4 us against 15.3.)
     bool pieces = !SWIGLU;
     if constexpr (SWIGLU) {
         const int64_t cus = device_cu_count(), last = wide_tiles % cus;

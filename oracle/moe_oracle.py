@@ -315,11 +315,10 @@ def grouped_gemm(a: np.ndarray, b: np.ndarray, offsets: np.ndarray, order: str =
     * ``"exact"``: float64 accumulation, one rounding to fp32 (the correctly
       rounded dot product);
     * ``"mfma"`` (default): the accumulation order of the HIP kernels, which
-      apply ``v_mfma_f32_16x16x32_bf16`` (fast path) or
-      ``v_mfma_f32_32x32x16_bf16`` (generic path) along k in ascending order,
+      apply ``v_mfma_f32_16x16x32_bf16`` along k in ascending order,
       modelled as: add the exact sum of each ascending group of 8 products to
       the fp32 accumulator with one round-to-nearest-even. Measured on MI355X
-      for both instructions: the grouping and rounding are right (groups of
+      (``v_mfma_f32_32x32x16_bf16`` behaves alike): the grouping and rounding are right (groups of
       4, 16 or 32 are far off), but the hardware sums the 8 products with a
       limited-width internal alignment, so ~0.2-0.3% of single-instruction
       fp32 results differ by one ulp; after the bf16 output rounding ~1e-5 of

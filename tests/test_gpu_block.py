@@ -131,7 +131,7 @@ def test_small_blocks(tokens, pattern, topk):
 @pytest.mark.parametrize("cfg,tokens", [
     ((64, 128, 1, 1), 50),         # one expert, top-1
     ((128, 64, 8, 8), 40),         # top-8 of 8: every token on every expert (row table)
-    ((72, 136, 12, 3), 60),        # hidden and intermediate not multiples of 64: the generic GEMM, packed rows
+    ((72, 136, 12, 3), 60),        # hidden and intermediate not multiples of 64: packed rows
     ((64, 64, 64, 8), 30),         # E=64, top-8, few tokens: most experts empty (row table)
     ((128, 128, 4, 2, 128), 100),  # alignment 128: most packed rows are padding
     ((128, 256, 8, 2), 2048),      # H=128: the down GEMM's 128-column halves past its last column

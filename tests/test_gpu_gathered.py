@@ -174,7 +174,7 @@ def test_gathered_gateup_rejects_hidden_not_a_multiple_of_64(ext):
     ((2048, 1408, 64, 6), 700, True),   # top-6: the row table
     ((256, 128, 16, 3), 300, True),     # top-3, hidden a multiple of 64
     ((512, 1024, 8, 2), 128, False),    # top-2 packs (the gathered GEMM's loads cost more than the copy)
-    ((96, 256, 8, 4), 100, False),      # hidden not a multiple of 64: the generic GEMM cannot gather
+    ((96, 256, 8, 4), 100, False),      # hidden not a multiple of 64: a partial stage cannot gather
 ])
 def test_block_forward_gathers_from_top3_on_and_matches_the_packed_forward(monkeypatch, cfg, tokens, gathers):
     """The block's forward, gathered or packed, is the same bit for bit."""

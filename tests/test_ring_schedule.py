@@ -1,6 +1,6 @@
 """The grouped GEMM's LDS ring schedule, simulated on the CPU.
 
-ring_tile (cuda-moe-engine_amd/csrc/gemm.hip) keeps SA stages of A and SB >= SA
+ring_tile (cuda-moe-engine_amd/csrc/gemm_ring.h) keeps SA stages of A and SB >= SA
 stages of B in LDS (equal depths of 3-4 for small tiles, 2 and 3 for the full
 256 x 256 tile), issues per stage window the A loads of stage u+SA and then
 the B loads of stage u+SB into the slots stage u freed, and before reading
