@@ -86,6 +86,9 @@ class BlockArgs(ctypes.Structure):
 BlockArgs._fields_ = [(name, _c_void_p if name in BlockArgs._POINTERS else _i64) for name in BlockArgs._ORDER]
 
 
+BLOCK_ARGS_BYTES = ctypes.sizeof(BlockArgs)
+
+
 def library_path() -> Path:
     override = os.environ.get("MOE_HIP_LIBRARY")
     if override:

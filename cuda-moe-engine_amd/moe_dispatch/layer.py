@@ -16,7 +16,7 @@ Top-k may be 1..8 (the reference allows 1 or 2); ``set_routing_bias`` sets an
 arbitrary router bias.
 """
 
-import ctypes
+from array import array
 from dataclasses import dataclass
 import math
 
@@ -406,9 +406,6 @@ def _one_pass_bytes(lib, tokens, cfg):
     return need if need >= 0 and _can_gather(tokens, cfg.hidden) else None
 
 
-_BLOCK_ARGS_BYTES = ctypes.sizeof(_lib.BlockArgs)
-
-
 class _FusedLaunches:
     """The C-ABI calls of one validated cuda_fused forward, for reuse.
 
@@ -453,24 +450,28 @@ class _FusedLaunches:
         if x.dtype != torch.bfloat16:
             raise RuntimeError("cuda_fused launches are bf16")
         sums = state.plane_sums
-        # The whole forward as one call (moe_block_forward). Every new token count pays for
-        # this: one constructor call (a setattr per field takes three times as long).
-        self.args = _lib.BlockArgs(
-            struct_bytes=_BLOCK_ARGS_BYTES, bias=block.routing_bias.data_ptr(), ids32=ids32.data_ptr(),
-            ids64=ids64.data_ptr(), weights=weights.data_ptr(), router_scratch=scratch.data_ptr(),
-            router_scratch_bytes=scratch.numel(), counts=t.counts.data_ptr(), offsets=t.offsets.data_ptr(),
-            slots=t.slots.data_ptr(), inverse=t.inverse.data_ptr(), row_src=t.row_src.data_ptr(),
-            packed=t.packed.data_ptr(), dispatch_scratch=t.scratch.data_ptr(), dispatch_scratch_bytes=t.scratch.numel(),
-            ranks=t.tile_ranks.data_ptr(), tile_counts=t.tile_counts.data_ptr(),
-            tile_counts_bytes=t.tile_counts.numel() * 4, tile_tokens=t.rank_tile,
-            sums=None if sums is None else sums.data_ptr(), sums_bytes=0 if sums is None else sums.numel(),
-            gate_up=block.gate_up_weight.data_ptr(), gate_up_row_stride=gate_up_stride,
-            down=block.down_weight.data_ptr(), down_row_stride=down_stride, activated=state.activated.data_ptr(),
-            expert_output=state.expert_output.data_ptr(), output=t.output.data_ptr(), tokens=tokens, hidden=hidden,
-            intermediate=cfg.intermediate, experts=cfg.experts, topk=cfg.topk, alignment=t.alignment,
-            packed_rows=t.capacity_rows, vectorized=bool(t.vectorized), gathered=self.gathered,
-            one_pass=state.one_pass)
-        self.args_address = ctypes.addressof(self.args)
+        # The whole forward as one call (moe_block_forward): moe_block_args as its 64-bit
+        # fields, in the header's order (``args`` names them; null pointers are 0). Every new
+        # token count pays for this, and names for the fields, in a dictionary or a structure's
+        # keywords, are allocations outside the interpreter's small ones: 10-45 us more.
+        self.packed_args = array("q", (
+            _lib.BLOCK_ARGS_BYTES, block.routing_bias.data_ptr(), ids32.data_ptr(), ids64.data_ptr(),
+            weights.data_ptr(), scratch.data_ptr(), scratch.numel(),
+            t.counts.data_ptr(), t.offsets.data_ptr(), t.slots.data_ptr(), t.inverse.data_ptr(), t.row_src.data_ptr(),
+            t.packed.data_ptr(), t.scratch.data_ptr(), t.scratch.numel(),
+            t.tile_ranks.data_ptr(), t.tile_counts.data_ptr(), t.tile_counts.numel() * 4, t.rank_tile,
+            0 if sums is None else sums.data_ptr(), 0 if sums is None else sums.numel(),
+            block.gate_up_weight.data_ptr(), gate_up_stride, block.down_weight.data_ptr(), down_stride,
+            state.activated.data_ptr(), state.expert_output.data_ptr(), t.output.data_ptr(),
+            tokens, hidden, cfg.intermediate, cfg.experts, cfg.topk, t.alignment, t.capacity_rows,
+            bool(t.vectorized), self.gathered, state.one_pass))
+        self.args_address = self.packed_args.buffer_info()[0]
+        self.hidden = hidden
+
+    @property
+    def args(self):
+        """The packed arguments by their names in the header (a view)."""
+        return _lib.BlockArgs.from_buffer(self.packed_args)
 
     @classmethod
     def _fingerprint(cls, block):
@@ -493,7 +494,7 @@ class _FusedLaunches:
     def accepts(self, x):
         """The caller's half of the checks (the key these launches are kept under has its
         token count and device; the weights' device and dtype are theirs)."""
-        return x.dtype == torch.bfloat16 and x.shape[1] == self.args.hidden and x.is_contiguous()
+        return x.dtype == torch.bfloat16 and x.shape[1] == self.hidden and x.is_contiguous()
 
     def __call__(self, block, x):
         router_weight, split_of = block._router_split_plan()

@@ -550,6 +550,24 @@ def test_first_forward_of_a_token_count_asks_the_library_once(monkeypatch):
         launches = block._launches[(tokens, x.device)]
         pairs = {name: value for name, value in vars(launches).items() if isinstance(value, tuple)}
         assert set(pairs) == {"fingerprint", "keep"}, set(pairs)
+        # Every field of the packed arguments under its name in the header.
+        args, state = launches.args, block.workspace(x)
+        t, (ids32, ids64, weights) = state.transport, block._route_buffers[(tokens, x.device)]
+        pointers = {"bias": block.routing_bias, "ids32": ids32, "ids64": ids64, "weights": weights,
+                    "router_scratch": block._router_scratch, "counts": t.counts, "offsets": t.offsets,
+                    "slots": t.slots, "inverse": t.inverse, "row_src": t.row_src, "packed": t.packed,
+                    "dispatch_scratch": t.scratch, "ranks": t.tile_ranks, "tile_counts": t.tile_counts,
+                    "sums": state.plane_sums, "gate_up": block.gate_up_weight, "down": block.down_weight,
+                    "activated": state.activated, "expert_output": state.expert_output, "output": t.output}
+        sizes = {"struct_bytes": 8 * len(args._ORDER), "router_scratch_bytes": block._router_scratch.numel(),
+                 "dispatch_scratch_bytes": t.scratch.numel(), "tile_counts_bytes": 4 * t.tile_counts.numel(),
+                 "tile_tokens": t.rank_tile, "sums_bytes": 0 if state.plane_sums is None else state.plane_sums.numel(),
+                 "gate_up_row_stride": cfg.hidden, "down_row_stride": cfg.intermediate, "tokens": tokens,
+                 "hidden": cfg.hidden, "intermediate": cfg.intermediate, "experts": cfg.experts, "topk": cfg.topk,
+                 "alignment": cfg.alignment, "packed_rows": t.capacity_rows, "vectorized": 1,
+                 "gathered": 1, "one_pass": int(tokens == 5)}
+        want = {name: v.data_ptr() if v is not None else None for name, v in pointers.items()} | sizes
+        assert {name: getattr(args, name) for name in args._ORDER} == want
 
 
 @pytest.mark.parametrize("cfg,tokens,first", [
