@@ -294,9 +294,11 @@ def gateup_roofline(config, counts, packed_rows, hidden, inter, n_assign, flop, 
     ``csrc/gemm.hip``): the weight-streaming (decode) kernel when the buffer
     has at most 128 rows, or at most 128 per expert while the 256 x 256 tiles
     (rows spread evenly over the experts) would number fewer than the CUs
-    (``cus``; default: the current GPU's, 256 without one). ``gathered``: the
-    forward's gate/up GEMM read its rows from x through the row table (the
-    kernels' GATHER instances).
+    (``cus``; default: the current GPU's, 256 without one); else the persistent
+    one, its instance that splits tiles (the last argument) when few rows per
+    expert or a last round at most half full of the first four ask for it.
+    ``gathered``: the forward's gate/up GEMM read its rows from x through the
+    row table. The argument after that: H is not a multiple of 64.
     """
     import torch
 
@@ -309,12 +311,13 @@ def gateup_roofline(config, counts, packed_rows, hidden, inter, n_assign, flop, 
     if cus is None:
         cus = torch.cuda.get_device_properties(0).multi_processor_count if torch.cuda.is_available() else 256
     wide_tiles = experts * ceil_div(ceil_div(packed_rows, experts), 256) * ceil_div(inter, 128)
-    decode = hidden % 64 == 0 and (packed_rows <= 128 or (packed_rows <= 128 * experts and wide_tiles < cus))
-    g = "true" if gathered else "false"
-    if decode:
-        kernel = f"grouped_gemm_decode_kernel<true, {64 if packed_rows <= 64 else 128}, {g}>"
+    source = f"{str(gathered).lower()}, {str(hidden % 64 != 0).lower()}"
+    if packed_rows <= 128 or (packed_rows <= 128 * experts and wide_tiles < cus):
+        kernel = f"grouped_gemm_decode_kernel<true, {64 if packed_rows <= 64 else 128}, {source}>"
     else:
-        kernel = f"grouped_gemm_persistent_kernel<true, {g}>"
+        last = wide_tiles % cus
+        pieces = ceil_div(packed_rows, experts) < 12 or 0 < 2 * last <= cus and wide_tiles < 4 * cus
+        kernel = f"grouped_gemm_persistent_kernel<true, {source}, {str(pieces).lower()}>"
     entry = {"kernel": kernel + " (gate/up GEMM + SwiGLU epilogue)"}
     if flop / byte < BF16_PEAK_TFLOPS * 1e12 / (HBM_PEAK_GBS * 1e9):
         achieved = byte / (launch_us * 1e-6) / 1e9
@@ -378,7 +381,7 @@ def transport_bench(args):
     comb_bytes = combine_bytes(tokens, hidden, topk)
     d_gbs = disp_bytes / (d_us * 1e-6) / 1e9
     c_gbs = comb_bytes / (c_us * 1e-6) / 1e9
-    traffic = measured_traffic(args.config, ("count_rank_kernel", "pack_kernel<16, false, false>"))
+    traffic = measured_traffic(args.config, ("count_rank_kernel", "pack_kernel<16, false, false, true>"))
     result = {
         "metric": "MoE block fwd latency (us) + expert TFLOP/s % bf16 MFMA peak; dispatch GB/s",
         "value": round(mean_us, 2),
