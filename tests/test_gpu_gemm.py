@@ -307,6 +307,7 @@ PARTIAL_STAGE_CASES = [
     ([700, 3, 40, 260, 1100], 8, 520, 248),              # four stages: chained tiles, short tiles
     ([1030, 1030, 2048], 8, 512, 328),                   # column pieces left after the rounds
     ([300, 420, 520, 700, 1034, 100], 8, 136, 2744),     # balanced row tiles (gate/up at K >= 2048)
+    ([700, 300, 40, 1100], 8, 1528, 200),                # persistent gate/up whose tiles stay whole
 ]
 
 
@@ -344,8 +345,8 @@ def test_partial_last_stage_equals_zero_padded(ext, counts, alignment, n, k):
 @pytest.mark.parametrize("counts,k", [
     ([3, 0, 5], 72),            # weight-streaming kernel, 64-row instance
     ([90, 20], 200),            # 128-row instance
-    ([700, 40, 300], 136),      # persistent kernel
-    ([5] * 40, 8),              # persistent kernel, column pieces
+    ([700, 40, 300], 136),      # persistent kernel, its instance that splits tiles
+    ([5] * 40, 8),              # weight-streaming kernel, many experts
 ])
 def test_partial_stage_activation_over_the_whole_range(ext, counts, k):
     """K not a multiple of 64: the fused epilogue gives the oracle's SwiGLU bit for bit
@@ -371,17 +372,20 @@ def test_partial_stage_activation_over_the_whole_range(ext, counts, k):
 
 
 GATEUP_PIECES_CASES = [
-    # counts per expert, alignment, intermediate, k, workgroup bounds (0: one per CU)
-    ([90, 3, 128, 0, 64, 33], 8, 1400, 128, (0, 8, 24)),       # short tiles alone: halves, quarters
-    ([5] * 40, 8, 200, 192, (0, 8, 16)),                        # few rows per expert; a last piece past the columns
-    ([700, 300, 900], 8, 264, 2048, (0, 8, 16, 24)),            # balanced tiles alone: halves of a last round
-    ([520, 40, 260, 7], 8, 384, 64, (0, 8, 24)),                # short tiles after rounds: quarters, never halves
-    ([90, 3, 128, 0, 64, 33], 8, 1400, 200, (0, 8)),            # K not a multiple of 64
+    # counts per expert, alignment, intermediate, k, workgroup bounds (0: one per CU), and what
+    # a last round splits into at each bound on 256 CUs (tests/test_ring_plan.py checks that the
+    # launch takes the instance that splits, and the splits)
+    ([90, 3, 128, 0, 64, 33] * 4, 8, 1400, 128, (0, 8, 24), ("whole", "halves", "quarters")),  # short tiles alone
+    ([5] * 40, 8, 840, 192, (0, 8, 16), ("quarters", "whole", "halves")),  # few rows; a last piece past the columns
+    ([5] * 40, 8, 840, 2048, (16, 64), ("whole", "halves")),  # rows 4 KiB apart: halves up to 3/8 of a round
+    ([700, 300, 900], 8, 264, 2048, (0, 8, 16, 24), ("halves", "halves", "whole", "halves")),  # balanced tiles alone
+    ([520, 40, 260, 7, 3], 8, 512, 64, (0, 8, 24), ("whole", "whole", "quarters")),  # after rounds: never halves
+    ([90, 3, 128, 0, 64, 33] * 4, 8, 1400, 200, (0, 8, 24), ("whole", "halves", "quarters")),  # K % 64 != 0
 ]
 
 
-@pytest.mark.parametrize("counts,alignment,inter,k,grids", GATEUP_PIECES_CASES)
-def test_gateup_pieces_do_not_change_results(ext, counts, alignment, inter, k, grids):
+@pytest.mark.parametrize("counts,alignment,inter,k,grids,splits", GATEUP_PIECES_CASES)
+def test_gateup_pieces_do_not_change_results(ext, counts, alignment, inter, k, grids, splits):
     """Gate/up tiles split into column halves and quarters: the fused output equals the
     unfused pipeline's (near bit-exact) and is the same bit for bit on every grid size,
     packed and gathered; rows past offsets[E] stay untouched."""

@@ -197,8 +197,10 @@ def test_grid_sizes_used_on_the_gpu_cover_each_path():
     for counts, alignment, n, k, swiglu, grids in SCHEDULE_CASES:
         n_tiles = -(-n // (128 if swiglu else 256))
         n1, n2 = phase_counts(counts, alignment, n_tiles, balanced_for(swiglu, k))
+        pieces = launch(counts, alignment, n, swiglu) == "pieces"
+        assert launch(counts, alignment, n, swiglu) in ("pieces", "whole")
         for grid in grids:
-            pl, runs = check_cover(n1, n2, grid, not swiglu)
+            pl, runs = check_cover(n1, n2, grid, pieces, swiglu and pieces, 2 * k % 4096 == 0)
             per_q = {}
             for seq in runs:
                 for q, _ in seq:
@@ -360,3 +362,42 @@ def test_width_cases_reach_every_width():
         assert columns == 1 << narrow_shift(5 if instance == 64 else 6, groups, n, a_rows, 256), (counts, n)
     reached = {(instance, columns) for _, _, instance, columns in WIDTH_CASES}
     assert reached == {(64, 32), (64, 64), (64, 128), (128, 64), (128, 128)}
+
+
+def launch(counts, alignment, n, swiglu, spare=5, cus=256):
+    """launch_gemm_t's kernel for a test's launch (its buffer holds `spare` rows more):
+    "stream64", "stream128", or the persistent instance that splits tiles ("pieces") or
+    does not ("whole")."""
+    experts = len(counts)
+    rows = sum(-(-c // alignment) * alignment for c in counts) + spare
+    per_expert = -(-rows // experts)
+    wide_tiles = experts * -(-per_expert // 256) * -(-n // (128 if swiglu else 256))
+    if rows <= 128 or (rows <= 128 * experts and wide_tiles < cus):
+        return "stream64" if rows <= 64 else "stream128"
+    last = wide_tiles % cus
+    return "pieces" if not swiglu or per_expert < 12 or (0 < 2 * last <= cus and wide_tiles < 4 * cus) else "whole"
+
+
+def test_gateup_pieces_cases_split_as_they_say():
+    from tests.test_gpu_gemm import GATEUP_PIECES_CASES
+
+    reached = set()
+    for counts, alignment, inter, k, grids, splits in GATEUP_PIECES_CASES:
+        assert launch(counts, alignment, inter, True) == "pieces", (counts, inter)
+        n1, n2 = phase_counts(counts, alignment, -(-inter // 128), balanced_for(True, k))
+        for grid, split in zip(grids, splits):
+            # At most one workgroup per unit of work, a multiple of 8.
+            pl, _ = check_cover(n1, n2, grid or 256, True, True, 2 * k % 4096 == 0)
+            got = {0: "whole", 2: "halves", 4: "quarters"}[pl["rest"]["ways"] if pl["rest"]["pieces"] else 0]
+            assert got == split, (counts, grid, got)
+            reached.add((n1 > 0, n2 > 0, split))
+    assert {(False, True, "halves"), (False, True, "quarters"), (True, False, "halves"),
+            (True, True, "quarters"), (True, True, "whole")} <= reached
+
+
+def test_partial_stage_cases_reach_every_instance():
+    from tests.test_gpu_gemm import PARTIAL_STAGE_CASES
+
+    for swiglu, want in ((False, {"stream64", "stream128", "pieces"}),
+                         (True, {"stream64", "stream128", "pieces", "whole"})):
+        assert {launch(c, al, n, swiglu) for c, al, n, _ in PARTIAL_STAGE_CASES} == want
