@@ -17,6 +17,8 @@ CASES = [
     (15, 1032, 10, 4, 16), (2, 2048, 3, 2, 8), (16, 320, 12, 8, 1),
     (1, 2048, 64, 6, 8), (8, 2048, 64, 8, 8), (9, 1000, 17, 3, 8), (128, 4096, 64, 8, 128), (17, 8, 24, 1, 1),
     (100, 256, 33, 2, 8), (128, 2048, 48, 6, 64), (16, 1088, 32, 4, 8),
+    # five fragments at the longest range; one token group at the shortest and longest ranges
+    (13, 6152, 13, 4, 8), (5, 640, 20, 2, 8), (3, 4096, 40, 4, 16),
 ]
 
 

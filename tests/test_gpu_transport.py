@@ -214,7 +214,9 @@ def test_rows_of_any_length_and_offset_views(ext, dtype, row_bytes):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("rows,width", [(5, 1), (3, 7), (9, 8), (300, 9), (40, 257), (2, 2049), (3000, 40)])
+@pytest.mark.parametrize("rows,width", [(5, 1), (3, 7), (9, 8), (300, 9), (40, 257), (2, 2049), (3000, 40),
+                                        # from 2^20 vectors on a thread owns several, stepping whole rows or a part
+                                        (9000, 1001), (350000, 7)])
 def test_standalone_swiglu_widths(ext, dtype, rows, width):
     """Widths around whole vectors, rows and blocks, with special gate values: bit-exact
     (16 bits: the fp32 activation times up, rounded once)."""
